@@ -44,11 +44,13 @@ SegLayout seg_layout(int npol, int nrhs, int nsets, int m32, int num_cu, int ext
     }
     L.vec = align256(sizeof(double) * ncols * n);
     L.xs = m32 == kBatchM32 ? align256(sizeof(unsigned short) * kBxParts * ncols * (size_t)bx_ld(npol)) : 0;
-    // the pair-once sweep at the sizes where the single-system solver uses it;
-    // wide batches run both matvecs on the matrix cores with their own tiling
-    // (partials per source split)
-    L.sym32 = m32 == 2 && tmv_pair_once(npol, 32, ncols, size_t(8) << 30);
-    L.sym64 = m32 == 2 && tmv_pair_once(npol, 64, ncols, size_t(8) << 30);
+    // the pair-once sweep from the sizes where it beats the batched per-target
+    // sweep (measured: FP32 11,000 sites with two columns, 7,000 with one; FP64
+    // 7,000 and 6,000), its partials under 8 GiB; wide batches run both matvecs
+    // on the matrix cores with their own tiling (partials per source split)
+    const bool sym_fits = m32 == 2 && tmv_sym_part_bytes(npol, std::max(ncols, 2), 64) <= size_t(8) << 30;
+    L.sym32 = sym_fits && npol >= (ncols >= 2 ? 11000 : 7000);
+    L.sym64 = sym_fits && npol >= (ncols >= 2 ? 7000 : 6000);
     size_t part = sizeof(double) * L.nsplit * ncols * n;
     if (L.sym32 || L.sym64) part = std::max(part, tmv_sym_part_bytes(npol, ncols, 64));
     L.part = align256(part);

@@ -84,15 +84,15 @@ void launch_rhs_sym(hipStream_t st, bool amoeba, int nmm, int npol, const int2 *
                     const int *polar_mm, const int *np_src, const CsrDev &sp, void *sympart, double *part_np,
                     int nsplit_np, double *e_m2d, hipEvent_t evb = nullptr, hipEvent_t eve = nullptr);
 
-// T matvec on the fly: y[m] = T x[m] (dodiag) or (T - diag) x[m], m < M.
+// T matvec on the fly, per target (tmv_rows.hip): y[m] = T x[m] (dodiag) or (T - diag) x[m], m < M.
 // prec 64 or 32 selects the pair arithmetic; corrections and the final sum are FP64.
-// If dotpart != nullptr, per-block partial sums of y.x go to dotpart[m * nblk + b]
-// where nblk = ceil(npol / kBlock).
-void launch_tmv_otf(hipStream_t st, int prec, bool amoeba, int npol, int M, const double4 *ps64,
-                    const double *pa64, const float4 *ps32, const float *pa32, const double *alpha,
-                    const CsrDev &pp, const double *x, long xstride, double *y, long ystride,
-                    bool dodiag, double *dotpart, void *part, int nsplit, const int *skip_flag,
-                    hipEvent_t evb = nullptr, hipEvent_t eve = nullptr);
+// If dotpart != nullptr, per-workgroup partial sums of y.x go to dotpart[m * nparts + b].
+void launch_tmv_rows(hipStream_t st, int prec, bool amoeba, int npol, int M, const double4 *ps64,
+                     const double *pa64, const float4 *ps32, const float *pa32, const double *alpha,
+                     const CsrDev &pp, const double *x, long xstride, double *y, long ystride,
+                     bool dodiag, double *dotpart, const int *skip_flag, hipEvent_t evb = nullptr,
+                     hipEvent_t eve = nullptr);
+int tmv_rows_dot_parts(int npol, int prec, int ncols);  // per-column y.x partials it writes
 // Finalize alone, for FP64 partial fields computed elsewhere (fast multipoles).
 void launch_tmv_finalize64(hipStream_t st, bool amoeba, int npol, int M, const double *part, int nsplit,
                            const double4 *ps64, const double *pa64, const double *alpha, const CsrDev &pp,
@@ -106,8 +106,8 @@ int tmv_sym_blocks(int npol);
 int tmv_sym_dot_parts(int npol);
 size_t tmv_sym_part_bytes(int npol, int M, int prec);
 // Whether the on-the-fly matvec of prec (32 / 64) with ncols columns uses the
-// pair-once sweep at npol sites (its partial sums at most max_bytes).
-bool tmv_pair_once(int npol, int prec, int ncols, size_t max_bytes = size_t(2) << 30);
+// pair-once sweep at npol sites.
+bool tmv_pair_once(int npol, int prec, int ncols);
 void launch_tmv_sym(hipStream_t st, int prec, bool amoeba, int npol, int M, const int2 *pairs, const double4 *ps64,
                     const double *pa64, const float4 *ps32, const float *pa32, const double *alpha,
                     const CsrDev &pp, const double *x, long xstride, double *y, long ystride, bool dodiag,
@@ -116,9 +116,7 @@ void launch_tmv_sym(hipStream_t st, int prec, bool amoeba, int npol, int M, cons
 void launch_rhs_finalize(hipStream_t st, bool amoeba, int npol, int nsplit, const double *part, const double4 *ms64,
                          const double *ma64, const double *mq, const double4 *ps64, const double *pa64,
                          const CsrDev &sp, double *e_m2d);
-int tmv_split(int npol);
 int balanced_split(int tb, int nsrc, int num_cu);
-size_t tmv_part_bytes(int npol, int M, int prec, int nsplit);
 // FMA rate (TFLOP/s, FMA = 2) of non-packed vector code on the current device,
 // prec 32 or 64: eight independent chains per thread, 8,192 x 256 threads.
 double vector_fma_tflops(int prec);

@@ -64,11 +64,8 @@ struct DeviceState {
     // CG state of each refinement step; pinned copy (allocated on first use)
     CgState *cs_spec = nullptr;
     CgState *cs_spec_host = nullptr;
-    void *mvpart = nullptr;
     int2 *sym_pairs = nullptr;  // block pairs of the pair-once matvec, on first use
     void *sympart = nullptr;
-    size_t mvpart_bytes = 0;
-    int nsplit = 1;
     double *rhs_part = nullptr;
     int rhs_split = 1;
     // static field with the pair-once sweep: the non-polarizable MM sources and
@@ -388,16 +385,14 @@ DeviceState &ensure_device(System &s) {
         for (auto v : vecs) *v = dalloc<double>(d, 2 * n);
         const int nb = std::max(vec_blocks(n), site_blocks(s.npol)) + 8;
         d.red_a = dalloc<double>(d, 24 * (size_t)nb);
-        d.red_b = dalloc<double>(d, 24 * (size_t)nb);
+        // y.x partials of the matvec: per workgroup of a few targets below the pair-once sizes
+        d.red_b = dalloc<double>(d, std::max(24 * (size_t)nb, 2 * (size_t)tmv_rows_dot_parts(s.npol, 64, 2)));
         d.red_c = dalloc<double>(d, 24 * (size_t)nb);
         d.scal = dalloc<double>(d, 64);
         d.tol_dev = dalloc<double>(d, 4);
         d.cs = dalloc<CgState>(d, 2);
         HCHECK(hipHostMalloc((void **)&d.cs_host, 2 * sizeof(CgState), hipHostMallocDefault));
         HCHECK(hipHostMalloc((void **)&d.scal_host, 64 * sizeof(double), hipHostMallocDefault));
-        d.nsplit = tmv_split(s.npol);
-        d.mvpart_bytes = tmv_part_bytes(s.npol, 2, 64, d.nsplit);
-        d.mvpart = dmalloc(d, d.mvpart_bytes);
         {
             hipDeviceProp_t prop;
             HCHECK(hipGetDeviceProperties(&prop, d.device));
@@ -543,8 +538,10 @@ void ensure_sym(const System &s, DeviceState &d) {
 
 // Number of y.x partials per column that matvec() of this kind writes to dotpart.
 static int matvec_dot_parts(const System &s, int kind, int M) {
-    if ((kind == kOtf64 || kind == kOtf32) && tmv_pair_once(s.npol, kind == kOtf32 ? 32 : 64, M))
-        return tmv_sym_dot_parts(s.npol);
+    const int prec = kind == kOtf32 ? 32 : 64;
+    if (kind == kOtf64 || kind == kOtf32)
+        return tmv_pair_once(s.npol, prec, M) ? tmv_sym_dot_parts(s.npol)
+                                                                  : tmv_rows_dot_parts(s.npol, prec, M);
     return site_blocks(s.npol);
 }
 
@@ -573,10 +570,9 @@ void matvec(System &s, DeviceState &d, int kind, int M, const double *x, double 
     }
     if (kind == kPlain64 || kind == kPlain32) {
         const int pi = prof_begin(d, kind == kPlain32 ? kOtf32 : kOtf64);
-        launch_tmv_otf(d.stream, kind == kPlain32 ? 32 : 64, s.amoeba, s.npol, M, d.ps64, d.pa64, d.ps32, d.pa32,
-                       d.alpha, d.pp, x, n, y, n, dodiag, dotpart, d.mvpart, d.nsplit,
-                       reinterpret_cast<const int *>(skip), pi >= 0 ? d.prof_pool[2 * pi] : nullptr,
-                       pi >= 0 ? d.prof_pool[2 * pi + 1] : nullptr);
+        launch_tmv_rows(d.stream, kind == kPlain32 ? 32 : 64, s.amoeba, s.npol, M, d.ps64, d.pa64, d.ps32, d.pa32,
+                        d.alpha, d.pp, x, n, y, n, dodiag, dotpart, reinterpret_cast<const int *>(skip),
+                        pi >= 0 ? d.prof_pool[2 * pi] : nullptr, pi >= 0 ? d.prof_pool[2 * pi + 1] : nullptr);
     } else {
         const int prec = kind == kPack32 ? 32 : 64;
         if (!d.tpack_valid || d.tpack_prec != prec) {
@@ -1047,7 +1043,12 @@ MixedResult mixed_solve(System &s, DeviceState &d, int M, const double *b, doubl
 // the true one; asking for that much (instead of stopping at the tolerance)
 // makes one refinement step enough for most warm-started solves.
 double refine_eta() { return 1e-6; }
-double refine_frac() { return 0.8; }
+// The last inner solve aims well below the tolerance: a CG iteration reduces the
+// residual by ~0.35, so an aim of f tol ends anywhere in 0.35 f tol .. f tol, and
+// with f = 0.25 the result's error does not depend on where the sums' rounding
+// makes it end (with 0.8 the gradient's error moved by 1.6 times between two
+// summation orders); about one inner iteration more.
+double refine_frac() { return 0.25; }
 
 // ===================================================================== API
 void device_release(System &s) {
@@ -1288,9 +1289,8 @@ size_t device_footprint_estimate(const System &s) {
     size_t b = np * (sizeof(double4) + sizeof(float4) + 3 * sizeof(double) + sizeof(float) + sizeof(int));
     b += nm * (sizeof(double4) + sizeof(double) + sizeof(double) * s.ld_cart + sizeof(int));
     b += sizeof(double) * (2 * n * 2 + n + 8 * 2 * n);     // e_m2d, ipd, ext, work vectors
-    b += 3 * 24 * sizeof(double) * (n / kBlock + 16);      // reduction scratch
-    const int nsplit = tmv_split(s.npol);
-    b += tmv_part_bytes(s.npol, 2, 64, nsplit) + sizeof(double) * n * 16;  // pair and static-field partials
+    b += 3 * 24 * sizeof(double) * (n / kBlock + 16) + 2 * sizeof(double) * tmv_rows_dot_parts(s.npol, 64, 2);  // reductions
+    b += sizeof(double) * n * 16;                          // static-field partials
     if (tmv_pair_once(s.npol, 64, 1) || rhs_pair_once(s.npol)) {  // block-pair partials and list of the pair-once sweeps
         const size_t nb = tmv_sym_blocks(s.npol);
         b += tmv_sym_part_bytes(s.npol, 2, 64) + sizeof(int2) * nb * (nb + 1) / 2;

@@ -179,106 +179,11 @@ void launch_rhs_m2d(hipStream_t st, bool amoeba, int nmm, int npol, const double
     HIP_CHECK(hipGetLastError());
 }
 
-// ============================================================ T on the fly
-// One target per thread, sources through LDS two at a time.  Tiles are padded
-// to an even count with far-away sources of zero dipole, which add exactly 0.
-template <typename R, int M, bool AMOEBA>
-__global__ __launch_bounds__(kBlock) void k_tmv_pairs(int npol, int chunk,
-                                                      const typename V4<R>::t *__restrict__ site,
-                                                      const R *__restrict__ adamp,
-                                                      const double *__restrict__ x, long xstride,
-                                                      R *__restrict__ part, const CgState *__restrict__ skip,
-                                                      int skipM) {
-    using R4 = typename V4<R>::t;
-    if (skip) {
-        bool all = true;
-        for (int m = 0; m < skipM; m++) all = all && skip[m].done;
-        if (all) return;
-    }
-    __shared__ R4 s_pos[kBlock];
-    __shared__ R4 s_x[M][kBlock];  // x, y, z of column m; w of column 0 holds the damping a
-    const int tid = threadIdx.x;
-    const int j = blockIdx.x * kBlock + tid;
-    const bool valid = j < npol;
-    R4 pj;
-    R aj;
-    if (valid) {
-        pj = site[j];
-        aj = adamp[j];
-    } else {
-        pj.x = pj.y = pj.z = R(0);
-        pj.w = R(1);
-        aj = R(0.39);
-    }
-    R acc[M][3];
-#pragma unroll
-    for (int m = 0; m < M; m++) acc[m][0] = acc[m][1] = acc[m][2] = R(0);
-    const int i0 = blockIdx.y * chunk;
-    const int i1 = min(npol, i0 + chunk);
-    for (int base = i0; base < i1; base += kBlock) {
-        const int cnt = min(kBlock, i1 - base);
-        __syncthreads();
-        if (tid < cnt) {
-            const int i = base + tid;
-            s_pos[tid] = site[i];
-#pragma unroll
-            for (int m = 0; m < M; m++) {
-                R4 v;
-                v.x = (R)x[m * xstride + 3L * i + 0];
-                v.y = (R)x[m * xstride + 3L * i + 1];
-                v.z = (R)x[m * xstride + 3L * i + 2];
-                v.w = m == 0 ? adamp[i] : R(0);
-                s_x[m][tid] = v;
-            }
-        } else if (tid == cnt) {
-            R4 far;
-            far.x = far.y = far.z = R(1e15);
-            far.w = R(1);
-            s_pos[tid] = far;
-#pragma unroll
-            for (int m = 0; m < M; m++) {
-                R4 z;
-                z.x = z.y = z.z = R(0);
-                z.w = R(0.39);
-                s_x[m][tid] = z;
-            }
-        }
-        __syncthreads();
-        const int cnt2 = (cnt + 1) & ~1;
-        for (int k = 0; k < cnt2; k += 2) {
-            R4 xa[M], xb[M];
-#pragma unroll
-            for (int m = 0; m < M; m++) {
-                xa[m] = s_x[m][k];
-                xb[m] = s_x[m][k + 1];
-            }
-            R dxa, dya, dza, k2a, k3a, arga, dxb, dyb, dzb, k2b, k3b, argb;
-            bool neara, nearb;
-            pair_geom<R, AMOEBA>(pj, aj, s_pos[k], xa[0].w, dxa, dya, dza, k2a, k3a, arga, neara);
-            pair_geom<R, AMOEBA>(pj, aj, s_pos[k + 1], xb[0].w, dxb, dyb, dzb, k2b, k3b, argb, nearb);
-            if (__ballot(neara || nearb)) {
-                pair_damp<R, AMOEBA>(arga, neara, k2a, k3a);
-                pair_damp<R, AMOEBA>(argb, nearb, k2b, k3b);
-            }
-            pair_accum<R, M>(acc, xa, dxa, dya, dza, k2a, k3a);
-            pair_accum<R, M>(acc, xb, dxb, dyb, dzb, k2b, k3b);
-        }
-    }
-    if (valid) {
-#pragma unroll
-        for (int m = 0; m < M; m++) {
-            R *o = part + ((long)blockIdx.y * M + m) * 3 * npol + 3L * j;
-            o[0] = acc[m][0];
-            o[1] = acc[m][1];
-            o[2] = acc[m][2];
-        }
-    }
-}
-
+// ================================================= T from partial fields
 // y = -(sum of partial fields part[split][m][3 npol]) + corrections (+ x / alpha);
 // optional y.x partials.
-template <typename R, int M, bool AMOEBA>
-__global__ __launch_bounds__(kBlock) void k_tmv_finalize(int npol, int nsplit, const R *__restrict__ part,
+template <int M, bool AMOEBA>
+__global__ __launch_bounds__(kBlock) void k_tmv_finalize(int npol, int nsplit, const double *__restrict__ part,
                                                          const double4 *__restrict__ ps,
                                                          const double *__restrict__ pa,
                                                          const double *__restrict__ alpha,
@@ -304,10 +209,10 @@ __global__ __launch_bounds__(kBlock) void k_tmv_finalize(int npol, int nsplit, c
         for (int s = 0; s < nsplit; s++)
 #pragma unroll
             for (int m = 0; m < M; m++) {
-                const R *p = part + ((long)s * M + m) * 3 * npol + 3L * j;
-                acc[m][0] -= (double)p[0];
-                acc[m][1] -= (double)p[1];
-                acc[m][2] -= (double)p[2];
+                const double *p = part + ((long)s * M + m) * 3 * npol + 3L * j;
+                acc[m][0] -= p[0];
+                acc[m][1] -= p[1];
+                acc[m][2] -= p[2];
             }
     }
     if (valid) {
@@ -375,74 +280,6 @@ int balanced_split(int tb, int nsrc, int num_cu) {
     return best;
 }
 
-int tmv_split(int npol) {
-    static int num_cu = 0;
-    if (num_cu == 0) {
-        int dev = 0;
-        hipDeviceProp_t prop;
-        if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess)
-            num_cu = prop.multiProcessorCount;
-        if (num_cu <= 0) num_cu = 256;
-    }
-    return balanced_split(site_blocks(npol), npol, num_cu);
-}
-
-size_t tmv_part_bytes(int npol, int M, int prec, int nsplit) {
-    return (size_t)nsplit * M * 3 * (size_t)npol * (prec == 32 ? 4 : 8);
-}
-
-template <typename R, int M>
-static void tmv_launch_t(hipStream_t st, bool amoeba, int npol, const typename V4<R>::t *site, const R *ad,
-                         const double4 *ps64, const double *pa64, const double *alpha, const CsrDev &pp,
-                         const double *x, long xs, double *y, long ys, bool dodiag, double *dotpart,
-                         R *part, int nsplit, const CgState *skip, int skipM, hipEvent_t evb, hipEvent_t eve) {
-    const int chunk = (npol + nsplit - 1) / nsplit;
-    dim3 grid(site_blocks(npol), nsplit);
-    if (evb) HIP_CHECK(hipEventRecord(evb, st));
-    if (amoeba)
-        hipLaunchKernelGGL((k_tmv_pairs<R, M, true>), grid, dim3(kBlock), 0, st, npol, chunk, site, ad, x, xs,
-                           part, skip, skipM);
-    else
-        hipLaunchKernelGGL((k_tmv_pairs<R, M, false>), grid, dim3(kBlock), 0, st, npol, chunk, site, ad, x, xs,
-                           part, skip, skipM);
-    HIP_CHECK(hipGetLastError());
-    if (eve) HIP_CHECK(hipEventRecord(eve, st));
-    if (amoeba)
-        hipLaunchKernelGGL((k_tmv_finalize<R, M, true>), dim3(site_blocks(npol)), dim3(kBlock), 0, st, npol,
-                           nsplit, part, ps64, pa64, alpha, pp.ri, pp.ci, pp.f, x, xs, y, ys, (int)dodiag,
-                           dotpart, skip, skipM);
-    else
-        hipLaunchKernelGGL((k_tmv_finalize<R, M, false>), dim3(site_blocks(npol)), dim3(kBlock), 0, st, npol,
-                           nsplit, part, ps64, pa64, alpha, pp.ri, pp.ci, pp.f, x, xs, y, ys, (int)dodiag,
-                           dotpart, skip, skipM);
-    HIP_CHECK(hipGetLastError());
-}
-
-void launch_tmv_otf(hipStream_t st, int prec, bool amoeba, int npol, int M, const double4 *ps64,
-                    const double *pa64, const float4 *ps32, const float *pa32, const double *alpha,
-                    const CsrDev &pp, const double *x, long xstride, double *y, long ystride, bool dodiag,
-                    double *dotpart, void *part, int nsplit, const int *skip_flag, hipEvent_t evb,
-                    hipEvent_t eve) {
-    if (npol == 0) return;
-    const CgState *skip = reinterpret_cast<const CgState *>(skip_flag);
-    const int skipM = M;
-    if (prec == 32) {
-        if (M == 1)
-            tmv_launch_t<float, 1>(st, amoeba, npol, ps32, pa32, ps64, pa64, alpha, pp, x, xstride, y, ystride,
-                                   dodiag, dotpart, (float *)part, nsplit, skip, skipM, evb, eve);
-        else
-            tmv_launch_t<float, 2>(st, amoeba, npol, ps32, pa32, ps64, pa64, alpha, pp, x, xstride, y, ystride,
-                                   dodiag, dotpart, (float *)part, nsplit, skip, skipM, evb, eve);
-    } else {
-        if (M == 1)
-            tmv_launch_t<double, 1>(st, amoeba, npol, ps64, pa64, ps64, pa64, alpha, pp, x, xstride, y, ystride,
-                                    dodiag, dotpart, (double *)part, nsplit, skip, skipM, evb, eve);
-        else
-            tmv_launch_t<double, 2>(st, amoeba, npol, ps64, pa64, ps64, pa64, alpha, pp, x, xstride, y, ystride,
-                                    dodiag, dotpart, (double *)part, nsplit, skip, skipM, evb, eve);
-    }
-}
-
 // Finalize of externally computed FP64 partial fields (the fast multipole
 // path: near and far field as two splits).
 void launch_tmv_finalize64(hipStream_t st, bool amoeba, int npol, int M, const double *part, int nsplit,
@@ -453,16 +290,16 @@ void launch_tmv_finalize64(hipStream_t st, bool amoeba, int npol, int M, const d
     const CgState *skip = reinterpret_cast<const CgState *>(skip_flag);
     const dim3 g(site_blocks(npol)), b(kBlock);
     if (amoeba && M == 1)
-        hipLaunchKernelGGL((k_tmv_finalize<double, 1, true>), g, b, 0, st, npol, nsplit, part, ps64, pa64, alpha,
+        hipLaunchKernelGGL((k_tmv_finalize<1, true>), g, b, 0, st, npol, nsplit, part, ps64, pa64, alpha,
                            pp.ri, pp.ci, pp.f, x, xstride, y, ystride, (int)dodiag, dotpart, skip, M);
     else if (amoeba)
-        hipLaunchKernelGGL((k_tmv_finalize<double, 2, true>), g, b, 0, st, npol, nsplit, part, ps64, pa64, alpha,
+        hipLaunchKernelGGL((k_tmv_finalize<2, true>), g, b, 0, st, npol, nsplit, part, ps64, pa64, alpha,
                            pp.ri, pp.ci, pp.f, x, xstride, y, ystride, (int)dodiag, dotpart, skip, M);
     else if (M == 1)
-        hipLaunchKernelGGL((k_tmv_finalize<double, 1, false>), g, b, 0, st, npol, nsplit, part, ps64, pa64, alpha,
+        hipLaunchKernelGGL((k_tmv_finalize<1, false>), g, b, 0, st, npol, nsplit, part, ps64, pa64, alpha,
                            pp.ri, pp.ci, pp.f, x, xstride, y, ystride, (int)dodiag, dotpart, skip, M);
     else
-        hipLaunchKernelGGL((k_tmv_finalize<double, 2, false>), g, b, 0, st, npol, nsplit, part, ps64, pa64, alpha,
+        hipLaunchKernelGGL((k_tmv_finalize<2, false>), g, b, 0, st, npol, nsplit, part, ps64, pa64, alpha,
                            pp.ri, pp.ci, pp.f, x, xstride, y, ystride, (int)dodiag, dotpart, skip, M);
     HIP_CHECK(hipGetLastError());
 }

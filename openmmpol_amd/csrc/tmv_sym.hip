@@ -184,17 +184,17 @@ int tmv_sym_blocks(int npol) { return (npol + kSymBlock - 1) / kSymBlock; }
 int tmv_sym_dot_parts(int npol) { return tmv_sym_blocks(npol) * kSymSub; }
 
 // The pair-once sweep evaluates half the pairs, at the price of a workgroup per
-// block pair and of its block-pair partial sums; below a few thousand sites it
-// has too few workgroups to fill the chip.  Crossovers against the per-target
-// sweep measured on MI355X (whole matvec, two targets per lane): FP32 two
-// columns ~11,000 sites (-5% at 12,000, -22% at 15,000), one column ~7,000;
-// FP64 two columns ~7,000 (-8% at 8,000), one column ~6,000 (-19% at 8,000).
+// block pair and of its block-pair partial sums; below several thousand sites it
+// has too few workgroups to fill the chip.  Against the per-target sweep
+// (tmv_rows.hip; us per matvec, pair-once / per target): FP64 one column 124 / 131
+// at 8,000 sites and 72 / 59 at 5,003, two columns 153 / 139 and 198 / 251 at 11,000;
+// FP32 one column 62 / 58 and 79 / 101, two columns 86 / 70 and 111 / 129.
 // Used from those sizes while its partial sums for max(ncols, 2) columns stay
-// under max_bytes (2 GiB: up to ~100,000 sites).
-bool tmv_pair_once(int npol, int prec, int ncols, size_t max_bytes) {
-    const int from = prec == 32 ? (ncols >= 2 ? 11000 : 7000) : (ncols >= 2 ? 7000 : 6000);
+// under 2 GiB (up to ~100,000 sites).
+bool tmv_pair_once(int npol, int prec, int ncols) {
+    const int from = prec == 32 ? (ncols >= 2 ? 9500 : 8500) : (ncols >= 2 ? 9000 : 7500);
     if (npol < from) return false;
-    return tmv_sym_part_bytes(npol, ncols > 2 ? ncols : 2, 64) <= max_bytes;
+    return tmv_sym_part_bytes(npol, ncols > 2 ? ncols : 2, 64) <= size_t(2) << 30;
 }
 
 size_t tmv_sym_part_bytes(int npol, int M, int prec) {
