@@ -117,6 +117,7 @@ void launch_rhs_finalize(hipStream_t st, bool amoeba, int npol, int nsplit, cons
                          const double *ma64, const double *mq, const double4 *ps64, const double *pa64,
                          const CsrDev &sp, double *e_m2d);
 int balanced_split(int tb, int nsrc, int num_cu);
+int sweep_split(int tb, int nsrc, int num_cu);
 // FMA rate (TFLOP/s, FMA = 2) of non-packed vector code on the current device,
 // prec 32 or 64: eight independent chains per thread, 8,192 x 256 threads.
 double vector_fma_tflops(int prec);
@@ -135,12 +136,13 @@ void launch_tpack_mv(hipStream_t st, int prec, int npol, int M, const void *tpac
 size_t tpack_part_bytes(int npol, int M);
 
 // Potential and field at n external points cext[n][3] of the multipoles (mm)
-// and/or of the induced dipoles (pol), FP64: out[n] = (V, Ex, Ey, Ez); part
-// holds (smm + spol) * n double4; *bad is set if a point sits on a source.
+// and/or of the induced dipoles (pol), FP64: out[n] = (V, Ex, Ey, Ez), with V or
+// E left 0 where not wanted; part holds (smm + spol) * n double4; *bad is set if
+// a point sits on a source.
 int x2e_splits(int n, int nsrc);
 void launch_x2e(hipStream_t st, int n, const double *cext, bool mm, bool pol, bool amoeba, int ld, int nmm,
-                const double4 *ms, const double *mq, int npol, const double4 *ps, const double *ipd, double4 *part,
-                int smm, int spol, double4 *out, int *bad);
+                const double4 *ms, const double *mq, int npol, const double4 *ps, const double *ipd, bool want_v,
+                bool want_e, double4 *part, int smm, int spol, double4 *out, int *bad);
 
 // The same for the field only, with no allocation: the points cext[n][3] and
 // the field e[n][3] (host, e += result) are staged in a static per-device

@@ -399,10 +399,12 @@ DeviceState &ensure_device(System &s) {
             // the FP64 static-field sweep hides its latency better with about six
             // workgroups per CU than with the ~3 of the balanced split (-8% at 15,000 sites)
             const int tb = std::max(1, site_blocks(s.npol)), ncu = prop.multiProcessorCount;
-            const int max_s = std::max(1, (s.nmm + kBlock - 1) / kBlock);
-            d.rhs_split = std::min(max_s, std::max(balanced_split(tb, s.nmm, ncu), (6 * ncu + tb - 1) / tb));
-            const int nnp = s.nmm - s.npol, max_np = std::max(1, (nnp + kBlock - 1) / kBlock);
-            d.rhs_split_np = std::min(max_np, std::max(balanced_split(tb, std::max(nnp, 1), ncu), (6 * ncu + tb - 1) / tb));
+            auto split = [&](int nsrc) {
+                const int max_s = std::max(1, (nsrc + kBlock - 1) / kBlock);
+                return std::max(sweep_split(tb, nsrc, ncu), std::min(max_s, (6 * ncu + tb - 1) / tb));
+            };
+            d.rhs_split = split(s.nmm);
+            d.rhs_split_np = split(std::max(s.nmm - s.npol, 1));
         }
         d.rhs_part = dalloc<double>(d, (size_t)std::max(d.rhs_split, d.rhs_split_np) * n + 1);
         if (s.nmm > s.npol) {
@@ -1290,7 +1292,7 @@ size_t device_footprint_estimate(const System &s) {
     b += nm * (sizeof(double4) + sizeof(double) + sizeof(double) * s.ld_cart + sizeof(int));
     b += sizeof(double) * (2 * n * 2 + n + 8 * 2 * n);     // e_m2d, ipd, ext, work vectors
     b += 3 * 24 * sizeof(double) * (n / kBlock + 16) + 2 * sizeof(double) * tmv_rows_dot_parts(s.npol, 64, 2);  // reductions
-    b += sizeof(double) * n * 16;                          // static-field partials
+    b += sizeof(double) * n * 16 + (size_t(4) << 20);      // static-field partials
     if (tmv_pair_once(s.npol, 64, 1) || rhs_pair_once(s.npol)) {  // block-pair partials and list of the pair-once sweeps
         const size_t nb = tmv_sym_blocks(s.npol);
         b += tmv_sym_part_bytes(s.npol, 2, 64) + sizeof(int2) * nb * (nb + 1) / 2;
@@ -1465,7 +1467,7 @@ void x2e_host(System &s, int n, const double *cext, bool mm, bool pol, double *V
     HCHECK(hipMemsetAsync(d.x2e_bad, 0, sizeof(int), d.stream));
     HCHECK(hipMemcpyAsync(d.x2e_c, cext, sizeof(double) * 3L * n, hipMemcpyHostToDevice, d.stream));
     launch_x2e(d.stream, n, d.x2e_c, mm, pol, s.amoeba, s.ld_cart, s.nmm, d.ms64, d.mq, s.npol, d.ps64, d.ipd,
-               d.x2e_part, smm, spol, d.x2e_out, d.x2e_bad);
+               V != nullptr, E != nullptr, d.x2e_part, smm, spol, d.x2e_out, d.x2e_bad);
     HCHECK(hipMemcpyAsync(out.data(), d.x2e_out, sizeof(double) * 4L * n, hipMemcpyDeviceToHost, d.stream));
     HCHECK(hipMemcpyAsync(&bad, d.x2e_bad, sizeof(int), hipMemcpyDeviceToHost, d.stream));
     HCHECK(hipStreamSynchronize(d.stream));
@@ -1550,9 +1552,9 @@ void ensure_grad(System &s, DeviceState &d) {
     int cu = 0;
     HCHECK(hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, d.device));
     cu = std::max(cu, 1);
-    d.g_split_s = balanced_split(site_blocks(npol), nmm, cu);
-    d.g_split_p = balanced_split(site_blocks(npol), npol, cu);
-    d.g_split_m = balanced_split(site_blocks(nmm), npol, cu);
+    d.g_split_s = sweep_split(site_blocks(npol), nmm, cu);
+    d.g_split_p = sweep_split(site_blocks(npol), npol, cu);
+    d.g_split_m = sweep_split(site_blocks(nmm), npol, cu);
     // partials of the per-target sweeps, or of the both-ends static sweep
     // (one per block of the other end) and the dipole-dipole part
     const bool both = grad_both_ends(npol, nmm, s.amoeba);

@@ -31,6 +31,7 @@
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
+#include <type_traits>
 
 #include "device.h"
 #include "grad_math.h"
@@ -328,15 +329,15 @@ __global__ __launch_bounds__(4 * kSymBlock) void k_sym3_reduce(int npol, int nb,
     }
 }
 
-// The finalizes take 64 sites per workgroup with kGfQ groups of 64 threads:
-// group q sums every kGfQ-th partial and every kGfQ-th listed pair of its
-// site, and group 0 adds the group results in a fixed order (one thread per
-// site waited on the latency of its whole chain of partials and pairs).
-constexpr int kGfQ = 4;
-constexpr int kGfSites = kBlock / kGfQ;
-static_assert(kGfSites == 64, "one wave of sites per group");
-
-template <bool AMOEBA>
+// The finalizes take kBlock / NG sites per workgroup with NG groups of threads:
+// group q sums every NG-th partial and every NG-th listed pair of its site, and
+// group 0 adds the group results in a fixed order (one thread per site waited on
+// the latency of its whole chain of partials and pairs).  Sixteen groups below
+// kGfWide sites, where the workgroups are few and a site has up to ~100 partials
+// (648 sites: 12 -> 8 us); above, four, whose rows of 64 sites read whole lines
+// (20,001 sites: 47 -> 32 us for the MM end).
+constexpr int kGfWide = 5000;
+template <bool AMOEBA, int NG>
 __global__ __launch_bounds__(kBlock) void k_gpol_finalize(int npol, int nparts, const double *__restrict__ part,
                                                           const double4 *__restrict__ ms,
                                                           const double *__restrict__ ma,
@@ -351,14 +352,14 @@ __global__ __launch_bounds__(kBlock) void k_gpol_finalize(int npol, int nparts, 
                                                           const double *__restrict__ pp_f,
                                                           double *__restrict__ gpol) {
     constexpr int LD = AMOEBA ? 10 : 1;
-    __shared__ double sh[kGfQ - 1][3][kGfSites];
-    const int q = threadIdx.x / kGfSites, li = threadIdx.x % kGfSites;
-    const int j = blockIdx.x * kGfSites + li;
+    __shared__ double sh[NG - 1][3][(kBlock / NG)];
+    const int q = threadIdx.x / (kBlock / NG), li = threadIdx.x % (kBlock / NG);
+    const int j = blockIdx.x * (kBlock / NG) + li;
     const bool valid = j < npol;
     const long n = 3L * npol;
     double gx = 0.0, gy = 0.0, gz = 0.0;
     if (valid) {
-        for (int s = q; s < nparts; s += kGfQ) {
+        for (int s = q; s < nparts; s += NG) {
             const double *p = part + (long)s * 3 * npol;
             gx += p[j];
             gy += p[npol + j];
@@ -371,7 +372,7 @@ __global__ __launch_bounds__(kBlock) void k_gpol_finalize(int npol, int nparts, 
                      pZ = AMOEBA ? ipd[n + 3L * j + 2] : dZ;
         // listed static sources: remove (1 - s_p) of the mu_D contraction and
         // (1 - s_d) of the mu_P one (AMBER: both slots hold 1 - s)
-        for (int k = sp_ri[j] + q; k < sp_ri[j + 1]; k += kGfQ) {
+        for (int k = sp_ri[j] + q; k < sp_ri[j + 1]; k += NG) {
             const int i = sp_ci[k];
             const double2 f = sp_f[k];
             const double wx = AMOEBA ? 0.5 * (f.y * dX + f.x * pX) : f.y * dX;
@@ -391,7 +392,7 @@ __global__ __launch_bounds__(kBlock) void k_gpol_finalize(int npol, int nparts, 
             gz -= cz;
         }
         // listed dipole sources: remove (1 - s_u) of the pair
-        for (int k = pp_ri[j] + q; k < pp_ri[j + 1]; k += kGfQ) {
+        for (int k = pp_ri[j] + q; k < pp_ri[j + 1]; k += NG) {
             const int i = pp_ci[k];
             const double4 pi = ps[i];
             const double dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
@@ -421,7 +422,7 @@ __global__ __launch_bounds__(kBlock) void k_gpol_finalize(int npol, int nparts, 
     }
     __syncthreads();
     if (q != 0 || !valid) return;
-    for (int g = 0; g < kGfQ - 1; g++) {
+    for (int g = 0; g < NG - 1; g++) {
         gx += sh[g][0][li];
         gy += sh[g][1][li];
         gz += sh[g][2][li];
@@ -600,7 +601,7 @@ __global__ __launch_bounds__(kBlock) void k_gstat_both(int nmm, int npol, const 
 // -q E + mu . Egrd - Q : EHes -> gtr[m][3].  direct (AMOEBA): the partials'
 // entries 9-11 hold the translational gradient itself (k_gstat_both), and the
 // formula applies to the listed-pair corrections only.
-template <bool AMOEBA>
+template <bool AMOEBA, int NG>
 __global__ __launch_bounds__(kBlock) void k_gmm_finalize(int nmm, int npol, int nparts, int direct,
                                                          const double *__restrict__ part,
                                                          const double4 *__restrict__ ms,
@@ -613,9 +614,9 @@ __global__ __launch_bounds__(kBlock) void k_gmm_finalize(int nmm, int npol, int 
                                                          double *__restrict__ egrd, double *__restrict__ gtr) {
     constexpr int NA = AMOEBA ? 12 : 3;
     constexpr int LD = AMOEBA ? 10 : 1;
-    __shared__ double sh[kGfQ - 1][2 * NA][kGfSites];
-    const int qg = threadIdx.x / kGfSites, li = threadIdx.x % kGfSites;
-    const int m = blockIdx.x * kGfSites + li;
+    __shared__ double sh[NG - 1][2 * NA][(kBlock / NG)];
+    const int qg = threadIdx.x / (kBlock / NG), li = threadIdx.x % (kBlock / NG);
+    const int m = blockIdx.x * (kBlock / NG) + li;
     const bool valid = m < nmm;
     const long n = 3L * npol;
     double acc[NA], corr[NA];
@@ -625,14 +626,14 @@ __global__ __launch_bounds__(kBlock) void k_gmm_finalize(int nmm, int npol, int 
     const double *Q = q + (AMOEBA ? 4 : 0);
     const double trQ = AMOEBA ? Q[0] + Q[2] + Q[5] : 0.0;
     if (valid) {
-        for (int s = qg; s < nparts; s += kGfQ) {
+        for (int s = qg; s < nparts; s += NG) {
             const double *p = part + (long)s * NA * nmm;
             for (int c = 0; c < NA; c++) acc[c] += p[(long)c * nmm + m];
         }
         const double4 pm = ms[m];
         const double am = ma[m];
         // listed sources: remove 1/2 ((1 - s_d) mu_P + (1 - s_p) mu_D) (AMBER: (1 - s) mu)
-        for (int k = mp_ri[m] + qg; k < mp_ri[m + 1]; k += kGfQ) {
+        for (int k = mp_ri[m] + qg; k < mp_ri[m + 1]; k += NG) {
             const int i = mp_ci[k];
             const double2 f = mp_f[k];
             double nx, ny, nz;
@@ -661,7 +662,7 @@ __global__ __launch_bounds__(kBlock) void k_gmm_finalize(int nmm, int npol, int 
     }
     __syncthreads();
     if (qg != 0 || !valid) return;
-    for (int g = 0; g < kGfQ - 1; g++)
+    for (int g = 0; g < NG - 1; g++)
         for (int c = 0; c < NA; c++) {
             acc[c] += sh[g][c][li];
             corr[c] += sh[g][NA + c][li];
@@ -896,23 +897,23 @@ void launch_geomgrad(hipStream_t st, const GradArgs &a, hipEvent_t evb, hipEvent
 void launch_geomgrad_finish(hipStream_t st, const GradArgs &a, int nparts_pol, int nparts_mm, bool direct) {
     const int nmm = a.nmm, npol = a.npol;
     const int mb = (nmm + kBlock - 1) / kBlock;
-    const int pbf = (npol + kGfSites - 1) / kGfSites, mbf = (nmm + kGfSites - 1) / kGfSites;
     if (npol > 0) {
-        if (a.amoeba) {
-            hipLaunchKernelGGL(k_gpol_finalize<true>, dim3(pbf), dim3(kBlock), 0, st, npol, nparts_pol, a.part_pol,
-                               a.ms, a.ma, a.mq, a.ps, a.pa, a.ipd, a.sp.ri, a.sp.ci, a.sp.f2, a.pp.ri, a.pp.ci,
-                               a.pp.f, a.gpol);
-            hipLaunchKernelGGL(k_gmm_finalize<true>, dim3(mbf), dim3(kBlock), 0, st, nmm, npol, nparts_mm,
-                               (int)direct, a.part_mm, a.ms, a.ma, a.mq, a.ps, a.pa, a.ipd, a.mp.ri, a.mp.ci,
-                               a.mp.f2, a.emm, a.egrd, a.gtr);
-        } else {
-            hipLaunchKernelGGL(k_gpol_finalize<false>, dim3(pbf), dim3(kBlock), 0, st, npol, nparts_pol, a.part_pol,
-                               a.ms, a.ma, a.mq, a.ps, a.pa, a.ipd, a.sp.ri, a.sp.ci, a.sp.f2, a.pp.ri, a.pp.ci,
-                               a.pp.f, a.gpol);
-            hipLaunchKernelGGL(k_gmm_finalize<false>, dim3(mbf), dim3(kBlock), 0, st, nmm, npol, nparts_mm,
-                               (int)direct, a.part_mm, a.ms, a.ma, a.mq, a.ps, a.pa, a.ipd, a.mp.ri, a.mp.ci,
-                               a.mp.f2, a.emm, a.egrd, a.gtr);
-        }
+        auto go = [&](auto am, auto groups) {
+            constexpr bool A = decltype(am)::value;
+            constexpr int Q = decltype(groups)::value, per = kBlock / Q;
+            hipLaunchKernelGGL((k_gpol_finalize<A, Q>), dim3((npol + per - 1) / per), dim3(kBlock), 0, st, npol,
+                               nparts_pol, a.part_pol, a.ms, a.ma, a.mq, a.ps, a.pa, a.ipd, a.sp.ri, a.sp.ci, a.sp.f2,
+                               a.pp.ri, a.pp.ci, a.pp.f, a.gpol);
+            hipLaunchKernelGGL((k_gmm_finalize<A, Q>), dim3((nmm + per - 1) / per), dim3(kBlock), 0, st, nmm, npol,
+                               nparts_mm, (int)direct, a.part_mm, a.ms, a.ma, a.mq, a.ps, a.pa, a.ipd, a.mp.ri,
+                               a.mp.ci, a.mp.f2, a.emm, a.egrd, a.gtr);
+        };
+        auto width = [&](auto am) {
+            if (nmm < kGfWide) go(am, std::integral_constant<int, 16>{});
+            else go(am, std::integral_constant<int, 4>{});
+        };
+        if (a.amoeba) width(std::true_type{});
+        else width(std::false_type{});
         HIP_CHECK(hipGetLastError());
     }
     if (a.amoeba) {

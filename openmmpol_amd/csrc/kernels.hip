@@ -88,6 +88,12 @@ __global__ __launch_bounds__(kBlock) void k_rhs_pairs(int nsrc, int npol, int ch
     }
 }
 
+// E_M2D from the partial fields part[split][3 npol]: kRfQ groups of kRfSites
+// threads per workgroup of kRfSites sites; group q adds every kRfQ-th split and
+// every kRfQ-th listed pair (f = 1 - s for the D and P sets), group 0 the group
+// results in a fixed order (one thread per site waited on its whole chain of
+// splits: 31 us for 1,295 sites and 94 splits).
+constexpr int kRfQ = 16, kRfSites = kBlock / kRfQ;
 template <bool AMOEBA>
 __global__ __launch_bounds__(kBlock) void k_rhs_finalize(int npol, int nsplit, const double *__restrict__ part,
                                                          const double4 *__restrict__ ms,
@@ -100,35 +106,52 @@ __global__ __launch_bounds__(kBlock) void k_rhs_finalize(int npol, int nsplit, c
                                                          const double2 *__restrict__ sp_f,
                                                          double *__restrict__ e_m2d) {
     constexpr int LD = AMOEBA ? 10 : 1;
-    const int j = blockIdx.x * kBlock + threadIdx.x;
-    if (j >= npol) return;
-    double e[3] = {0.0, 0.0, 0.0};
-    for (int s = 0; s < nsplit; s++) {
-        const double *p = part + (long)s * 3 * npol + 3L * j;
-        e[0] += p[0];
-        e[1] += p[1];
-        e[2] += p[2];
+    __shared__ double sh[kRfQ - 1][6][kRfSites];
+    const int q = threadIdx.x / kRfSites, li = threadIdx.x % kRfSites;
+    const int j = blockIdx.x * kRfSites + li;
+    const bool valid = j < npol;
+    double ed[3] = {0.0, 0.0, 0.0}, ep[3] = {0.0, 0.0, 0.0};
+    if (valid) {
+        double e[3] = {0.0, 0.0, 0.0};
+        for (int s = q; s < nsplit; s += kRfQ) {
+            const double *p = part + (long)s * 3 * npol + 3L * j;
+            e[0] += p[0];
+            e[1] += p[1];
+            e[2] += p[2];
+        }
+        for (int c = 0; c < 3; c++) ed[c] = ep[c] = e[c];
+        const double4 pj = ps[j];
+        const double aj = pa[j];
+        for (int k = sp_ri[j] + q; k < sp_ri[j + 1]; k += kRfQ) {
+            const int i = sp_ci[k];
+            const double2 f = sp_f[k];
+            const double4 pi = ms[i];
+            const double dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
+            const double ir = rsqrt(dx * dx + dy * dy + dz * dz);
+            double qs[LD];
+            for (int c = 0; c < LD; c++) qs[c] = mq[(long)LD * i + c];
+            double fx, fy, fz;
+            m2d_pair<AMOEBA>(dx, dy, dz, ir, pi.w, pj.w, ma[i], aj, qs, fx, fy, fz);
+            ed[0] -= f.x * fx;
+            ed[1] -= f.x * fy;
+            ed[2] -= f.x * fz;
+            ep[0] -= f.y * fx;
+            ep[1] -= f.y * fy;
+            ep[2] -= f.y * fz;
+        }
     }
-    double ed[3] = {e[0], e[1], e[2]}, ep[3] = {e[0], e[1], e[2]};
-    const double4 pj = ps[j];
-    const double aj = pa[j];
-    for (int k = sp_ri[j]; k < sp_ri[j + 1]; k++) {
-        const int i = sp_ci[k];
-        const double2 f = sp_f[k];
-        const double4 pi = ms[i];
-        const double dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
-        const double ir = rsqrt(dx * dx + dy * dy + dz * dz);
-        double q[LD];
-        for (int c = 0; c < LD; c++) q[c] = mq[(long)LD * i + c];
-        double fx, fy, fz;
-        m2d_pair<AMOEBA>(dx, dy, dz, ir, pi.w, pj.w, ma[i], aj, q, fx, fy, fz);
-        ed[0] -= f.x * fx;
-        ed[1] -= f.x * fy;
-        ed[2] -= f.x * fz;
-        ep[0] -= f.y * fx;
-        ep[1] -= f.y * fy;
-        ep[2] -= f.y * fz;
-    }
+    if (q > 0)
+        for (int c = 0; c < 3; c++) {
+            sh[q - 1][c][li] = ed[c];
+            sh[q - 1][3 + c][li] = ep[c];
+        }
+    __syncthreads();
+    if (q != 0 || !valid) return;
+    for (int g = 0; g < kRfQ - 1; g++)
+        for (int c = 0; c < 3; c++) {
+            ed[c] += sh[g][c][li];
+            ep[c] += sh[g][3 + c][li];
+        }
     if (AMOEBA) {
         for (int c = 0; c < 3; c++) {
             e_m2d[3L * j + c] = ed[c];
@@ -171,10 +194,10 @@ void launch_rhs_m2d(hipStream_t st, bool amoeba, int nmm, int npol, const double
     HIP_CHECK(hipGetLastError());
     if (eve) HIP_CHECK(hipEventRecord(eve, st));
     if (amoeba)
-        hipLaunchKernelGGL(k_rhs_finalize<true>, dim3(site_blocks(npol)), dim3(kBlock), 0, st, npol, nsplit,
+        hipLaunchKernelGGL(k_rhs_finalize<true>, dim3((npol + kRfSites - 1) / kRfSites), dim3(kBlock), 0, st, npol, nsplit,
                            part, ms64, ma64, mq, ps64, pa64, sp.ri, sp.ci, sp.f2, e_m2d);
     else
-        hipLaunchKernelGGL(k_rhs_finalize<false>, dim3(site_blocks(npol)), dim3(kBlock), 0, st, npol, nsplit,
+        hipLaunchKernelGGL(k_rhs_finalize<false>, dim3((npol + kRfSites - 1) / kRfSites), dim3(kBlock), 0, st, npol, nsplit,
                            part, ms64, ma64, mq, ps64, pa64, sp.ri, sp.ci, sp.f2, e_m2d);
     HIP_CHECK(hipGetLastError());
 }
@@ -280,6 +303,16 @@ int balanced_split(int tb, int nsrc, int num_cu) {
     return best;
 }
 
+// Source splits of an FP64 sweep with one target per thread: a thread's sources
+// are one serial chain, so a few target blocks are cut into thin splits, down to
+// 16 sources, until there are two workgroups per CU (per sweep at 648 sites, 3
+// splits of 216 -> 41 of 16: static field 68 -> 8 us, gradient 70-89 -> 8-13 us);
+// from there on balanced_split.
+int sweep_split(int tb, int nsrc, int num_cu) {
+    const int thin = std::min((nsrc + 15) / 16, (2 * num_cu + tb - 1) / std::max(tb, 1));
+    return std::max(1, std::max(thin, balanced_split(tb, nsrc, num_cu)));
+}
+
 // Finalize of externally computed FP64 partial fields (the fast multipole
 // path: near and far field as two splits).
 void launch_tmv_finalize64(hipStream_t st, bool amoeba, int npol, int M, const double *part, int nsplit,
@@ -309,10 +342,10 @@ void launch_rhs_finalize(hipStream_t st, bool amoeba, int npol, int nsplit, cons
                          const CsrDev &sp, double *e_m2d) {
     if (npol == 0) return;
     if (amoeba)
-        hipLaunchKernelGGL(k_rhs_finalize<true>, dim3(site_blocks(npol)), dim3(kBlock), 0, st, npol, nsplit, part,
+        hipLaunchKernelGGL(k_rhs_finalize<true>, dim3((npol + kRfSites - 1) / kRfSites), dim3(kBlock), 0, st, npol, nsplit, part,
                            ms64, ma64, mq, ps64, pa64, sp.ri, sp.ci, sp.f2, e_m2d);
     else
-        hipLaunchKernelGGL(k_rhs_finalize<false>, dim3(site_blocks(npol)), dim3(kBlock), 0, st, npol, nsplit, part,
+        hipLaunchKernelGGL(k_rhs_finalize<false>, dim3((npol + kRfSites - 1) / kRfSites), dim3(kBlock), 0, st, npol, nsplit, part,
                            ms64, ma64, mq, ps64, pa64, sp.ri, sp.ci, sp.f2, e_m2d);
     HIP_CHECK(hipGetLastError());
 }

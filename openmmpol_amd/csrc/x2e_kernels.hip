@@ -1,9 +1,13 @@
 // Potential and field of the static multipoles and of the induced dipoles at
 // arbitrary external points (potential_M2E / potential_D2E / field_M2E /
 // field_D2E, mod_electrostatics.F90:3067-3336): undamped, unscreened, FP64.
-// One thread per external point, sources staged through LDS in tiles of 256,
-// the source range split over gridDim.y; the per-split partial results are
-// added in a fixed order by the finalize kernel.
+// One thread per 1, 2 or 4 external points, sources staged through LDS in tiles of 256,
+// the source range split over gridDim.y (down to 16 sources a split where there
+// are few points: 30 points and 2,001 sources 34 -> 6 us); the per-split partial
+// results are added in a fixed order by the finalize kernel.  The sweeps are
+// bound by the FP64 vector ALUs and form the potential, the field or both as the
+// entry point asks (20,000 points, 24,000 multipoles, potential alone: 1,238 -> 564 us with
+// four points per thread and the quadrupole as a quadratic form, 38 instructions a pair).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -11,32 +15,70 @@
 #include <cstdlib>
 #include <mutex>
 #include <string>
+#include <type_traits>
 
 #include "device.h"
+#include "pair_math.h"
 
 namespace ommp {
 
 constexpr double kEps2 = kEpsRpDev * kEpsRpDev;
 
+// d and 1/r of one source and a thread's P points.  1/r is the refined hardware
+// estimate; where some lane's r2 is not clearly between kEps2 and 1e300 (one test
+// of the high word for all P, a branch that is never taken in earnest) the
+// general routine is used instead, and 0 with *hit set for a point on the source.
+template <int P>
+__device__ __forceinline__ void x2e_geom(const double (&px)[P], const double (&py)[P], const double (&pz)[P],
+                                         const double4 &s, double (&dx)[P], double (&dy)[P], double (&dz)[P],
+                                         double (&k1)[P], int &hit) {
+    constexpr unsigned lo = 0x3A500000u, span = 0x7E370000u - lo;  // high words above kEps2 = 4.93e-28 and below 1e300
+    static_assert(kEps2 < 5e-28, "lo is the high word of 8.1e-28");
+    unsigned odd = 0;
+#pragma unroll
+    for (int h = 0; h < P; h++) {
+        dx[h] = px[h] - s.x;
+        dy[h] = py[h] - s.y;
+        dz[h] = pz[h] - s.z;
+        const double r2 = fma(dz[h], dz[h], fma(dy[h], dy[h], dx[h] * dx[h]));
+        odd = max(odd, (unsigned)__double2hiint(r2) - lo);
+        k1[h] = fast_rsqrt(r2);
+    }
+    if (__ballot(odd >= span)) {
+#pragma unroll
+        for (int h = 0; h < P; h++) {
+            double r2 = fma(dz[h], dz[h], fma(dy[h], dy[h], dx[h] * dx[h]));
+            asm volatile("" : "+v"(r2));  // keeps the general routine's work inside the branch
+            if (r2 < kEps2) hit = 1;
+            k1[h] = r2 < kEps2 ? 0.0 : rsqrt(r2);
+        }
+    }
+}
+
+// P points per thread (x2e_points): every source read from LDS then meets P
+// points; with one point per thread the sweep waits on the LDS (14 broadcast
+// doubles per multipole).
+//
 // Multipole sources: ms[i] = (x, y, z, .), mq[i][LD] = q, mu, quadrupole / 3
 // (xx, xy, yy, xz, yz, zz).  V = q k1 + (mu.d) k2 + 3 (d.Q d) k3;
 // E = q k2 d + 3 (mu.d) k3 d - k2 mu + 15 (d.Q d) k4 d - 6 k3 Q d, d = r_ext - r_i.
-template <int LD>
+template <int LD, bool V, bool E, int P>
 __global__ __launch_bounds__(kBlock) void k_m2e(int n, const double *__restrict__ cext, int nsrc, int chunk,
                                                 const double4 *__restrict__ ms, const double *__restrict__ mq,
                                                 double4 *__restrict__ part, int *__restrict__ bad) {
     __shared__ double4 s_pos[kBlock];
-    __shared__ double s_q[LD][kBlock];
+    __shared__ double s_q[kBlock][LD];
     const int tid = threadIdx.x;
-    const int j = blockIdx.x * kBlock + tid;
-    const bool valid = j < n;
-    double px = 0.0, py = 0.0, pz = 0.0;
-    if (valid) {
-        px = cext[3L * j];
-        py = cext[3L * j + 1];
-        pz = cext[3L * j + 2];
+    const int j0 = blockIdx.x * kBlock * P + tid;  // points j0, j0 + kBlock, ...
+    double px[P], py[P], pz[P], v[P], ex[P], ey[P], ez[P];
+#pragma unroll
+    for (int h = 0; h < P; h++) {
+        const int j = min(j0 + h * kBlock, n - 1);  // past the end: the last point again, not written
+        px[h] = cext[3L * j];
+        py[h] = cext[3L * j + 1];
+        pz[h] = cext[3L * j + 2];
+        v[h] = ex[h] = ey[h] = ez[h] = 0.0;
     }
-    double v = 0.0, ex = 0.0, ey = 0.0, ez = 0.0;
     int hit = 0;
     const int i0 = blockIdx.y * chunk;
     const int i1 = min(nsrc, i0 + chunk);
@@ -46,61 +88,81 @@ __global__ __launch_bounds__(kBlock) void k_m2e(int n, const double *__restrict_
         if (tid < cnt) {
             s_pos[tid] = ms[base + tid];
 #pragma unroll
-            for (int c = 0; c < LD; c++) s_q[c][tid] = mq[(long)LD * (base + tid) + c];
+            for (int c = 0; c < LD; c++) {
+                const double v = mq[(long)LD * (base + tid) + c];
+                // the potential alone takes 3 d.Q d as a quadratic form: its factors
+                // are put into the coefficients here
+                s_q[tid][c] = E || c < 4 ? v : (c == 4 || c == 6 || c == 9 ? 3.0 * v : 6.0 * v);
+            }
         }
         __syncthreads();
-        if (!valid) continue;
         for (int k = 0; k < cnt; k++) {
-            const double dx = px - s_pos[k].x, dy = py - s_pos[k].y, dz = pz - s_pos[k].z;
-            const double r2 = dx * dx + dy * dy + dz * dz;
-            if (r2 < kEps2) {
-                hit = 1;
-                continue;
-            }
-            const double k1 = rsqrt(r2), ir2 = k1 * k1, k2 = k1 * ir2;
-            const double q = s_q[0][k];
-            if (LD == 1) {
-                v += q * k1;
-                ex += q * k2 * dx;
-                ey += q * k2 * dy;
-                ez += q * k2 * dz;
-            } else {
-                const double k3 = k2 * ir2, k4 = k3 * ir2;
-                const double mx = s_q[1][k], my = s_q[2][k], mz = s_q[3][k];
-                const double md = mx * dx + my * dy + mz * dz;
-                const double qx = s_q[4][k] * dx + s_q[5][k] * dy + s_q[7][k] * dz;
-                const double qy = s_q[5][k] * dx + s_q[6][k] * dy + s_q[8][k] * dz;
-                const double qz = s_q[7][k] * dx + s_q[8][k] * dy + s_q[9][k] * dz;
-                const double qrr = qx * dx + qy * dy + qz * dz;
-                v += q * k1 + md * k2 + 3.0 * qrr * k3;
-                const double cd = q * k2 + 3.0 * md * k3 + 15.0 * qrr * k4;
-                ex += cd * dx - mx * k2 - 6.0 * qx * k3;
-                ey += cd * dy - my * k2 - 6.0 * qy * k3;
-                ez += cd * dz - mz * k2 - 6.0 * qz * k3;
+            const double4 ps = s_pos[k];
+            double m[LD];
+#pragma unroll
+            for (int c = 0; c < LD; c++) m[c] = s_q[k][c];
+            double ax[P], ay[P], az[P], ak[P];
+            x2e_geom<P>(px, py, pz, ps, ax, ay, az, ak, hit);
+#pragma unroll
+            for (int h = 0; h < P; h++) {
+                const double dx = ax[h], dy = ay[h], dz = az[h], k1 = ak[h], ir2 = k1 * k1;
+                if (LD == 1) {
+                    if (V) v[h] += m[0] * k1;
+                    if (E) {
+                        const double c = m[0] * (k1 * ir2);
+                        ex[h] += c * dx;
+                        ey[h] += c * dy;
+                        ez[h] += c * dz;
+                    }
+                } else {
+                    const double md = m[1] * dx + m[2] * dy + m[3] * dz;
+                    if (!E) {
+                        const double q3 = (m[4] * dx + m[5] * dy + m[7] * dz) * dx + (m[6] * dy + m[8] * dz) * dy +
+                                          m[9] * dz * dz;
+                        v[h] += k1 * (m[0] + ir2 * (md + ir2 * q3));
+                        continue;
+                    }
+                    const double qx = m[4] * dx + m[5] * dy + m[7] * dz;
+                    const double qy = m[5] * dx + m[6] * dy + m[8] * dz;
+                    const double qz = m[7] * dx + m[8] * dy + m[9] * dz;
+                    const double q3 = 3.0 * (qx * dx + qy * dy + qz * dz);
+                    if (V) v[h] += k1 * (m[0] + ir2 * (md + ir2 * q3));
+                    const double k2 = k1 * ir2, k3 = k2 * ir2;
+                    const double cd = k2 * (m[0] + ir2 * (3.0 * md + ir2 * (5.0 * q3)));
+                    ex[h] += cd * dx - m[1] * k2 - 6.0 * qx * k3;
+                    ey[h] += cd * dy - m[2] * k2 - 6.0 * qy * k3;
+                    ez[h] += cd * dz - m[3] * k2 - 6.0 * qz * k3;
+                }
             }
         }
     }
-    if (valid) part[(long)blockIdx.y * n + j] = make_double4(v, ex, ey, ez);
+#pragma unroll
+    for (int h = 0; h < P; h++) {
+        const int j = j0 + h * kBlock;
+        if (j < n) part[(long)blockIdx.y * n + j] = make_double4(v[h], ex[h], ey[h], ez[h]);
+    }
     if (hit) *bad = 1;
 }
 
 // Induced-dipole sources: ps[i] = position, potential from muV (the D set for
 // AMOEBA), field from muE (1/2 (mu_D + mu_P) for AMOEBA, mod_electrostatics.F90:3250).
+template <bool V, bool E, int P>
 __global__ __launch_bounds__(kBlock) void k_d2e(int n, const double *__restrict__ cext, int nsrc, int chunk,
                                                 const double4 *__restrict__ ps, const double *__restrict__ ipd,
                                                 int amoeba, double4 *__restrict__ part, int *__restrict__ bad) {
     __shared__ double4 s_pos[kBlock];
     __shared__ double s_mv[3][kBlock], s_me[3][kBlock];
     const int tid = threadIdx.x;
-    const int j = blockIdx.x * kBlock + tid;
-    const bool valid = j < n;
-    double px = 0.0, py = 0.0, pz = 0.0;
-    if (valid) {
-        px = cext[3L * j];
-        py = cext[3L * j + 1];
-        pz = cext[3L * j + 2];
+    const int j0 = blockIdx.x * kBlock * P + tid;
+    double px[P], py[P], pz[P], v[P], ex[P], ey[P], ez[P];
+#pragma unroll
+    for (int h = 0; h < P; h++) {
+        const int j = min(j0 + h * kBlock, n - 1);
+        px[h] = cext[3L * j];
+        py[h] = cext[3L * j + 1];
+        pz[h] = cext[3L * j + 2];
+        v[h] = ex[h] = ey[h] = ez[h] = 0.0;
     }
-    double v = 0.0, ex = 0.0, ey = 0.0, ez = 0.0;
     int hit = 0;
     const int i0 = blockIdx.y * chunk;
     const int i1 = min(nsrc, i0 + chunk);
@@ -115,78 +177,122 @@ __global__ __launch_bounds__(kBlock) void k_d2e(int n, const double *__restrict_
             for (int c = 0; c < 3; c++) {
                 const double d = ipd[3 * i + c];
                 s_mv[c][tid] = d;
-                s_me[c][tid] = amoeba ? 0.5 * (ipd[np3 + 3 * i + c] + d) : d;
+                if (E) s_me[c][tid] = amoeba ? 0.5 * (ipd[np3 + 3 * i + c] + d) : d;
             }
         }
         __syncthreads();
-        if (!valid) continue;
         for (int k = 0; k < cnt; k++) {
-            const double dx = px - s_pos[k].x, dy = py - s_pos[k].y, dz = pz - s_pos[k].z;
-            const double r2 = dx * dx + dy * dy + dz * dz;
-            if (r2 < kEps2) {
-                hit = 1;
-                continue;
+            const double4 q = s_pos[k];
+            const double vx = s_mv[0][k], vy = s_mv[1][k], vz = s_mv[2][k];
+            const double mx = E ? s_me[0][k] : 0.0, my = E ? s_me[1][k] : 0.0, mz = E ? s_me[2][k] : 0.0;
+            double ax[P], ay[P], az[P], ak[P];
+            x2e_geom<P>(px, py, pz, q, ax, ay, az, ak, hit);
+#pragma unroll
+            for (int h = 0; h < P; h++) {
+                const double dx = ax[h], dy = ay[h], dz = az[h], k1 = ak[h], ir2 = k1 * k1, k2 = k1 * ir2;
+                if (V) v[h] += (vx * dx + vy * dy + vz * dz) * k2;
+                if (E) {
+                    const double c3 = 3.0 * (mx * dx + my * dy + mz * dz) * (k2 * ir2);
+                    ex[h] += c3 * dx - mx * k2;
+                    ey[h] += c3 * dy - my * k2;
+                    ez[h] += c3 * dz - mz * k2;
+                }
             }
-            const double k1 = rsqrt(r2), ir2 = k1 * k1, k2 = k1 * ir2, k3 = k2 * ir2;
-            v += (s_mv[0][k] * dx + s_mv[1][k] * dy + s_mv[2][k] * dz) * k2;
-            const double mx = s_me[0][k], my = s_me[1][k], mz = s_me[2][k];
-            const double c3 = 3.0 * (mx * dx + my * dy + mz * dz) * k3;
-            ex += c3 * dx - mx * k2;
-            ey += c3 * dy - my * k2;
-            ez += c3 * dz - mz * k2;
         }
     }
-    if (valid) part[(long)blockIdx.y * n + j] = make_double4(v, ex, ey, ez);
+#pragma unroll
+    for (int h = 0; h < P; h++) {
+        const int j = j0 + h * kBlock;
+        if (j < n) part[(long)blockIdx.y * n + j] = make_double4(v[h], ex[h], ey[h], ez[h]);
+    }
     if (hit) *bad = 1;
 }
 
+// kXfQ groups of kXfPts threads per workgroup of kXfPts points: group q adds
+// every kXfQ-th partial, group 0 the group results in a fixed order.
+constexpr int kXfQ = 16, kXfPts = kBlock / kXfQ;
 __global__ __launch_bounds__(kBlock) void k_x2e_finalize(int n, int nparts, const double4 *__restrict__ part,
                                                          double4 *__restrict__ out) {
-    const int j = blockIdx.x * kBlock + threadIdx.x;
-    if (j >= n) return;
+    __shared__ double4 sh[kXfQ - 1][kXfPts];
+    const int q = threadIdx.x / kXfPts, li = threadIdx.x % kXfPts;
+    const int j = blockIdx.x * kXfPts + li;
     double4 a = make_double4(0.0, 0.0, 0.0, 0.0);
-    for (int s = 0; s < nparts; s++) {
-        const double4 p = part[(long)s * n + j];
+    auto add = [&](const double4 &p) {
         a.x += p.x;
         a.y += p.y;
         a.z += p.z;
         a.w += p.w;
-    }
+    };
+    if (j < n)
+        for (int s = q; s < nparts; s += kXfQ) add(part[(long)s * n + j]);
+    if (q > 0) sh[q - 1][li] = a;
+    __syncthreads();
+    if (q != 0 || j >= n) return;
+    for (int g = 0; g < kXfQ - 1; g++) add(sh[g][li]);
     out[j] = a;
 }
 
+// Points per thread: two from 2,048 points, four from 16,384, where the source
+// splits still give several workgroups per CU.  Up to kX2eNoAllocMaxPoints the
+// splits are those of one point per thread, which bounds the partial sums of the
+// no-allocation entry.
+constexpr int kX2eNoAllocMaxPoints = 8192;
+static int x2e_points(int n) { return n >= 16384 ? 4 : (n >= 2048 ? 2 : 1); }
+static int x2e_point_blocks(int n) { return (n + kBlock * x2e_points(n) - 1) / (kBlock * x2e_points(n)); }
+
 int x2e_splits(int n, int nsrc) {
-    const int pb = (n + kBlock - 1) / kBlock;
-    const int max_s = std::max(1, (nsrc + kBlock - 1) / kBlock);
-    const int want = (2048 + pb - 1) / pb;
-    return std::max(1, std::min(want, max_s));
+    const int pb = x2e_point_blocks(n), pf = n > kX2eNoAllocMaxPoints ? pb : (n + kBlock - 1) / kBlock;
+    const int thin = std::min((nsrc + 15) / 16, (512 + pb - 1) / pb);  // two workgroups per CU
+    const int full = std::min((nsrc + kBlock - 1) / kBlock, (2048 + pf - 1) / pf);
+    return std::max(1, std::max(thin, full));
+}
+
+// f with the compile-time choice of potential, field or both and of the points per thread.
+template <typename F>
+static void x2e_dispatch(int n, bool v, bool e, F &&f) {
+    auto points = [&](auto wv, auto we) {
+        const int p = x2e_points(n);
+        if (p == 4) f(wv, we, std::integral_constant<int, 4>{});
+        else if (p == 2) f(wv, we, std::integral_constant<int, 2>{});
+        else f(wv, we, std::integral_constant<int, 1>{});
+    };
+    if (v && e) points(std::true_type{}, std::true_type{});
+    else if (v) points(std::true_type{}, std::false_type{});
+    else points(std::false_type{}, std::true_type{});
+    HIP_CHECK(hipGetLastError());
 }
 
 void launch_x2e(hipStream_t st, int n, const double *cext, bool mm, bool pol, bool amoeba, int ld, int nmm,
-                const double4 *ms, const double *mq, int npol, const double4 *ps, const double *ipd, double4 *part,
-                int smm, int spol, double4 *out, int *bad) {
+                const double4 *ms, const double *mq, int npol, const double4 *ps, const double *ipd, bool want_v,
+                bool want_e, double4 *part, int smm, int spol, double4 *out, int *bad) {
     if (n == 0) return;
-    const int pb = (n + kBlock - 1) / kBlock;
+    const int pb = x2e_point_blocks(n);
     int off = 0;
     if (mm && nmm > 0) {
         const int chunk = (nmm + smm - 1) / smm;
-        if (ld == 10)
-            hipLaunchKernelGGL(k_m2e<10>, dim3(pb, smm), dim3(kBlock), 0, st, n, cext, nmm, chunk, ms, mq, part,
-                               bad);
-        else
-            hipLaunchKernelGGL(k_m2e<1>, dim3(pb, smm), dim3(kBlock), 0, st, n, cext, nmm, chunk, ms, mq, part,
-                               bad);
-        HIP_CHECK(hipGetLastError());
+        x2e_dispatch(n, want_v, want_e, [&](auto v, auto e, auto p) {
+            constexpr bool V = decltype(v)::value, E = decltype(e)::value;
+            constexpr int P = decltype(p)::value;
+            if (ld == 10)
+                hipLaunchKernelGGL((k_m2e<10, V, E, P>), dim3(pb, smm), dim3(kBlock), 0, st, n, cext, nmm, chunk, ms,
+                                   mq, part, bad);
+            else
+                hipLaunchKernelGGL((k_m2e<1, V, E, P>), dim3(pb, smm), dim3(kBlock), 0, st, n, cext, nmm, chunk, ms,
+                                   mq, part, bad);
+        });
         off = smm;
     }
     if (pol && npol > 0) {
         const int chunk = (npol + spol - 1) / spol;
-        hipLaunchKernelGGL(k_d2e, dim3(pb, spol), dim3(kBlock), 0, st, n, cext, npol, chunk, ps, ipd,
-                           amoeba ? 1 : 0, part + (long)off * n, bad);
-        HIP_CHECK(hipGetLastError());
+        x2e_dispatch(n, want_v, want_e, [&](auto v, auto e, auto p) {
+            constexpr bool V = decltype(v)::value, E = decltype(e)::value;
+            constexpr int P = decltype(p)::value;
+            hipLaunchKernelGGL((k_d2e<V, E, P>), dim3(pb, spol), dim3(kBlock), 0, st, n, cext, npol, chunk, ps, ipd,
+                               amoeba ? 1 : 0, part + (long)off * n, bad);
+        });
         off += spol;
     }
-    hipLaunchKernelGGL(k_x2e_finalize, dim3(pb), dim3(kBlock), 0, st, n, off, part, out);
+    hipLaunchKernelGGL(k_x2e_finalize, dim3((n + kXfPts - 1) / kXfPts), dim3(kBlock), 0, st, n, off, part, out);
     HIP_CHECK(hipGetLastError());
 }
 
@@ -196,11 +302,11 @@ void launch_x2e(hipStream_t st, int n, const double *cext, bool mm, bool pol, bo
 // points and the caller's field (copied in), the per-split partial sums, the
 // summed result and the coincident-point flag.  Split counts are those of the
 // allocating entry (x2e_splits), so both give the same bits.  For n points
-// each source kind takes at most ceil(2048 / ceil(n / 256)) splits, so the
+// each source kind takes at most ceil(2048 / ceil(n / 256)) splits, or
+// ceil(512 / ceil(n / 512)) or ceil(512 / ceil(n / 256)), which is fewer, so the
 // partial sums need at most 2 (2048 + ceil(n / 256) - 1) 256 double4.
 // Every call on a GPU uses that GPU's array: calls that overlap on one GPU
 // (other host threads, other streams) race; each call waits for its own work.
-constexpr int kX2eNoAllocMaxPoints = 8192;
 constexpr long kX2eNoAllocMaxParts = 2L * (2048 + (kX2eNoAllocMaxPoints + kBlock - 1) / kBlock - 1) * kBlock;
 constexpr size_t kScrPart = 0;
 constexpr size_t kScrOut = kScrPart + sizeof(double4) * kX2eNoAllocMaxParts;
@@ -277,7 +383,7 @@ int x2e_field_noalloc(hipStream_t st, int device, int n, const double *cext, boo
     HIP_CHECK(hipMemcpyAsync(es, e, sizeof(double) * 3L * n, hipMemcpyHostToDevice, st));
     hipLaunchKernelGGL(k_zero_flag, dim3(1), dim3(64), 0, st, bad);
     HIP_CHECK(hipGetLastError());
-    launch_x2e(st, n, c, mm, pol, amoeba, ld, nmm, ms, mq, npol, ps, ipd, part, smm, spol, out, bad);
+    launch_x2e(st, n, c, mm, pol, amoeba, ld, nmm, ms, mq, npol, ps, ipd, false, true, part, smm, spol, out, bad);
     hipLaunchKernelGGL(k_add_x2e_field, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, n, out, es);
     HIP_CHECK(hipGetLastError());
     int bad_h = 0;

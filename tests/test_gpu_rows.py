@@ -62,3 +62,41 @@ def test_per_target_matvec(n, amoeba):
             assert np.abs(y - want[:ncols]).max() <= tol * np.abs(want).max(), (kind, ncols)
         assert np.array_equal(s.tmatvec(x, kind=kind)[0], y)
     s.terminate()
+
+
+@pytest.mark.parametrize("amoeba", [True, False])
+@pytest.mark.parametrize("n", [1, 15, 17, 260, 1030])
+def test_thin_source_splits(n, amoeba):
+    """The static field and the gradient with sources split down to 16 per
+    workgroup (one site, one split short or past full, several target blocks)
+    against the oracle; bars as the larger systems' (1e-12 and 1e-11 of the
+    largest component: sums of at most 1,030 pairs)."""
+    s, o = pair(chain(n, amoeba))
+    e, eo = s.e_m2d, o.m2d()
+    assert np.abs(e - eo).max() <= 1e-12 * max(np.abs(eo).max(), 1e-300)
+    s.set_external_field(np.random.default_rng(n).normal(0.0, 1e-2, size=(n, 3)))
+    g = s.polelec_geomgrad()
+    want = o.polelec_geomgrad(np.array(s.ipd))
+    assert np.abs(g - want).max() <= 1e-11 * max(np.abs(want).max(), 1e-300)
+    s.terminate()
+
+
+@pytest.mark.parametrize("amoeba", [True, False])
+@pytest.mark.parametrize("npoints", [1, 2047, 2049, 8193, 16383, 16385])
+def test_external_points(npoints, amoeba):
+    """Potential and field at external points around the sizes where the points
+    per thread and the source splits change, against the oracle (1e-12 of the
+    largest value: 300 sources)."""
+    n = 300
+    s, o = pair(chain(n, amoeba))
+    s.set_external_field(np.zeros((n, 3)))
+    ipd = np.array(s.ipd)
+    rng = np.random.default_rng(npoints)
+    c = rng.uniform(-30.0, -2.5, size=(npoints, 3))
+    for name, which in (("mm", 1), ("pol", 2), ("mmpol", 3)):
+        v, e = o.x2e(c, which, ipd)
+        got = getattr(s, f"potential_{name}2ext")(c)
+        assert np.abs(got - v).max() <= 1e-12 * np.abs(v).max(), name
+        got = getattr(s, f"field_{name}2ext")(c)
+        assert np.abs(got - e).max() <= 1e-12 * np.abs(e).max(), name
+    s.terminate()
