@@ -261,6 +261,16 @@ void launch_jacobi(hipStream_t st, long n, const double *rhs, const double *ox, 
 void launch_multi_dot(hipStream_t st, long n, int k, const double *const *vecs, const double *e,
                       double *red, double *out);
 void launch_lincomb(hipStream_t st, long n, int k, const double *const *vecs, const double *coef,
+// The same pieces for columns small enough for one workgroup each (kernels.hip):
+// the guess's zero-norm rule; start of the solve (h = T x unless zero_guess); one
+// iteration's update, convergence test and new direction.  z is not stored.
+bool cg_small(long n);
+void launch_cg_guess_small(hipStream_t st, long n, int M, double *x, const double *alpha);
+void launch_cg_init_small(hipStream_t st, long n, int M, const double *b, const double *h, double *x, double *r,
+                          double *p, const double *alpha, CgState *cs, bool zero_guess, const double *tol, double eps);
+void launch_cg_step(hipStream_t st, long n, int M, int it, const double *h, double *x, double *r, double *p,
+                    const double *alpha, const double *red_hp, int nred_hp, CgState *cs);
+
                     double *out);
 void launch_maxabs_diff(hipStream_t st, long n, const double *a, const double *b, double *red,
                         double *out);

@@ -722,6 +722,7 @@ struct CgResult {
     double beta[2] = {0, 0};
 };
 
+    const bool small = !nb && cg_small(n);
 // With nb (inner solves of the mixed solver, zero guess only) the iterations
 // use the near-field preconditioner, r alternating between vr and vr3.
 CgResult cg_solve(System &s, DeviceState &d, int kind, int M, const double *b, double *x, const double *tol,
@@ -729,14 +730,17 @@ CgResult cg_solve(System &s, DeviceState &d, int kind, int M, const double *b, d
     const long n = d.n;
     CgResult res;
     double te[4] = {tol[0], M > 1 ? tol[1] : tol[0], small_step_eps, small_step_eps};
-    HCHECK(hipMemcpyAsync(d.tol_dev, te, sizeof(te), hipMemcpyHostToDevice, d.stream));
+    if (!small) HCHECK(hipMemcpyAsync(d.tol_dev, te, sizeof(te), hipMemcpyHostToDevice, d.stream));
     if (nb && !zero_guess) fatal("Internal error: the near-field preconditioned solve starts from zero");
     if (!zero_guess) {
-        launch_norm2_guess(d.stream, n, M, x, d.alpha, d.red_a);
+        if (small) launch_cg_guess_small(d.stream, n, M, x, d.alpha);
+        else launch_norm2_guess(d.stream, n, M, x, d.alpha, d.red_a);
         matvec(s, d, kind, M, x, d.vh, true, nullptr, nullptr);
     }
     double *rb[2] = {d.vr, nb ? d.vr3 : d.vr};
-    if (nb)
+    if (small)
+        launch_cg_init_small(d.stream, n, M, b, d.vh, x, d.vr, d.vp, d.alpha, d.cs, zero_guess, te, small_step_eps);
+    else if (nb)
         launch_cg_init_nb(d.stream, s.npol, M, b, x, rb[0], d.vz, d.vp, d.alpha, d.nb, d.red_a, d.cs, d.tol_dev,
                           nullptr);
     else
@@ -749,6 +753,8 @@ CgResult cg_solve(System &s, DeviceState &d, int kind, int M, const double *b, d
     bool all_done = false;
     while (it <= maxit && !all_done) {
         const int end = std::min(maxit, it + chunk - 1);
+            } else if (small) {
+                launch_cg_step(d.stream, n, M, it, d.vh, x, d.vr, d.vp, d.alpha, d.red_b, nred_hp, d.cs);
         for (; it <= end; it++) {
             matvec(s, d, kind, M, d.vp, d.vh, true, d.red_b, d.cs);
             if (nb) {
@@ -1176,7 +1182,9 @@ void polarization(System &s, const double *d_field, int solver, int matv, int ma
             CgState *cs_save = d.cs;
             d.cs = cs_save + k;
             double tol = s.tol;
-            CgResult r = cg_solve(s, d, kind, 1, d.vb + k * n, d.vx + k * n, &tol, s.max_iter, false, kEpsRp,
+            // the guess is 0 for the first set solved from nothing: T 0 = 0 needs no matvec
+            const bool zero = !s.ipd_use_guess && (k == 0 || !mD);
+            CgResult r = cg_solve(s, d, kind, 1, d.vb + k * n, d.vx + k * n, &tol, s.max_iter, zero, kEpsRp,
                                   s.ipd_use_guess ? -1 : k);
             d.cs = cs_save;
             s.last_iters[k] = r.iters[0];

@@ -961,6 +961,166 @@ void launch_cg_direction(hipStream_t st, long n, int M, int it, const double *z,
     HIP_CHECK(hipGetLastError());
 }
 
+// ------------------------------------------------ small systems: one workgroup
+// Up to kCgSmall elements a column's vectors fit one 1,024-thread workgroup, kept
+// in registers across the two reductions of an iteration: the start of a solve
+// is two launches instead of five and an iteration's vector work one instead of
+// two (a launch costs ~4.5 us whatever it does; 648 sites: 4.6 + 4.5 -> 4.9 us per
+// iteration; at 6,003 elements one workgroup takes 8.5 us, as long as the two launches).
+constexpr int kCgThreads = 1024;
+constexpr long kCgSmall = 4 * kCgThreads;
+
+// Sum over the workgroup, valid in every thread (fixed order).
+__device__ __forceinline__ double cg_sum(double v, double *sh) {
+    v = wave_sum(v);
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    __syncthreads();
+    if (lane == 0) sh[w] = v;
+    __syncthreads();
+    double t = sh[0];
+#pragma unroll
+    for (int q = 1; q < kCgThreads / 64; q++) t += sh[q];
+    return t;
+}
+
+// Guess of column blockIdx.x: k_norm2 + k_guess_fix.
+__global__ __launch_bounds__(kCgThreads) void k_cg_guess_small(int n, double *__restrict__ x,
+                                                               const double *__restrict__ alpha) {
+    __shared__ double sh[kCgThreads / 64];
+    x += (long)blockIdx.x * n;
+    double v = 0.0;
+    for (int k = threadIdx.x; k < n; k += kCgThreads) v += x[k] * x[k];
+    v = cg_sum(v, sh);
+    if (v < kEpsRpDev)
+        for (int k = threadIdx.x; k < n; k += kCgThreads) x[k] *= alpha[k / 3];
+}
+
+// k_cg_init + k_cg_init2 of column blockIdx.x.
+__global__ __launch_bounds__(kCgThreads) void k_cg_init_small(int n, const double *__restrict__ b,
+                                                              const double *__restrict__ h, double *__restrict__ x,
+                                                              double *__restrict__ r, double *__restrict__ p,
+                                                              const double *__restrict__ alpha, int zero_guess,
+                                                              double tol0, double tol1, double eps, CgState *cs) {
+    __shared__ double sh[kCgThreads / 64];
+    const int m = blockIdx.x;
+    const long o = (long)m * n;
+    double v = 0.0;
+    for (int k = threadIdx.x; k < n; k += kCgThreads) {
+        double rr = b[o + k];
+        if (zero_guess) x[o + k] = 0.0;
+        else rr -= h[o + k];
+        const double zz = alpha[k / 3] * rr;
+        r[o + k] = rr;
+        p[o + k] = zz;
+        v += rr * zz;
+    }
+    v = cg_sum(v, sh);
+    if (threadIdx.x == 0) {
+        cs[m].g[0] = cs[m].g[1] = v;
+        cs[m].rms = 0.0;
+        cs[m].last_beta = 0.0;
+        cs[m].tol = m == 0 ? tol0 : tol1;
+        cs[m].eps = eps;
+        cs[m].done = 0;
+        cs[m].status = 2;
+        cs[m].iters = 0;
+    }
+}
+
+// k_cg_update + k_cg_direction of column blockIdx.x, E elements per thread.
+template <int E>
+__global__ __launch_bounds__(kCgThreads) void k_cg_step(int n, int it, const double *__restrict__ h,
+                                                        double *__restrict__ x, double *__restrict__ r,
+                                                        double *__restrict__ p, const double *__restrict__ alpha,
+                                                        const double *__restrict__ red_hp, int nred, CgState *cs) {
+    __shared__ double sh[kCgThreads / 64];
+    __shared__ CgState s_cs;
+    const int m = blockIdx.x, tid = threadIdx.x;
+    if (tid == 0) s_cs = cs[m];
+    const long o = (long)m * n;
+    double hv[E], xv[E], rv[E], pv[E], al[E];
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        const int k = tid + e * kCgThreads;
+        const bool ok = k < n;
+        hv[e] = ok ? h[o + k] : 0.0;
+        xv[e] = ok ? x[o + k] : 0.0;
+        rv[e] = ok ? r[o + k] : 0.0;
+        pv[e] = ok ? p[o + k] : 0.0;
+        al[e] = ok ? alpha[k / 3] : 0.0;
+    }
+    double v = 0.0;
+    for (int i = tid; i < nred; i += kCgThreads) v += red_hp[(long)m * nred + i];
+    const double gama = cg_sum(v, sh);
+    if (s_cs.done) return;  // uniform: read before the barriers of the sum
+    if (fabs(gama) < s_cs.eps || gama == 0.0) {
+        if (tid == 0) {
+            cs[m].status = 1;
+            cs[m].iters = it;
+            cs[m].done = 1;
+        }
+        return;
+    }
+    const double gold = s_cs.g[(it + 1) & 1], a = gold / gama;
+    v = 0.0;
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        xv[e] += a * pv[e];
+        rv[e] -= a * hv[e];
+        v += rv[e] * (al[e] * rv[e]);
+    }
+    const double gnew = cg_sum(v, sh);
+    const double rms = sqrt(gnew / (double)n);
+    const bool conv = rms < s_cs.tol;
+    const double beta = gnew / gold;
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        const int k = tid + e * kCgThreads;
+        if (k < n) {
+            x[o + k] = xv[e];
+            r[o + k] = rv[e];
+            if (!conv) p[o + k] = beta * pv[e] + al[e] * rv[e];
+        }
+    }
+    if (tid == 0) {
+        cs[m].rms = rms;
+        cs[m].iters = it;
+        if (conv) {
+            cs[m].status = 0;
+            cs[m].done = 1;
+        } else {
+            cs[m].g[it & 1] = gnew;
+            cs[m].last_beta = beta;
+        }
+    }
+}
+
+bool cg_small(long n) { return n <= kCgSmall; }
+
+void launch_cg_guess_small(hipStream_t st, long n, int M, double *x, const double *alpha) {
+    hipLaunchKernelGGL(k_cg_guess_small, dim3(M), dim3(kCgThreads), 0, st, (int)n, x, alpha);
+    HIP_CHECK(hipGetLastError());
+}
+
+void launch_cg_init_small(hipStream_t st, long n, int M, const double *b, const double *h, double *x, double *r,
+                          double *p, const double *alpha, CgState *cs, bool zero_guess, const double *tol, double eps) {
+    hipLaunchKernelGGL(k_cg_init_small, dim3(M), dim3(kCgThreads), 0, st, (int)n, b, h, x, r, p, alpha,
+                       (int)zero_guess, tol[0], M > 1 ? tol[1] : tol[0], eps, cs);
+    HIP_CHECK(hipGetLastError());
+}
+
+void launch_cg_step(hipStream_t st, long n, int M, int it, const double *h, double *x, double *r, double *p,
+                    const double *alpha, const double *red_hp, int nred_hp, CgState *cs) {
+    const dim3 g(M), b(kCgThreads);
+    if (n <= kCgThreads)
+        hipLaunchKernelGGL(k_cg_step<1>, g, b, 0, st, (int)n, it, h, x, r, p, alpha, red_hp, nred_hp, cs);
+    else if (n <= 2 * kCgThreads)
+        hipLaunchKernelGGL(k_cg_step<2>, g, b, 0, st, (int)n, it, h, x, r, p, alpha, red_hp, nred_hp, cs);
+    else
+        hipLaunchKernelGGL(k_cg_step<4>, g, b, 0, st, (int)n, it, h, x, r, p, alpha, red_hp, nred_hp, cs);
+    HIP_CHECK(hipGetLastError());
+}
+
 // ========================================================= element-wise
 __global__ void k_add_field(long n, int nsets, const double *__restrict__ e_m2d, const double *__restrict__ ext,
                             double *__restrict__ ef) {
