@@ -215,6 +215,29 @@ struct NbDev {
     bool list_valid = false;  // lists of the current coordinates uploaded
     bool valid = false;       // B computed
 };
+// Uniform grid over the MM atoms (geom.hip): cells at least kNbCut wide, atoms by
+// cell in order[start[cell] ..); flags[0] = 1 where a polarizable site coincides
+// with another atom, flags[1] = entries of the neighbour lists.
+struct GridGeom {
+    double lo[3] = {0.0, 0.0, 0.0}, inv_h = 0.0;
+    int dim[3] = {1, 1, 1};
+};
+struct GridDev {
+    GridGeom geom;
+    int *count = nullptr, *start = nullptr, *cell = nullptr, *rank = nullptr, *order = nullptr, *rows = nullptr;
+    int *flags = nullptr;
+    long cell_cap = 0;
+    bool valid = false;  // of the current coordinates
+    long nnz = 0;
+};
+// ms, ps and ps32 from the coordinates c[nmm][3] and w[nmm] = 1/thole.
+void launch_geom_sites(hipStream_t st, int nmm, const double *c, const double *w, const int *mm_polar, double4 *ms,
+                       double4 *ps, float4 *ps32);
+// The grid, flags and row_ptr[npol + 1] of the neighbour lists; then ci and rowi.
+void launch_grid(hipStream_t st, int nmm, int npol, const GridDev &g, const int *polar_mm, const int *mm_polar,
+                 const double4 *ms, int *row_ptr);
+void launch_nb_lists(hipStream_t st, int npol, const GridDev &g, const int *polar_mm, const int *mm_polar,
+                     const double4 *ms, const int *row_ptr, int *ci, int *rowi);
 int nb_blocks(int npol);  // per-column partial sums of the preconditioned CG kernels
 void launch_nb_tensors(hipStream_t st, bool amoeba, const NbDev &nb, const float4 *ps32, const float *pa32,
                        const double *alpha, const CsrDev &pp);
@@ -237,6 +260,16 @@ void launch_cg_update(hipStream_t st, long n, int M, int it, const double *h, do
                       int nred_hp, double *red_rz, CgState *cs);
 void launch_cg_direction(hipStream_t st, long n, int M, int it, const double *z, double *p,
                          const double *red_rz, CgState *cs, int *all_done);
+
+// The same pieces for columns small enough for one workgroup each (kernels.hip):
+// the guess's zero-norm rule; start of the solve (h = T x unless zero_guess); one
+// iteration's update, convergence test and new direction.  z is not stored.
+bool cg_small(long n);
+void launch_cg_guess_small(hipStream_t st, long n, int M, double *x, const double *alpha);
+void launch_cg_init_small(hipStream_t st, long n, int M, const double *b, const double *h, double *x, double *r,
+                          double *p, const double *alpha, CgState *cs, bool zero_guess, const double *tol, double eps);
+void launch_cg_step(hipStream_t st, long n, int M, int it, const double *h, double *x, double *r, double *p,
+                    const double *alpha, const double *red_hp, int nred_hp, CgState *cs);
 
 // Interaction energy of the static multipoles (energy_MM_MM), FP64: part holds
 // nsplit * nmm doubles, red site_blocks(nmm); ss = S-S list by target with
@@ -261,16 +294,6 @@ void launch_jacobi(hipStream_t st, long n, const double *rhs, const double *ox, 
 void launch_multi_dot(hipStream_t st, long n, int k, const double *const *vecs, const double *e,
                       double *red, double *out);
 void launch_lincomb(hipStream_t st, long n, int k, const double *const *vecs, const double *coef,
-// The same pieces for columns small enough for one workgroup each (kernels.hip):
-// the guess's zero-norm rule; start of the solve (h = T x unless zero_guess); one
-// iteration's update, convergence test and new direction.  z is not stored.
-bool cg_small(long n);
-void launch_cg_guess_small(hipStream_t st, long n, int M, double *x, const double *alpha);
-void launch_cg_init_small(hipStream_t st, long n, int M, const double *b, const double *h, double *x, double *r,
-                          double *p, const double *alpha, CgState *cs, bool zero_guess, const double *tol, double eps);
-void launch_cg_step(hipStream_t st, long n, int M, int it, const double *h, double *x, double *r, double *p,
-                    const double *alpha, const double *red_hp, int nred_hp, CgState *cs);
-
                     double *out);
 void launch_maxabs_diff(hipStream_t st, long n, const double *a, const double *b, double *red,
                         double *out);

@@ -47,7 +47,9 @@ struct DeviceState {
     float *pa32 = nullptr;
     int *polar_mm = nullptr;
     double4 *ms64 = nullptr;
-    double *ma64 = nullptr, *mq = nullptr;
+    double *ma64 = nullptr, *mq = nullptr, *cmm = nullptr, *mw = nullptr;  // mw: 1 / thole
+    int *mm_polar = nullptr;
+    GridDev grid;
     CsrDev sp, pp, pd;
     CsrDev ss;  // S-S pairs by target, f = 1 - s (fixed-multipole energy)
     // fields, dipoles, work vectors ([2][n] each)
@@ -114,7 +116,6 @@ struct DeviceState {
     // geometric gradient (built on first use): MM-target correction list, frames,
     // per-atom rotation index, partial sums and results
     CsrDev mp;
-    int *mm_polar = nullptr;
     double *q0 = nullptr;
     int4 *frames = nullptr;
     int *rev_ri = nullptr, *rev_ci = nullptr;
@@ -194,6 +195,10 @@ int prof_begin(DeviceState &d, int cls) {
     HCHECK(hipEventRecord(d.prof_pool[2 * i], d.stream));
     return i;
 }
+
+const char *const kCoincident =
+    "Requesting Coulomb kernel for two atoms placed in the same point, this could be an internal bug "
+    "or a problem in your input file, please check.";
 
 void upload(const void *h, void *d, size_t bytes) {
     if (bytes) HCHECK(hipMemcpy(d, h, bytes, hipMemcpyHostToDevice));
@@ -310,39 +315,97 @@ void upload_lists(System &s, DeviceState &d) {
     upload_csr(d, npol, rows, d.pd, false);
 }
 
+// Grid over the current coordinates: counts of the neighbour lists and the
+// coincident-site check, one small readback.
+void ensure_grid(System &s, DeviceState &d) {
+    GridDev &g = d.grid;
+    if (g.valid) return;
+    double lo[3], hi[3];
+    for (int c = 0; c < 3; c++) lo[c] = hi[c] = s.cmm[c];
+    for (int i = 0; i < s.nmm; i++)
+        for (int c = 0; c < 3; c++) {
+            lo[c] = std::min(lo[c], s.cmm[3 * i + c]);
+            hi[c] = std::max(hi[c], s.cmm[3 * i + c]);
+        }
+    // cells a rounding wider than kNbCut, at most ~8 per atom; one cell when the
+    // extent is not finite
+    double h = kNbCut * (1.0 + 1e-9), dim[3] = {1.0, 1.0, 1.0};
+    bool finite = true;
+    for (int c = 0; c < 3; c++) finite = finite && std::isfinite(hi[c] - lo[c]);
+    for (; finite; h *= 1.5) {
+        for (int c = 0; c < 3; c++) dim[c] = std::floor((hi[c] - lo[c]) / h) + 1.0;
+        if (dim[0] * dim[1] * dim[2] <= 8.0 * s.nmm + 64.0) break;
+    }
+    for (int c = 0; c < 3; c++) {
+        g.geom.lo[c] = lo[c];
+        g.geom.dim[c] = (int)dim[c];
+    }
+    g.geom.inv_h = 1.0 / h;
+    const long ncell = (long)g.geom.dim[0] * g.geom.dim[1] * g.geom.dim[2];
+    if (!g.cell) {
+        g.cell = dalloc<int>(d, s.nmm);
+        g.rank = dalloc<int>(d, s.nmm);
+        g.order = dalloc<int>(d, s.nmm);
+        g.rows = dalloc<int>(d, s.npol);
+        g.flags = dalloc<int>(d, 2);
+        d.nb.row_ptr = dalloc<int>(d, s.npol + 1);
+    }
+    if (ncell > g.cell_cap) {
+        dfree(d, g.count);
+        dfree(d, g.start);
+        g.cell_cap = ncell + ncell / 4;
+        g.count = dalloc<int>(d, g.cell_cap);
+        g.start = dalloc<int>(d, g.cell_cap + 1);
+    }
+    launch_grid(d.stream, s.nmm, s.npol, g, d.polar_mm, d.mm_polar, d.ms64, d.nb.row_ptr);
+    int *flags = reinterpret_cast<int *>(d.scal_host + 60);
+    HCHECK(hipMemcpyAsync(flags, g.flags, 2 * sizeof(int), hipMemcpyDeviceToHost, d.stream));
+    HCHECK(hipStreamSynchronize(d.stream));
+    if (flags[0]) fatal(kCoincident);
+    g.nnz = flags[1];
+    g.valid = true;
+}
+
+// Up to this many atoms the coincident-site check is cheaper on the host (all
+// pairs: 10 us at 99 atoms) than as the grid's launches and readback.
+constexpr int kHostCheckAtoms = 160;
+
 void upload_geometry(System &s, DeviceState &d) {
-    check_coincident_sites(s);  // once per geometry, not per solve
+    HCHECK(hipMemcpyAsync(d.cmm, s.cmm.data(), sizeof(double) * 3 * s.nmm, hipMemcpyHostToDevice, d.stream));
+    HCHECK(hipMemcpyAsync(d.mq, s.q.data(), sizeof(double) * s.ld_cart * s.nmm, hipMemcpyHostToDevice, d.stream));
+    launch_geom_sites(d.stream, s.nmm, d.cmm, d.mw, d.mm_polar, d.ms64, d.ps64, d.ps32);
+    d.tpack_valid = false;
+    d.lu_valid = false;
+    d.grid.valid = false;
+    d.nb.list_valid = false;
+    d.nb.valid = false;
+    // once per geometry, not per solve
+    if (s.npol > 0 && s.nmm > kHostCheckAtoms) ensure_grid(s, d);
+    else if (coincident_sites(s)) fatal(kCoincident);
+    s.dev_geometry_dirty = false;
+}
+
+// What does not change with the coordinates.
+void upload_sites(System &s, DeviceState &d) {
     const double inf = std::numeric_limits<double>::infinity();
-    std::vector<double4> ps(s.npol), ms(s.nmm);
-    std::vector<float4> ps32(s.npol);
-    std::vector<double> pa(s.npol), ma(s.nmm);
+    std::vector<double> w(s.nmm), ma(s.nmm), pa(s.npol);
     std::vector<float> pa32(s.npol);
     for (int i = 0; i < s.nmm; i++) {
         const double t = s.thole[i];
-        ms[i] = make_double4(s.cmm[3 * i], s.cmm[3 * i + 1], s.cmm[3 * i + 2], t > kEpsRp ? 1.0 / t : inf);
+        w[i] = t > kEpsRp ? 1.0 / t : inf;
         ma[i] = s.mm_polar[i] >= 0 ? s.thole_damping_mm[i] : inf;
     }
     for (int p = 0; p < s.npol; p++) {
-        const int i = s.polar_mm[p];
-        ps[p] = ms[i];
-        pa[p] = s.thole_damping_mm[i];
-        ps32[p] = make_float4((float)ps[p].x, (float)ps[p].y, (float)ps[p].z, (float)ps[p].w);
+        pa[p] = s.thole_damping_mm[s.polar_mm[p]];
         pa32[p] = (float)pa[p];
     }
-    upload(ps.data(), d.ps64, sizeof(double4) * s.npol);
-    upload(ps32.data(), d.ps32, sizeof(float4) * s.npol);
+    upload(w.data(), d.mw, sizeof(double) * s.nmm);
+    upload(ma.data(), d.ma64, sizeof(double) * s.nmm);
     upload(pa.data(), d.pa64, sizeof(double) * s.npol);
     upload(pa32.data(), d.pa32, sizeof(float) * s.npol);
     upload(s.pol.data(), d.alpha, sizeof(double) * s.npol);
     upload(s.polar_mm.data(), d.polar_mm, sizeof(int) * s.npol);
-    upload(ms.data(), d.ms64, sizeof(double4) * s.nmm);
-    upload(ma.data(), d.ma64, sizeof(double) * s.nmm);
-    upload(s.q.data(), d.mq, sizeof(double) * s.ld_cart * s.nmm);
-    d.tpack_valid = false;
-    d.lu_valid = false;
-    d.nb.list_valid = false;
-    d.nb.valid = false;
-    s.dev_geometry_dirty = false;
+    upload(s.mm_polar.data(), d.mm_polar, sizeof(int) * s.nmm);
 }
 
 DeviceState &ensure_device(System &s) {
@@ -378,6 +441,9 @@ DeviceState &ensure_device(System &s) {
         d.ms64 = dalloc<double4>(d, s.nmm);
         d.ma64 = dalloc<double>(d, s.nmm);
         d.mq = dalloc<double>(d, (size_t)s.ld_cart * s.nmm);
+        d.cmm = dalloc<double>(d, 3 * (size_t)s.nmm);
+        d.mw = dalloc<double>(d, s.nmm);
+        d.mm_polar = dalloc<int>(d, s.nmm);
         d.e_m2d = dalloc<double>(d, 2 * n);
         d.ipd = dalloc<double>(d, 2 * n);
         d.ext = dalloc<double>(d, n);
@@ -418,6 +484,7 @@ DeviceState &ensure_device(System &s) {
         HCHECK(hipMemset(d.ipd, 0, sizeof(double) * 2 * n));
         HCHECK(hipMemset(d.e_m2d, 0, sizeof(double) * 2 * n));
         s.dev = dp;
+        upload_sites(s, d);
         upload_lists(s, d);
         s.dev_geometry_dirty = true;
     }
@@ -603,106 +670,33 @@ void matvec(System &s, DeviceState &d, int kind, int M, const double *x, double 
     }
 }
 
-// Neighbour lists of the near-field preconditioner: for every polarizable site
-// the sites closer than kNbCut, in site order.  A function of the coordinates
-// alone, built on the host with a grid of cells at least kNbCut wide (only the
-// 27 cells around a site can hold its neighbours) when the coordinates reach
-// the device; distances in FP64, the same for (i, j) and (j, i), so the lists
-// are symmetric.
-void build_nb_lists(const System &s, std::vector<int> &row_ptr, std::vector<int> &ci) {
-    const int n = s.npol;
-    row_ptr.assign(n + 1, 0);
-    ci.clear();
-    if (n == 0) return;
-    double lo[3], hi[3];
-    for (int c = 0; c < 3; c++) lo[c] = hi[c] = s.cpol[c];
-    for (int i = 0; i < n; i++)
-        for (int c = 0; c < 3; c++) {
-            lo[c] = std::min(lo[c], s.cpol[3 * i + c]);
-            hi[c] = std::max(hi[c], s.cpol[3 * i + c]);
-        }
-    // cells at least kNbCut wide, at most ~8 per site
-    double h = kNbCut;
-    long dim[3];
-    for (;;) {
-        for (int c = 0; c < 3; c++) dim[c] = (long)std::floor((hi[c] - lo[c]) / h) + 1;
-        if (dim[0] * dim[1] * dim[2] <= 8L * n + 64) break;
-        h *= 1.5;
-    }
-    auto cell_of = [&](int i, long *g) {
-        for (int c = 0; c < 3; c++)
-            g[c] = std::min(dim[c] - 1, (long)std::floor((s.cpol[3 * i + c] - lo[c]) / h));
-    };
-    const long ncell = dim[0] * dim[1] * dim[2];
-    std::vector<int> start(ncell + 1, 0), order(n), cell(n);
-    for (int i = 0; i < n; i++) {
-        long g[3];
-        cell_of(i, g);
-        cell[i] = (int)((g[2] * dim[1] + g[1]) * dim[0] + g[0]);
-        start[cell[i] + 1]++;
-    }
-    for (long k = 0; k < ncell; k++) start[k + 1] += start[k];
-    {
-        std::vector<int> fill(start.begin(), start.end() - 1);
-        for (int i = 0; i < n; i++) order[fill[cell[i]]++] = i;
-    }
-    const double rc2 = kNbCut * kNbCut;
-    std::vector<int> row;
-    ci.reserve((size_t)n * 12);
-    for (int i = 0; i < n; i++) {
-        long g[3];
-        cell_of(i, g);
-        row.clear();
-        for (long z = std::max(0L, g[2] - 1); z <= std::min(dim[2] - 1, g[2] + 1); z++)
-            for (long y = std::max(0L, g[1] - 1); y <= std::min(dim[1] - 1, g[1] + 1); y++)
-                for (long x = std::max(0L, g[0] - 1); x <= std::min(dim[0] - 1, g[0] + 1); x++) {
-                    const long k = (z * dim[1] + y) * dim[0] + x;
-                    for (int q = start[k]; q < start[k + 1]; q++) {
-                        const int j = order[q];
-                        if (j == i) continue;
-                        const double dx = s.cpol[3 * i] - s.cpol[3 * j], dy = s.cpol[3 * i + 1] - s.cpol[3 * j + 1],
-                                     dz = s.cpol[3 * i + 2] - s.cpol[3 * j + 2];
-                        if (dx * dx + dy * dy + dz * dz < rc2) row.push_back(j);
-                    }
-                }
-        std::sort(row.begin(), row.end());
-        ci.insert(ci.end(), row.begin(), row.end());
-        row_ptr[i + 1] = (int)ci.size();
-    }
-}
-
-// The preconditioner of the current geometry on the device: lists uploaded
-// once per coordinates, tensors B recomputed before the first mixed solve of a
+// The preconditioner of the current geometry on the device: lists built once per
+// coordinates (the sites closer than kNbCut, each row in site order), tensors B recomputed before the first mixed solve of a
 // geometry (and after a reset of the static field), which also clears a
 // breakdown switch-off.
 void ensure_nb(System &s, DeviceState &d) {
     NbDev &nb = d.nb;
     if (!nb.list_valid) {
-        std::vector<int> rp, ci;
-        build_nb_lists(s, rp, ci);
-        const long nnz = (long)ci.size();
-        if (!nb.row_ptr) {
-            nb.row_ptr = dalloc<int>(d, s.npol + 1);
+        ensure_grid(s, d);
+        if (!nb.off_flag) {
             nb.off_flag = dalloc<int>(d, 1);
             d.vr3 = dalloc<double>(d, 2 * d.n);
             d.red_d = dalloc<double>(d, 2 * (size_t)nb_blocks(s.npol) + 8);
         }
-        if (nnz > nb.cap) {
+        nb.nnz = d.grid.nnz;
+        if (nb.nnz > nb.cap) {
             dfree(d, nb.ci);
             dfree(d, nb.rowi);
             dfree(d, nb.b);
-            nb.cap = std::max(1L, nnz + nnz / 4);
+            nb.cap = nb.nnz + nb.nnz / 4;
+        }
+        if (!nb.ci) {
+            nb.cap = std::max(1L, nb.cap);
             nb.ci = dalloc<int>(d, nb.cap);
             nb.rowi = dalloc<int>(d, nb.cap);
             nb.b = dalloc<float>(d, 6 * (size_t)nb.cap);
         }
-        std::vector<int> rowi(nnz);
-        for (int i = 0; i < s.npol; i++)
-            for (int k = rp[i]; k < rp[i + 1]; k++) rowi[k] = i;
-        upload(rp.data(), nb.row_ptr, sizeof(int) * (s.npol + 1));
-        upload(ci.data(), nb.ci, sizeof(int) * nnz);
-        upload(rowi.data(), nb.rowi, sizeof(int) * nnz);
-        nb.nnz = nnz;
+        launch_nb_lists(d.stream, s.npol, d.grid, d.polar_mm, d.mm_polar, d.ms64, nb.row_ptr, nb.ci, nb.rowi);
         nb.list_valid = true;
         nb.valid = false;
     }
@@ -722,13 +716,13 @@ struct CgResult {
     double beta[2] = {0, 0};
 };
 
-    const bool small = !nb && cg_small(n);
 // With nb (inner solves of the mixed solver, zero guess only) the iterations
 // use the near-field preconditioner, r alternating between vr and vr3.
 CgResult cg_solve(System &s, DeviceState &d, int kind, int M, const double *b, double *x, const double *tol,
                   int maxit, bool zero_guess, double small_step_eps, int slot, bool nb = false) {
     const long n = d.n;
     CgResult res;
+    const bool small = !nb && cg_small(n);
     double te[4] = {tol[0], M > 1 ? tol[1] : tol[0], small_step_eps, small_step_eps};
     if (!small) HCHECK(hipMemcpyAsync(d.tol_dev, te, sizeof(te), hipMemcpyHostToDevice, d.stream));
     if (nb && !zero_guess) fatal("Internal error: the near-field preconditioned solve starts from zero");
@@ -753,14 +747,14 @@ CgResult cg_solve(System &s, DeviceState &d, int kind, int M, const double *b, d
     bool all_done = false;
     while (it <= maxit && !all_done) {
         const int end = std::min(maxit, it + chunk - 1);
-            } else if (small) {
-                launch_cg_step(d.stream, n, M, it, d.vh, x, d.vr, d.vp, d.alpha, d.red_b, nred_hp, d.cs);
         for (; it <= end; it++) {
             matvec(s, d, kind, M, d.vp, d.vh, true, d.red_b, d.cs);
             if (nb) {
                 launch_cg_update_nb(d.stream, s.npol, M, it, d.vh, x, rb[(it - 1) & 1], rb[it & 1], d.vz, d.vp,
                                     d.alpha, d.red_b, nred_hp, d.red_c, d.red_d, d.cs, d.nb);
                 launch_cg_direction_nb(d.stream, s.npol, M, it, d.vz, d.vp, d.red_c, d.red_d, d.cs, d.nb);
+            } else if (small) {
+                launch_cg_step(d.stream, n, M, it, d.vh, x, d.vr, d.vp, d.alpha, d.red_b, nred_hp, d.cs);
             } else {
                 launch_cg_update(d.stream, n, M, it, d.vh, x, d.vr, d.vz, d.vp, d.alpha, d.red_b, nred_hp, d.red_c,
                                  d.cs);
@@ -1277,8 +1271,7 @@ double fixedelec_energy(System &s) {
     int bad = 0;
     std::memcpy(&bad, d.scal_host + 1, sizeof(int));
     if (bad)
-        fatal("Requesting Coulomb kernel for two atoms placed in the same point, this could be an internal bug "
-              "or a problem in your input file, please check.");
+        fatal(kCoincident);
     s.e_mm = d.scal_host[0];
     s.m2m_done = true;
     return s.e_mm;
@@ -1297,7 +1290,8 @@ void refresh_host_ipd(System &s) {
 size_t device_footprint_estimate(const System &s) {
     const size_t np = s.npol, nm = s.nmm, n = 3 * np;
     size_t b = np * (sizeof(double4) + sizeof(float4) + 3 * sizeof(double) + sizeof(float) + sizeof(int));
-    b += nm * (sizeof(double4) + sizeof(double) + sizeof(double) * s.ld_cart + sizeof(int));
+    b += nm * (sizeof(double4) + 5 * sizeof(double) + sizeof(double) * s.ld_cart + 5 * sizeof(int));
+    b += (np + 20 * nm) * sizeof(int);                     // grid: rows, cells (at most ~8 per atom, two arrays)
     b += sizeof(double) * (2 * n * 2 + n + 8 * 2 * n);     // e_m2d, ipd, ext, work vectors
     b += 3 * 24 * sizeof(double) * (n / kBlock + 16) + 2 * sizeof(double) * tmv_rows_dot_parts(s.npol, 64, 2);  // reductions
     b += sizeof(double) * n * 16 + (size_t(4) << 20);      // static-field partials
@@ -1480,8 +1474,7 @@ void x2e_host(System &s, int n, const double *cext, bool mm, bool pol, double *V
     HCHECK(hipMemcpyAsync(&bad, d.x2e_bad, sizeof(int), hipMemcpyDeviceToHost, d.stream));
     HCHECK(hipStreamSynchronize(d.stream));
     if (bad)
-        fatal("Requesting Coulomb kernel for two atoms placed in the same point, this could be an internal bug "
-              "or a problem in your input file, please check.");
+        fatal(kCoincident);
     for (long j = 0; j < n; j++) {
         if (V) V[j] += out[4 * j];
         if (E)
@@ -1507,8 +1500,7 @@ void x2e_field_noalloc_host(System &s, int n, const double *cext, double *E) {
     const int bad = x2e_field_noalloc(d.stream, d.device, n, cext, true, pol, s.amoeba, s.ld_cart, s.nmm, d.ms64,
                                       d.mq, s.npol, d.ps64, d.ipd, E);
     if (bad)
-        fatal("Requesting Coulomb kernel for two atoms placed in the same point, this could be an internal bug "
-              "or a problem in your input file, please check.");
+        fatal(kCoincident);
 }
 
 namespace {
@@ -1527,8 +1519,6 @@ void ensure_grad(System &s, DeviceState &d) {
     }
     if (d.grad_static_ready) return;
     const int nmm = s.nmm, npol = s.npol;
-    d.mm_polar = dalloc<int>(d, nmm);
-    upload(s.mm_polar.data(), d.mm_polar, sizeof(int) * nmm);
     std::vector<int> rri(nmm + 1, 0), rci;
     if (s.amoeba) {
         d.q0 = dalloc<double>(d, 10L * nmm);

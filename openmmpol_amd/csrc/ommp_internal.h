@@ -103,7 +103,7 @@ System *build_from_arrays(int ff_type, int ff_rules, int nmm, const double *cmm,
 void prepare(System &s);                 // mmpol_prepare
 void rotate_multipoles(System &s);
 void make_screening_lists(System &s);
-void check_coincident_sites(const System &s);
+bool coincident_sites(const System &s);
 void set_default_scales(System &s);
 
 // io.cpp

@@ -22,9 +22,8 @@
 // never changes halfway.
 //
 // The neighbour lists (pairs closer than the cut, each row in site order) are
-// a function of the coordinates alone and are built on the host with a cell
-// grid when the coordinates are uploaded (engine.cpp), next to the
-// coincident-site check; the tensors B are computed on the device, one thread
+// a function of the coordinates alone and are built with the cell grid that also
+// serves the coincident-site check (geom.hip); the tensors B are computed on the device, one thread
 // per list entry, before the first mixed solve of a geometry.  Four lanes share
 // a site in the CG kernels below, each summing every fourth neighbour, so that
 // a site's chain of dependent loads is short.

@@ -7,7 +7,6 @@
 #include <cstring>
 #include <fstream>
 #include <sstream>
-#include <unordered_map>
 
 #include "ommp_internal.h"
 
@@ -565,46 +564,21 @@ void make_screening_lists(System &s) {
 }
 
 // coulomb_kernel refuses two sites closer than eps_rp (mod_electrostatics.F90:1003-1008);
-// every pair with a polarizable end is evaluated, so check those up front with a grid.
-void check_coincident_sites(const System &s) {
-    if (s.npol == 0) return;
-    struct Key {
-        long x, y, z;
-        bool operator==(const Key &o) const { return x == o.x && y == o.y && z == o.z; }
-    };
-    struct Hash {
-        size_t operator()(const Key &k) const {
-            return (size_t)(k.x * 73856093L) ^ (size_t)(k.y * 19349663L) ^ (size_t)(k.z * 83492791L);
-        }
-    };
-    std::unordered_map<Key, std::vector<int>, Hash> grid;
-    grid.reserve(2 * s.nmm);
-    auto key = [&](int i) {
-        return Key{(long)std::floor(s.cmm[3 * i]), (long)std::floor(s.cmm[3 * i + 1]),
-                   (long)std::floor(s.cmm[3 * i + 2])};
-    };
-    for (int i = 0; i < s.nmm; i++) grid[key(i)].push_back(i);
+// every pair with a polarizable end is evaluated, so check those up front.  All
+// pairs, for systems too small for the device's grid.
+bool coincident_sites(const System &s) {
     for (int p = 0; p < s.npol; p++) {
         const int i = s.polar_mm[p];
-        Key k = key(i);
-        for (long dx = -1; dx <= 1; dx++)
-            for (long dy = -1; dy <= 1; dy++)
-                for (long dz = -1; dz <= 1; dz++) {
-                    auto it = grid.find(Key{k.x + dx, k.y + dy, k.z + dz});
-                    if (it == grid.end()) continue;
-                    for (int j : it->second) {
-                        if (j == i) continue;
-                        double d2 = 0;
-                        for (int c = 0; c < 3; c++) {
-                            double d = s.cmm[3 * i + c] - s.cmm[3 * j + c];
-                            d2 += d * d;
-                        }
-                        if (std::sqrt(d2) < kEpsRp)
-                            fatal("Requesting Coulomb kernel for two atoms placed in the same point, this "
-                                  "could be an internal bug or a problem in your input file, please check.");
-                    }
-                }
+        for (int j = 0; j < s.nmm; j++) {
+            double d2 = 0;
+            for (int c = 0; c < 3; c++) {
+                const double d = s.cmm[3 * i + c] - s.cmm[3 * j + c];
+                d2 += d * d;
+            }
+            if (j != i && std::sqrt(d2) < kEpsRp) return true;
+        }
     }
+    return false;
 }
 
 }  // namespace ommp

@@ -100,3 +100,50 @@ def test_external_points(npoints, amoeba):
         got = getattr(s, f"field_{name}2ext")(c)
         assert np.abs(got - e).max() <= 1e-12 * np.abs(e).max(), name
     s.terminate()
+
+
+@pytest.mark.parametrize("n,spacing", [(1, 4.0), (2, 4.0), (161, 4.0), (700, 3.0), (125, 0.9)])
+def test_neighbour_lists(n, spacing):
+    """The near-field preconditioner (lists built with the device's grid) against
+    2 alpha r - alpha T_near alpha r from the oracle's dense T, before and after a
+    change of coordinates: no neighbours, a few, rows longer than the 64 gathered
+    at once.  FP32 tensors: 2e-6 of the largest component, as the 3,000-site test."""
+    spec = chain(n, True, seed=8)
+    rng = np.random.default_rng(9)
+    cut = 3.0 * 1.8897261245650
+    s = None
+    for scale in (1.0, 1.13):
+        spec["cmm"] = spec["cmm"] / (4.0 if scale == 1.0 else spacing) * spacing * scale
+        if s is None:
+            s, o = pair(spec)
+        else:
+            s.update_coordinates(spec["cmm"])
+            o = pair(spec)[1]
+        d = np.linalg.norm(spec["cmm"][:, None] - spec["cmm"][None], axis=2)
+        near = (d < cut) & (d > 0.0)
+        if n == 125:
+            assert near.sum(axis=1).max() > 64
+        al = np.repeat(spec["pol"], 3)
+        T = np.where(np.repeat(np.repeat(near, 3, 0), 3, 1), o.tmat(), 0.0)
+        r = rng.normal(size=(2, n, 3))
+        want = np.array([2.0 * al * v - al * (T @ (al * v)) for v in r.reshape(2, -1)]).reshape(2, n, 3)
+        z, on = s.inner_precond_apply(r)
+        assert on and np.abs(z - want).max() <= 2e-6 * np.abs(want).max()
+    s.terminate()
+
+
+@pytest.mark.parametrize("n", [10, 300])
+def test_coincident_sites_are_refused(n):
+    """Two atoms at one point end the process with the reference's message, on the
+    host's check (10 atoms) and on the grid's (300)."""
+    import os
+    import subprocess
+    import sys
+    code = ("import sys; sys.path[:0] = ['tests', '.']; import numpy as np, test_gpu_rows as t\n"
+            f"spec = t.chain({n}, True); spec['cmm'][{n - 3}] = spec['cmm'][1]\n"
+            "s, _ = t.pair(spec); print('built', flush=True)\n"
+            f"s.set_external_field(np.zeros(({n}, 3))); print('solved')\n")
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    p = subprocess.run([sys.executable, "-c", code], cwd=root, capture_output=True, text=True, timeout=100)
+    assert p.returncode == 1 and "built" in p.stdout and "solved" not in p.stdout
+    assert "two atoms placed in the same point" in p.stdout + p.stderr
