@@ -10,6 +10,7 @@
 #include <cstring>
 #include <limits>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "batch.h"
@@ -507,6 +508,9 @@ void fmm_release(DeviceState &d) {
     d.fmm_valid = false;
 }
 
+// Whether the fast multipole matvec is the matrix-core one (order p_tab throughout).
+bool fmm_far_matvec(const DeviceState &d) { return d.fmm.far.nc > 0 && d.fmm.p_pol == d.fmm.far.p; }
+
 // Octree, sorted copies of the sites and atoms, tables and expansion storage
 // for the current coordinates.
 void ensure_fmm(System &s, DeviceState &d) {
@@ -585,7 +589,58 @@ void ensure_fmm(System &s, DeviceState &d) {
     f.xs = fmm_alloc<double>(d, 9L * npol);
     f.mstatic = fmm_alloc<double2>(d, std::max<size_t>((size_t)(h.cell_off.back() - h.cell_off[h.levels]), 1) *
                                           f.ncoef_tab);
-    d.fmm_part = fmm_alloc<double>(d, (size_t)(kFmmNearSplits + 1) * 2 * 3 * npol);
+    if (fmm_uses_far(h.levels, h.p_tab)) {
+        FarDev<double> &r = f.far;
+        r.p = h.p_tab;
+        r.nc = far_coefs(h.p_tab);
+        r.lv.levels = h.levels;
+        r.lv.side = h.side;
+        for (int c = 0; c < 3; c++) r.lv.origin[c] = h.origin[c];
+        for (int l = 0; l < (int)h.cell_off.size(); l++) r.lv.off[l] = h.cell_off[l];
+        r.cells = h.levels >= 2 ? h.cell_off[h.levels + 1] - h.cell_off[2] : 0;
+        r.npol = npol;
+        r.leaf_start = f.pol_leaf_start;
+        r.order = f.pol_order;
+        r.leaf = f.pol_leaf;
+        r.pos = f.pol_pos;
+        r.a = f.pol_a;
+        auto up = [&](const auto &v) {
+            using T = std::decay_t<decltype(v[0])>;
+            T *p = fmm_alloc<T>(d, std::max<size_t>(v.size(), 1));
+            upload(v.data(), p, sizeof(T) * v.size());
+            return p;
+        };
+        auto group = [&](const std::vector<int> &cnt, FarGroups &g) {
+            std::vector<int> cell, level;
+            far_group_cells(r.lv, cnt, g.width, cell, level);
+            g.n = (int)level.size();
+            g.cell = up(cell);
+            g.level = up(level);
+        };
+        group(h.cnt_pol, r.groups);
+        group(h.cnt_mm, f.far_mm);
+        const int most = std::max(r.groups.n, f.far_mm.n);
+        r.nsplit = far_splits(most);
+        const FarTables<double> &t = far_tables<double>(r.p);
+        r.K = up(t.K);
+        r.K0 = up(t.K0);
+        r.zero = up(std::vector<double>(r.nc, 0.0));
+        r.mom = fmm_alloc<double>(d, (size_t)r.cells * r.nc);
+        r.mom_static = fmm_alloc<double>(d, (size_t)r.cells * r.nc);
+        r.mom0 = fmm_alloc<double>(d, r.cells);
+        r.part = fmm_alloc<double>(d, (size_t)r.nsplit * most * 32 * r.nc);
+        r.grad = fmm_alloc<double>(d, (size_t)r.cells * 3 * kFarBasis);
+        r.basis = fmm_alloc<double>(d, (size_t)std::max(h.levels - 1, 0) * npol * kFarBasis);
+        std::vector<int2> blocks;
+        const int T = kFarNearTargets;
+        for (int k = 0; k + 1 < (int)h.pol_leaf_start.size(); k++)
+            for (int t0 = h.pol_leaf_start[k]; t0 < h.pol_leaf_start[k + 1]; t0 += T) blocks.push_back(make_int2(k, t0));
+        r.nblocks = (int)blocks.size();
+        r.blocks = up(blocks);
+        r.dots = fmm_alloc<double>(d, r.nblocks);
+        far_launch_basis(d.stream, r, d.ps64);
+    }
+    if (!fmm_far_matvec(d)) d.fmm_part = fmm_alloc<double>(d, (size_t)(kFmmNearSplits + 1) * 2 * 3 * npol);
     d.fmm_rhs_part = fmm_alloc<double>(d, (size_t)(kFmmNearSplits + 1) * 3 * npol);
     fmm_launch_static_moments(d.stream, f, ld);
     d.fmm_valid = true;
@@ -606,7 +661,11 @@ void ensure_sym(const System &s, DeviceState &d) {
 }
 
 // Number of y.x partials per column that matvec() of this kind writes to dotpart.
-static int matvec_dot_parts(const System &s, int kind, int M) {
+static int matvec_dot_parts(System &s, DeviceState &d, int kind, int M) {
+    if (kind == kFmm) {
+        ensure_fmm(s, d);
+        if (fmm_far_matvec(d)) return kFarDots;
+    }
     const int prec = kind == kOtf32 ? 32 : 64;
     if (kind == kOtf64 || kind == kOtf32)
         return tmv_pair_once(s.npol, prec, M) ? tmv_sym_dot_parts(s.npol)
@@ -619,6 +678,13 @@ void matvec(System &s, DeviceState &d, int kind, int M, const double *x, double 
     const long n = d.n;
     if (kind == kFmm) {
         ensure_fmm(s, d);
+        if (fmm_far_matvec(d)) {
+            const FarDev<double> &r = d.fmm.far;
+            for (int m = 0; m < M; m++)
+                far_launch_matvec(d.stream, r, s.amoeba, 1, d.fmm.cnt_pol, d.ps64, d.pa64, d.alpha, d.pp, x + m * n,
+                                  n, y + m * n, n, dodiag, dotpart ? dotpart + m * kFarDots : nullptr, skip ? skip + m : nullptr);
+            return;
+        }
         fmm_launch_matvec_fields(d.stream, d.fmm, s.amoeba, M, x, n, d.fmm_part);
         launch_tmv_finalize64(d.stream, s.amoeba, s.npol, M, d.fmm_part, kFmmNearSplits + 1, d.ps64, d.pa64, d.alpha,
                               d.pp, x, n, y, n, dodiag, dotpart, reinterpret_cast<const int *>(skip));
@@ -739,7 +805,7 @@ CgResult cg_solve(System &s, DeviceState &d, int kind, int M, const double *b, d
                           nullptr);
     else
         launch_cg_init(d.stream, n, M, b, d.vh, x, d.vr, d.vz, d.vp, d.alpha, d.red_a, d.cs, zero_guess, d.tol_dev);
-    const int nred_hp = matvec_dot_parts(s, kind, M);
+    const int nred_hp = matvec_dot_parts(s, d, kind, M);
     int it = 1;
     // first batch: as many iterations as this call site needed last time
     const int pred = (slot >= 0 && slot < 16) ? s.pred_iters[slot] : 0;
@@ -927,7 +993,7 @@ int mixed_solve_ahead(System &s, DeviceState &d, int M, const double *b, double 
         HCHECK(hipHostMalloc((void **)&d.cs_spec_host, W * sizeof(CgState), hipHostMallocDefault));
     }
     CgState *out = d.cs_spec;
-    const int nred_hp = matvec_dot_parts(s, kind32, M);
+    const int nred_hp = matvec_dot_parts(s, d, kind32, M);
     bool xzero = zero_guess;
     for (int o = 0; o < K; o++) {
         if (xzero) {

@@ -202,7 +202,9 @@ FmmHost fmm_build(const System &s, int p_pol, int p_static, double min_cell, dou
     f.ncoef2_tab = (2 * pt + 1) * (2 * pt + 1);
     f.tab_m2m.assign((size_t)(L + 1) * 8 * f.ncoef_tab, make_double2(0.0, 0.0));
     f.tab_l2l.assign((size_t)(L + 1) * 8 * f.ncoef_tab, make_double2(0.0, 0.0));
-    f.tab_m2l.assign((size_t)(L + 1) * 343 * f.ncoef2_tab, make_double2(0.0, 0.0));
+    // the complex M2L also serves an order below p_tab where the two orders differ
+    const bool m2l = !(fmm_uses_far(L, pt) && p_pol == p_static);
+    f.tab_m2l.assign(m2l ? (size_t)(L + 1) * 343 * f.ncoef2_tab : 1, make_double2(0.0, 0.0));
     for (int l = 0; l <= L; l++) {
         const double h = side / (double)(1 << l);
         if (l < L)
@@ -212,7 +214,7 @@ FmmHost fmm_build(const System &s, int p_pol, int p_static, double min_cell, dou
                 r_all(pt, v, &f.tab_m2m[((size_t)l * 8 + oct) * f.ncoef_tab]);
                 s_all(pt, v, &f.tab_l2l[((size_t)l * 8 + oct) * f.ncoef_tab]);
             }
-        if (l >= 2)
+        if (l >= 2 && m2l)
             for (int dz = -3; dz <= 3; dz++)
                 for (int dy = -3; dy <= 3; dy++)
                     for (int dx = -3; dx <= 3; dx++) {

@@ -9,6 +9,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "far.h"
+
 namespace ommp {
 
 constexpr int kFmmMaxLevels = 7;   // 2^21 leaves at most (dense per-level arrays)
@@ -44,7 +46,11 @@ struct FmmDev {
     double2 *mexp = nullptr, *lexp = nullptr;
     double2 *tab_m2m = nullptr;    // [level][8][ncoef_tab]   R(c_child - c_parent), parent level
     double2 *tab_l2l = nullptr;    // [level][8][ncoef_tab]   S(c_child - c_parent), parent level
-    double2 *tab_m2l = nullptr;    // [level][343][ncoef2_tab] T(c_source - c_target)
+    double2 *tab_m2l = nullptr;    // [level][343][ncoef2_tab] T(c_source - c_target) where far is not used
+    // transfer and T matvec on the matrix cores for order p_tab (far.h), where
+    // far.nc > 0; target groups of the polarizable sites (far.groups) and MM atoms
+    FarDev<double> far;
+    FarGroups far_mm;
     double *xs = nullptr;          // sorted dipole columns [3][npol][3]
     double2 *mstatic = nullptr;    // [nleaf][ncoef_tab] static multipole moments of the leaves (order p_tab)
 };

@@ -24,6 +24,10 @@ struct FmmHost {
 
 // Octree with leaves of side >= max(min_cell, distance) (bohr) over the MM
 // atoms of s, at most kFmmMaxLevels levels below the root.
+// Whether trees of L levels and order p use the matrix-core transfer and matvec
+// (far.h): orders up to 8, and up to 6 levels (their per-cell arrays stay under
+// 0.5 GB); others use the complex kernels and tables.
+inline bool fmm_uses_far(int L, int p) { return L <= 6 && far_order(p); }
 FmmHost fmm_build(const System &s, int p_pol, int p_static, double min_cell, double distance);
 
 }  // namespace ommp

@@ -935,26 +935,49 @@ static void leaf_static(hipStream_t st, const FmmDev &f, int p, double2 *leafm) 
     HIP_CHECK(hipGetLastError());
 }
 
-// Local expansions at the leaves of one source set (already expanded into the
-// leaf multipoles at level L): M2M, M2L, L2L; cells with no target (cnt_tgt)
-// are skipped.  False when the tree has no far field (L < 2).
-static bool far_locals(hipStream_t st, const FmmDev &f, int p, const int *cnt_src, const int *cnt_tgt) {
-    const int L = f.levels;
+// Moments of the levels 2 .. L - 1 from the leaves' (cells with no source are skipped).
+static void moments_up(hipStream_t st, const FmmDev &f, int p, const int *cnt_src) {
     const int ncoef = (p + 1) * (p + 1);
-    if (L < 2) return false;
-    for (int l = L - 1; l >= 2; l--) {
+    for (int l = f.levels - 1; l >= 2; l--) {
         const int ns = 1 << l;
         hipLaunchKernelGGL(k_fmm_m2m, dim3(ns * ns * ns), dim3(256), sizeof(double2) * ncoef, st, p, ns,
                            cnt_src + f.cell_off[l + 1], f.mexp + f.cell_off[l + 1] * ncoef,
                            f.tab_m2m + (long)l * 8 * f.ncoef_tab, f.ncoef_tab, f.mexp + f.cell_off[l] * ncoef);
         HIP_CHECK(hipGetLastError());
     }
-    for (int l = 2; l <= L; l++) {
-        const int ns = 1 << l;
-        hipLaunchKernelGGL(k_fmm_m2l, dim3(ns * ns * ns), dim3(256), lds_m2l(p), st, p, ns, cnt_src + f.cell_off[l],
-                           cnt_tgt + f.cell_off[l], f.mexp + f.cell_off[l] * ncoef,
-                           f.tab_m2l + (long)l * 343 * f.ncoef2_tab, f.ncoef2_tab, f.lexp + f.cell_off[l] * ncoef);
-        HIP_CHECK(hipGetLastError());
+}
+
+// Local expansions at the leaves of one source set: the static multipoles of the
+// MM atoms (with_static) and / or the dipoles dip[npol][3] of the sorted
+// polarizable sites; cells with no target (cnt_tgt) are skipped.  On the matrix
+// cores (far.h) where the order has its tables, else leaf moments, M2M and M2L;
+// then L2L.  False when the tree has no far field (L < 2).
+static bool far_locals(hipStream_t st, const FmmDev &f, int p, bool with_static, const double *dip,
+                       const int *cnt_tgt) {
+    const int L = f.levels, nleaf = 1 << 3 * L;
+    const int ncoef = (p + 1) * (p + 1);
+    if (L < 2) return false;
+    const int *cnt_src = with_static ? f.cnt_mm : f.cnt_pol;
+    if (f.far.nc > 0 && f.far.p == p) {
+        const FarGroups &pol = f.far.groups;
+        far_launch_locals(st, f.far, cnt_tgt == f.cnt_mm ? f.far_mm : pol, with_static ? f.far_mm : pol, cnt_src,
+                          with_static, dip, f.lexp);
+    } else {
+        double2 *leafm = f.mexp + f.cell_off[L] * ncoef;
+        if (with_static) leaf_static(st, f, p, leafm);
+        if (dip) {
+            hipLaunchKernelGGL(k_fmm_p2m<0>, dim3(p2m_blocks(p, nleaf)), dim3(256), 0, st, p, 1 << L, f.leaf_h,
+                               f.origin, nleaf, f.pol_leaf_start, f.pol_pos, dip, 3, (int)with_static, leafm);
+            HIP_CHECK(hipGetLastError());
+        }
+        moments_up(st, f, p, cnt_src);
+        for (int l = 2; l <= L; l++) {
+            const int ns = 1 << l;
+            hipLaunchKernelGGL(k_fmm_m2l, dim3(ns * ns * ns), dim3(256), lds_m2l(p), st, p, ns,
+                               cnt_src + f.cell_off[l], cnt_tgt + f.cell_off[l], f.mexp + f.cell_off[l] * ncoef,
+                               f.tab_m2l + (long)l * 343 * f.ncoef2_tab, f.ncoef2_tab, f.lexp + f.cell_off[l] * ncoef);
+            HIP_CHECK(hipGetLastError());
+        }
     }
     for (int l = 2; l < L; l++) {
         const int ns = 1 << (l + 1);
@@ -968,10 +991,10 @@ static bool far_locals(hipStream_t st, const FmmDev &f, int p, const int *cnt_sr
 
 // Far field of one source set at the polarizable sites: local expansions, then
 // L2P into field[npol][3].
-static void far_field(hipStream_t st, const FmmDev &f, int p, const int *cnt_src, double *field) {
+static void far_field(hipStream_t st, const FmmDev &f, int p, bool with_static, const double *dip, double *field) {
     const int L = f.levels;
     const int ncoef = (p + 1) * (p + 1);
-    if (far_locals(st, f, p, cnt_src, f.cnt_pol)) {
+    if (far_locals(st, f, p, with_static, dip, f.cnt_pol)) {
         hipLaunchKernelGGL(k_fmm_l2p, dim3((f.npol + 255) / 256), dim3(256), 0, st, p, f.npol, 1 << L, f.leaf_h,
                            f.origin, f.pol_pos, f.pol_leaf, f.pol_order, f.lexp + f.cell_off[L] * ncoef, field);
         HIP_CHECK(hipGetLastError());
@@ -982,9 +1005,8 @@ static void far_field(hipStream_t st, const FmmDev &f, int p, const int *cnt_src
 
 void fmm_launch_matvec_fields(hipStream_t st, const FmmDev &f, bool amoeba, int M, const double *x, long xstride,
                               double *part) {
-    const int L = f.levels, ns = 1 << L, nleaf = ns * ns * ns;
+    const int L = f.levels, ns = 1 << L;
     const int p = f.p_pol;
-    const int ncoef = (p + 1) * (p + 1);
     const long n3 = 3L * f.npol;
     hipLaunchKernelGGL(k_fmm_gather, dim3((f.npol + 255) / 256), dim3(256), 0, st, f.npol, M, f.pol_order, x,
                        xstride, f.xs);
@@ -999,21 +1021,13 @@ void fmm_launch_matvec_fields(hipStream_t st, const FmmDev &f, bool amoeba, int 
                            f.pol_order, f.pol_self, f.pol_leaf_start, f.pol_pos, f.pol_a, f.xs, 0, M, part);
     HIP_CHECK(hipGetLastError());
     // far field per column: split 27
-    for (int c = 0; c < M; c++) {
-        if (L >= 2) {
-            hipLaunchKernelGGL(k_fmm_p2m<0>, dim3(p2m_blocks(p, nleaf)), dim3(256), 0, st, p, ns, f.leaf_h,
-                               f.origin, nleaf, f.pol_leaf_start, f.pol_pos, f.xs + c * n3, 3, 0,
-                               f.mexp + f.cell_off[L] * ncoef);
-            HIP_CHECK(hipGetLastError());
-        }
-        far_field(st, f, p, f.cnt_pol, part + ((long)kFmmNearSplits * M + c) * n3);
-    }
+    for (int c = 0; c < M; c++)
+        far_field(st, f, p, false, f.xs + c * n3, part + ((long)kFmmNearSplits * M + c) * n3);
 }
 
 void fmm_launch_static_fields(hipStream_t st, const FmmDev &f, bool amoeba, int ld, double *part) {
     const int L = f.levels, ns = 1 << L;
     const int p = f.p_static;
-    const int ncoef = (p + 1) * (p + 1);
     const long n3 = 3L * f.npol;
     const dim3 ng((f.npol + 255) / 256, kFmmNearSplits);
     if (amoeba)
@@ -1023,8 +1037,7 @@ void fmm_launch_static_fields(hipStream_t st, const FmmDev &f, bool amoeba, int 
         hipLaunchKernelGGL((k_fmm_near<1, false>), ng, dim3(256), 0, st, f.npol, ns, f.pol_pos, f.pol_a, f.pol_leaf,
                            f.pol_order, f.pol_mmself, f.mm_leaf_start, f.mm_pos, f.mm_a, f.mm_q, ld, 1, part);
     HIP_CHECK(hipGetLastError());
-    if (L >= 2) leaf_static(st, f, p, f.mexp + f.cell_off[L] * ncoef);
-    far_field(st, f, p, f.cnt_mm, part + (long)kFmmNearSplits * n3);
+    far_field(st, f, p, true, nullptr, part + (long)kFmmNearSplits * n3);
 }
 
 void fmm_launch_static_moments(hipStream_t st, const FmmDev &f, int ld) {
@@ -1033,11 +1046,16 @@ void fmm_launch_static_moments(hipStream_t st, const FmmDev &f, int ld) {
     hipLaunchKernelGGL(k_fmm_p2m<1>, dim3(p2m_blocks(f.p_tab, nleaf)), dim3(256), 0, st, f.p_tab, ns, f.leaf_h,
                        f.origin, nleaf, f.mm_leaf_start, f.mm_pos, f.mm_q, ld, 0, f.mstatic);
     HIP_CHECK(hipGetLastError());
+    if (f.far.nc == 0) return;
+    // the moments of every level for the matrix-core transfer
+    leaf_static(st, f, f.p_tab, f.mexp + f.cell_off[L] * f.ncoef_tab);
+    moments_up(st, f, f.p_tab, f.cnt_mm);
+    far_launch_moments(st, f.far, f.mexp);
 }
 
 void fmm_launch_grad_fields(hipStream_t st, const FmmDev &f, bool amoeba, int ld, const double *ipd,
                             double *part_pol, double *part_mm) {
-    const int L = f.levels, ns = 1 << L, nleaf = ns * ns * ns;
+    const int L = f.levels, ns = 1 << L;
     const int npol = f.npol, nmm = f.nmm;
     const long n3 = 3L * npol;
     const int na = amoeba ? 12 : 3;
@@ -1072,29 +1090,19 @@ void fmm_launch_grad_fields(hipStream_t st, const FmmDev &f, bool amoeba, int ld
         return;
     }
     const int p = f.p_tab;
-    const int ncoef = (p + 1) * (p + 1);
-    double2 *leafm = f.mexp + f.cell_off[L] * ncoef;
-    const double2 *leafl = f.lexp + f.cell_off[L] * ncoef;
+    const double2 *leafl = f.lexp + f.cell_off[L] * (p + 1) * (p + 1);
     const dim3 lp((npol + 255) / 256), lm((nmm + 255) / 256);
     // polarizable targets: static multipoles + one dipole set per pass, contracted
     // with half of the other set (AMOEBA: P sources against D / 2, D against P / 2)
     for (int pass = 0; pass < npass; pass++) {
-        leaf_static(st, f, p, leafm);
-        const double *dip = amoeba ? f.xs + (pass == 0 ? n3 : 0) : f.xs;
-        hipLaunchKernelGGL(k_fmm_p2m<0>, dim3(p2m_blocks(p, nleaf)), dim3(256), 0, st, p, ns, f.leaf_h, f.origin,
-                           nleaf, f.pol_leaf_start, f.pol_pos, dip, 3, 1, leafm);
-        HIP_CHECK(hipGetLastError());
-        far_locals(st, f, p, f.cnt_mm, f.cnt_pol);
+        far_locals(st, f, p, true, amoeba ? f.xs + (pass == 0 ? n3 : 0) : f.xs, f.cnt_pol);
         const double c0 = amoeba ? (pass == 0 ? 0.5 : 0.0) : 1.0, c1 = amoeba ? (pass == 0 ? 0.0 : 0.5) : 0.0;
         hipLaunchKernelGGL(k_fmm_l2p_grad<0>, lp, dim3(256), 0, st, p, npol, ns, f.leaf_h, f.origin, f.pol_pos,
                            f.pol_leaf, f.pol_order, leafl, ipd, n3, c0, c1, f.mm_q, far_pol + pass * n3, (long)npol);
         HIP_CHECK(hipGetLastError());
     }
     // MM targets: the dipoles nu
-    hipLaunchKernelGGL(k_fmm_p2m<0>, dim3(p2m_blocks(p, nleaf)), dim3(256), 0, st, p, ns, f.leaf_h, f.origin, nleaf,
-                       f.pol_leaf_start, f.pol_pos, nu, 3, 0, leafm);
-    HIP_CHECK(hipGetLastError());
-    far_locals(st, f, p, f.cnt_pol, f.cnt_mm);
+    far_locals(st, f, p, false, nu, f.cnt_mm);
     if (amoeba)
         hipLaunchKernelGGL(k_fmm_l2p_grad<1>, lm, dim3(256), 0, st, p, nmm, ns, f.leaf_h, f.origin, f.mm_pos,
                            f.mm_leaf, f.mm_order, leafl, ipd, n3, 0.0, 0.0, f.mm_q, far_mm, (long)nmm);

@@ -1,0 +1,69 @@
+"""The matrix-core transfer and T matvec of the fast multipoles (orders up to 8)
+on small trees: one leaf, two per side (no far field), and far fields of two and
+three levels, odd sizes, orders whose coefficients fill 1 to 5 tiles; AMOEBA and
+AMBER.  Against the complex kernels, which an order of the static field above 8
+selects and which sum the same truncated expansions in another order: 1e-12 of
+the largest component (FP64 sums of a few thousand terms); and with no far field
+against the direct matvec, 1e-13."""
+import numpy as np
+import pytest
+
+from test_gpu_rows import chain
+
+pytestmark = pytest.mark.gpu
+
+
+def _system(n, amoeba):
+    from openmmpol_amd import OMMPSystem
+    spec = chain(n, amoeba, seed=n)
+    return OMMPSystem.from_arrays(amoeba, spec["cmm"], spec["q"], spec["pol"], spec["bonds_ri"], spec["bonds_ci"],
+                                  pgroup=spec["pgroup"] if amoeba else None)
+
+
+@pytest.mark.parametrize("amoeba", [True, False])
+@pytest.mark.parametrize("n,cell", [(7, 40.0), (301, 12.0), (1003, 8.0), (3001, 7.0)])
+def test_matvec_small_trees(n, cell, amoeba):
+    s = _system(n, amoeba)
+    x = np.random.default_rng(3).normal(0.0, 0.05, size=(2, n, 3))
+    want, _ = s.tmatvec(x, kind="plain64")
+    scale = np.abs(want).max()
+    for p in (2, 4, 6, 8):
+        s.enable_fmm(lmax=p, lmax_pol=p, distance=1.0, min_cell_size=cell)
+        y, _ = s.tmatvec(x, kind="fmm")
+        assert np.array_equal(s.tmatvec(x, kind="fmm")[0], y)
+        one, _ = s.tmatvec(x[:1], kind="fmm")
+        assert np.array_equal(one, y[:1])
+        s.enable_fmm(lmax=9, lmax_pol=p, distance=1.0, min_cell_size=cell)
+        old, _ = s.tmatvec(x, kind="fmm")
+        assert np.abs(y - old).max() <= 1e-12 * scale, p
+        if n == 7:
+            assert np.abs(y - want).max() <= 1e-13 * scale
+    s.terminate()
+
+
+@pytest.mark.parametrize("p", [1, 3, 5, 7, 8])
+def test_static_field_and_gradient_orders(p):
+    """The static field and the gradient through the transfer against the complex
+    kernels (selected by an order of 9 for the other of the two expansions where
+    the pass allows it: the gradient runs at the larger of the two orders, so it
+    is compared at 8 and 9 through the truncation error against the direct one)."""
+    n = 3001
+    s = _system(n, True)
+    direct = s.e_m2d
+    s.set_solver_tolerance(1e-10, 500)
+    s.set_external_field(np.zeros((n, 3)))
+    gd = s.polelec_geomgrad()
+    s.enable_fmm(lmax=p, lmax_pol=p, distance=1.0, min_cell_size=7.0)
+    new = s.e_m2d
+    s.enable_fmm(lmax=p, lmax_pol=9, distance=1.0, min_cell_size=7.0)
+    old = s.e_m2d
+    scale = np.abs(direct).max()
+    assert np.abs(new - old).max() <= 1e-12 * scale
+    if p == 8:
+        err = []
+        for q in (4, 8, 9):
+            s.enable_fmm(lmax=q, lmax_pol=q, distance=1.0, min_cell_size=7.0)
+            s.set_external_field(np.zeros((n, 3)))
+            err.append(np.abs(s.polelec_geomgrad() - gd).max() / np.abs(gd).max())
+        assert err[1] <= err[0] / 4.0 and err[2] <= 1.5 * err[1]
+    s.terminate()
