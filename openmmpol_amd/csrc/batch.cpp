@@ -45,12 +45,14 @@ SegLayout seg_layout(int npol, int nrhs, int nsets, int m32, int num_cu, int ext
     L.vec = align256(sizeof(double) * ncols * n);
     L.xs = m32 == kBatchM32 ? align256(sizeof(unsigned short) * kBxParts * ncols * (size_t)bx_ld(npol)) : 0;
     // the pair-once sweep from the sizes where it beats the batched per-target
-    // sweep (measured: FP32 11,000 sites with two columns, 7,000 with one; FP64
-    // 7,000 and 6,000), its partials under 8 GiB; wide batches run both matvecs
-    // on the matrix cores with their own tiling (partials per source split)
+    // sweep, its partials under 8 GiB (SCF sequences of six systems of 500 to 9,000
+    // sites: from 11,000 / 7,000 sites in FP32 / FP64 20.2 ms, from 6,000 / 5,000
+    // 17.5, from 4,000 17.6, from 2,500 18.1; three systems up to 4,000 sites: 7.3 ms
+    // below the limit, 9.5 above it); wide batches run both matvecs on the matrix
+    // cores with their own tiling (partials per source split)
     const bool sym_fits = m32 == 2 && tmv_sym_part_bytes(npol, std::max(ncols, 2), 64) <= size_t(8) << 30;
-    L.sym32 = sym_fits && npol >= (ncols >= 2 ? 11000 : 7000);
-    L.sym64 = sym_fits && npol >= (ncols >= 2 ? 7000 : 6000);
+    L.sym32 = sym_fits && npol >= 6000;
+    L.sym64 = sym_fits && npol >= 5000;
     size_t part = sizeof(double) * L.nsplit * ncols * n;
     if (L.sym32 || L.sym64) part = std::max(part, tmv_sym_part_bytes(npol, ncols, 64));
     L.part = align256(part);
@@ -192,6 +194,8 @@ int BatchEngine::add(const DeviceView &v, int nrhs, int extra) {
     d.amoeba = v.amoeba;
     d.ps32 = v.ps32;
     d.pa32 = v.pa32;
+    d.rc64 = v.rc64;
+    d.rc32 = v.rc32;
     d.ps64 = v.ps64;
     d.pa64 = v.pa64;
     d.alpha = v.alpha;
@@ -262,12 +266,13 @@ void BatchEngine::commit() {
     for (int si : order) {
         const BSeg &d = segs[si].dev;
         const int g32 = (d.ncols + m32 - 1) / m32, g64 = (d.ncols + m64 - 1) / m64;
-        // pair-once items: every block pair (I <= J), row-major (index order)
+        // pair-once items: every block pair (I <= J) with its index (row-major), the
+        // diagonal ones first: they take longest
         auto sym_items = [&](std::vector<int4> &out, int groups) {
             for (int g = 0; g < groups; g++) {
-                int idx = 0;
-                for (int I = 0; I < d.tblocks; I++)
-                    for (int J = I; J < d.tblocks; J++) out.push_back(make_int4(si, I | (J << 16), idx++, g));
+                for (int k = 0; k < d.tblocks; k++)
+                    for (int I = 0; I + k < d.tblocks; I++)
+                        out.push_back(make_int4(si, I | ((I + k) << 16), I * d.tblocks - I * (I - 1) / 2 + k, g));
             }
         };
         if (d.sym32) {

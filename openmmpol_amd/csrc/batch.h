@@ -66,6 +66,8 @@ struct BSeg {
     int amoeba;
     const float4 *ps32;
     const float *pa32;
+    const double *rc64;  // damping cutoffs of the sites (row_sweep.h)
+    const float *rc32;
     const double4 *ps64;
     const double *pa64;
     const double *alpha;
@@ -197,6 +199,8 @@ struct DeviceView {
     const double *pa64;
     const float4 *ps32;
     const float *pa32;
+    const double *rc64;  // damping cutoffs of the sites (row_sweep.h)
+    const float *rc32;
     const double *alpha;
     CsrDev pp;
     const double *e_m2d;

@@ -19,10 +19,12 @@ template <typename R> struct SegSites;
 template <> struct SegSites<float> {
     __device__ static const float4 *site(const BSeg &s) { return s.ps32; }
     __device__ static const float *damp(const BSeg &s) { return s.pa32; }
+    __device__ static const float *cut(const BSeg &s) { return s.rc32; }
 };
 template <> struct SegSites<double> {
     __device__ static const double4 *site(const BSeg &s) { return s.ps64; }
     __device__ static const double *damp(const BSeg &s) { return s.pa64; }
+    __device__ static const double *cut(const BSeg &s) { return s.rc64; }
 };
 
 // Does column c take part in this matvec?  FP32 (use_p): inner PCG columns in
@@ -32,7 +34,7 @@ __device__ __forceinline__ bool mv_active(const BCol &c, int use_p) {
 }
 
 // Grouped on-the-fly pair kernel body: one target per thread, sources of one
-// split staged through LDS, MM columns cidx[] (as k_tmv_pairs).
+// split staged through LDS, MM columns cidx[] (per-pair arithmetic of pair_math.h).
 template <typename R, int MM, bool AMOEBA>
 __device__ __forceinline__ void bpairs_body(const BSeg &S, const int4 w, const double *__restrict__ xin,
                                             const int (&cidx)[MM]) {
@@ -47,10 +49,11 @@ __device__ __forceinline__ void bpairs_body(const BSeg &S, const int4 w, const d
     const int j = w.y * kBlock + tid;
     const bool valid = j < npol;
     R4 pj;
-    R aj;
+    R aj, rj = R(0);
     if (valid) {
         pj = site[j];
         aj = adamp[j];
+        rj = SegSites<R>::cut(S)[j];
     } else {
         pj.x = pj.y = pj.z = R(0);
         pj.w = R(1);
@@ -103,13 +106,18 @@ __device__ __forceinline__ void bpairs_body(const BSeg &S, const int4 w, const d
                 xa[m] = s_x[m][k];
                 xb[m] = s_x[m][k + 1];
             }
-            R dxa, dya, dza, k2a, k3a, arga, dxb, dyb, dzb, k2b, k3b, argb;
-            bool neara, nearb;
-            pair_geom<R, AMOEBA>(pj, aj, s_pos[k], xa[0].w, dxa, dya, dza, k2a, k3a, arga, neara);
-            pair_geom<R, AMOEBA>(pj, aj, s_pos[k + 1], xb[0].w, dxb, dyb, dzb, k2b, k3b, argb, nearb);
-            if (__ballot(neara || nearb)) {
-                pair_damp<R, AMOEBA>(arga, neara, k2a, k3a);
-                pair_damp<R, AMOEBA>(argb, nearb, k2b, k3b);
+            // the self pair is inside its site's cutoff: guarded in the branch
+            const R4 pa = s_pos[k], pb = s_pos[k + 1];
+            R dxa, dya, dza, k2a, k3a, dxb, dyb, dzb, k2b, k3b;
+            const R r2a = pair_bare<R>(pj, pa, dxa, dya, dza, k2a, k3a);
+            const R r2b = pair_bare<R>(pj, pb, dxb, dyb, dzb, k2b, k3b);
+            if (__ballot(r2a < rj || r2b < rj)) {
+                R arg;
+                bool near;
+                pair_geom<R, AMOEBA>(pj, aj, pa, xa[0].w, dxa, dya, dza, k2a, k3a, arg, near);
+                pair_damp<R, AMOEBA>(arg, near, k2a, k3a);
+                pair_geom<R, AMOEBA>(pj, aj, pb, xb[0].w, dxb, dyb, dzb, k2b, k3b, arg, near);
+                pair_damp<R, AMOEBA>(arg, near, k2b, k3b);
             }
             pair_accum<R, MM>(acc, xa, dxa, dya, dza, k2a, k3a);
             pair_accum<R, MM>(acc, xb, dxb, dyb, dzb, k2b, k3b);
@@ -182,7 +190,7 @@ __device__ __forceinline__ void bsym_body(const BSeg &S, const int4 w, const dou
         oj[m] = part_j + o;
     }
     sym_block_pair_any<R, M, AMOEBA>(S.npol, w.y & 0xffff, w.y >> 16, SegSites<R>::site(S), SegSites<R>::damp(S),
-                                     xcol, oi, oj, lds);
+                                     SegSites<R>::cut(S), xcol, oi, oj, lds);
 }
 
 template <typename R, int M, bool AMOEBA>

@@ -86,12 +86,13 @@ void launch_rhs_sym(hipStream_t st, bool amoeba, int nmm, int npol, const int2 *
 
 // T matvec on the fly, per target (tmv_rows.hip): y[m] = T x[m] (dodiag) or (T - diag) x[m], m < M.
 // prec 64 or 32 selects the pair arithmetic; corrections and the final sum are FP64.
-// If dotpart != nullptr, per-workgroup partial sums of y.x go to dotpart[m * nparts + b].
+// rc64 / rc32: damping cutoffs of the sites (row_sweep.h).  If dotpart != nullptr,
+// per-workgroup partial sums of y.x go to dotpart[m * nparts + b].
 void launch_tmv_rows(hipStream_t st, int prec, bool amoeba, int npol, int M, const double4 *ps64,
-                     const double *pa64, const float4 *ps32, const float *pa32, const double *alpha,
-                     const CsrDev &pp, const double *x, long xstride, double *y, long ystride,
-                     bool dodiag, double *dotpart, const int *skip_flag, hipEvent_t evb = nullptr,
-                     hipEvent_t eve = nullptr);
+                     const double *pa64, const float4 *ps32, const float *pa32, const double *rc64,
+                     const float *rc32, const double *alpha, const CsrDev &pp, const double *x, long xstride,
+                     double *y, long ystride, bool dodiag, double *dotpart, const int *skip_flag,
+                     hipEvent_t evb = nullptr, hipEvent_t eve = nullptr);
 int tmv_rows_dot_parts(int npol, int prec, int ncols);  // per-column y.x partials it writes
 // Finalize alone, for FP64 partial fields computed elsewhere (fast multipoles).
 void launch_tmv_finalize64(hipStream_t st, bool amoeba, int npol, int M, const double *part, int nsplit,
@@ -105,11 +106,11 @@ int tmv_sym_blocks(int npol);
 // Per-column y.x partials written by the pair-once matvec's finalize.
 int tmv_sym_dot_parts(int npol);
 size_t tmv_sym_part_bytes(int npol, int M, int prec);
-// Whether the on-the-fly matvec of prec (32 / 64) with ncols columns uses the
-// pair-once sweep at npol sites.
-bool tmv_pair_once(int npol, int prec, int ncols);
+// Whether the on-the-fly matvec with ncols columns uses the pair-once sweep at npol
+// sites.
+bool tmv_pair_once(int npol, int ncols);
 void launch_tmv_sym(hipStream_t st, int prec, bool amoeba, int npol, int M, const int2 *pairs, const double4 *ps64,
-                    const double *pa64, const float4 *ps32, const float *pa32, const double *alpha,
+                    const double *pa64, const float4 *ps32, const float *pa32, const double *rc64, const float *rc32, const double *alpha,
                     const CsrDev &pp, const double *x, long xstride, double *y, long ystride, bool dodiag,
                     double *dotpart, void *part, const int *skip_flag, hipEvent_t evb = nullptr,
                     hipEvent_t eve = nullptr);

@@ -46,6 +46,8 @@ struct DeviceState {
     double *pa64 = nullptr, *alpha = nullptr;
     float4 *ps32 = nullptr;
     float *pa32 = nullptr;
+    double *rc64 = nullptr;  // squared distance beyond which no pair of a site is damped
+    float *rc32 = nullptr;
     int *polar_mm = nullptr;
     double4 *ms64 = nullptr;
     double *ma64 = nullptr, *mq = nullptr, *cmm = nullptr, *mw = nullptr;  // mw: 1 / thole
@@ -400,6 +402,29 @@ void upload_sites(System &s, DeviceState &d) {
         pa[p] = s.thole_damping_mm[s.polar_mm[p]];
         pa32[p] = (float)pa[p];
     }
+    // The damping factors of a pair, 1 - (1 + x) exp(-x) the farther from 1, x = min(a_i,
+    // a_j) r^3 w_i^3 w_j^3 (AMOEBA), round to 1 from x = 42 in FP64 (43 exp(-42) = 2.5e-17)
+    // and from x = 21 in FP32 (1.7e-8); Wang's are 1 from r w_i w_j = 1.  With the
+    // smallest a and w of all sites in the source's place, a bound for every source; a
+    // margin for the rounding of FP32 distances; the site itself is always inside.
+    double wmin = inf, amin = inf;
+    for (int p = 0; p < s.npol; p++) {
+        wmin = std::min(wmin, w[s.polar_mm[p]]);
+        amin = std::min(amin, pa[p]);
+    }
+    std::vector<double> rc(s.npol);
+    std::vector<float> rcf(s.npol);
+    for (int p = 0; p < s.npol; p++) {
+        const double ww = w[s.polar_mm[p]] * wmin;
+        auto cut = [&](double x) {
+            const double r = s.amoeba ? std::cbrt(x / (amin * ww * ww * ww)) : 1.0 / ww;
+            return std::max(r * r * (1.0 + 1e-4), 1e-3);
+        };
+        rc[p] = cut(42.0);
+        rcf[p] = (float)cut(21.0);
+    }
+    upload(rc.data(), d.rc64, sizeof(double) * s.npol);
+    upload(rcf.data(), d.rc32, sizeof(float) * s.npol);
     upload(w.data(), d.mw, sizeof(double) * s.nmm);
     upload(ma.data(), d.ma64, sizeof(double) * s.nmm);
     upload(pa.data(), d.pa64, sizeof(double) * s.npol);
@@ -437,6 +462,8 @@ DeviceState &ensure_device(System &s) {
         d.ps32 = dalloc<float4>(d, s.npol);
         d.pa64 = dalloc<double>(d, s.npol);
         d.pa32 = dalloc<float>(d, s.npol);
+        d.rc64 = dalloc<double>(d, s.npol);
+        d.rc32 = dalloc<float>(d, s.npol);
         d.alpha = dalloc<double>(d, s.npol);
         d.polar_mm = dalloc<int>(d, s.npol);
         d.ms64 = dalloc<double4>(d, s.nmm);
@@ -604,6 +631,7 @@ void ensure_fmm(System &s, DeviceState &d) {
         r.leaf = f.pol_leaf;
         r.pos = f.pol_pos;
         r.a = f.pol_a;
+        r.rc2 = d.rc64;
         auto up = [&](const auto &v) {
             using T = std::decay_t<decltype(v[0])>;
             T *p = fmm_alloc<T>(d, std::max<size_t>(v.size(), 1));
@@ -653,8 +681,8 @@ void ensure_sym(const System &s, DeviceState &d) {
     const int nb = tmv_sym_blocks(s.npol);
     std::vector<int2> pr;
     pr.reserve((size_t)nb * (nb + 1) / 2);
-    for (int I = 0; I < nb; I++)
-        for (int J = I; J < nb; J++) pr.push_back(make_int2(I, J));
+    for (int k = 0; k < nb; k++)  // the diagonal first: they take longest
+        for (int I = 0; I + k < nb; I++) pr.push_back(make_int2(I, I + k));
     d.sym_pairs = dalloc<int2>(d, pr.size());
     upload(pr.data(), d.sym_pairs, sizeof(int2) * pr.size());
     d.sympart = dmalloc(d, tmv_sym_part_bytes(s.npol, 2, 64));
@@ -668,8 +696,7 @@ static int matvec_dot_parts(System &s, DeviceState &d, int kind, int M) {
     }
     const int prec = kind == kOtf32 ? 32 : 64;
     if (kind == kOtf64 || kind == kOtf32)
-        return tmv_pair_once(s.npol, prec, M) ? tmv_sym_dot_parts(s.npol)
-                                                                  : tmv_rows_dot_parts(s.npol, prec, M);
+        return tmv_pair_once(s.npol, M) ? tmv_sym_dot_parts(s.npol) : tmv_rows_dot_parts(s.npol, prec, M);
     return site_blocks(s.npol);
 }
 
@@ -691,14 +718,14 @@ void matvec(System &s, DeviceState &d, int kind, int M, const double *x, double 
         return;
     }
     if (kind == kOtf64 || kind == kOtf32) {
-        const bool sym = tmv_pair_once(s.npol, kind == kOtf32 ? 32 : 64, M);
+        const bool sym = tmv_pair_once(s.npol, M);
         kind = kind == kOtf32 ? (sym ? kSym32 : kPlain32) : (sym ? kSym64 : kPlain64);
     }
     if (kind == kSym64 || kind == kSym32) {
         ensure_sym(s, d);
         const int pi = prof_begin(d, kind == kSym32 ? kOtf32 : kOtf64);
         launch_tmv_sym(d.stream, kind == kSym32 ? 32 : 64, s.amoeba, s.npol, M, d.sym_pairs, d.ps64, d.pa64, d.ps32,
-                       d.pa32, d.alpha, d.pp, x, n, y, n, dodiag, dotpart, d.sympart,
+                       d.pa32, d.rc64, d.rc32, d.alpha, d.pp, x, n, y, n, dodiag, dotpart, d.sympart,
                        reinterpret_cast<const int *>(skip), pi >= 0 ? d.prof_pool[2 * pi] : nullptr,
                        pi >= 0 ? d.prof_pool[2 * pi + 1] : nullptr);
         return;
@@ -706,7 +733,7 @@ void matvec(System &s, DeviceState &d, int kind, int M, const double *x, double 
     if (kind == kPlain64 || kind == kPlain32) {
         const int pi = prof_begin(d, kind == kPlain32 ? kOtf32 : kOtf64);
         launch_tmv_rows(d.stream, kind == kPlain32 ? 32 : 64, s.amoeba, s.npol, M, d.ps64, d.pa64, d.ps32, d.pa32,
-                        d.alpha, d.pp, x, n, y, n, dodiag, dotpart, reinterpret_cast<const int *>(skip),
+                        d.rc64, d.rc32, d.alpha, d.pp, x, n, y, n, dodiag, dotpart, reinterpret_cast<const int *>(skip),
                         pi >= 0 ? d.prof_pool[2 * pi] : nullptr, pi >= 0 ? d.prof_pool[2 * pi + 1] : nullptr);
     } else {
         const int prec = kind == kPack32 ? 32 : 64;
@@ -1111,12 +1138,21 @@ MixedResult mixed_solve(System &s, DeviceState &d, int M, const double *b, doubl
 // the true one; asking for that much (instead of stopping at the tolerance)
 // makes one refinement step enough for most warm-started solves.
 double refine_eta() { return 1e-6; }
+// In the serving loop a solve starts from its predecessor, about 1e6 tolerances away,
+// so that 1e-6 of it ends on either side of the tolerance by the sums' rounding (errors
+// of 2e-9 or 1e-8 in the dipoles); a quarter of it, still above FP32's reach, ends below
+// in one inner solve (all under 5e-9; six systems of 500 to 9,000 sites 17.5 -> 18.0 ms).
+double refine_eta_serving() { return 2.5e-7; }
 // The last inner solve aims well below the tolerance: a CG iteration reduces the
 // residual by ~0.35, so an aim of f tol ends anywhere in 0.35 f tol .. f tol, and
 // with f = 0.25 the result's error does not depend on where the sums' rounding
 // makes it end (with 0.8 the gradient's error moved by 1.6 times between two
 // summation orders); about one inner iteration more.
 double refine_frac() { return 0.25; }
+// A wide batch iterates over all its columns until the last one is done, so that one
+// more iteration costs every column (5% at 15,000 sites and 64 right-hand sides): they
+// stop at the tolerance itself.
+double refine_frac_wide() { return 0.8; }
 
 // ===================================================================== API
 void device_release(System &s) {
@@ -1361,7 +1397,7 @@ size_t device_footprint_estimate(const System &s) {
     b += sizeof(double) * (2 * n * 2 + n + 8 * 2 * n);     // e_m2d, ipd, ext, work vectors
     b += 3 * 24 * sizeof(double) * (n / kBlock + 16) + 2 * sizeof(double) * tmv_rows_dot_parts(s.npol, 64, 2);  // reductions
     b += sizeof(double) * n * 16 + (size_t(4) << 20);      // static-field partials
-    if (tmv_pair_once(s.npol, 64, 1) || rhs_pair_once(s.npol)) {  // block-pair partials and list of the pair-once sweeps
+    if (tmv_pair_once(s.npol, 1) || rhs_pair_once(s.npol)) {  // block-pair partials and list of the pair-once sweeps
         const size_t nb = tmv_sym_blocks(s.npol);
         b += tmv_sym_part_bytes(s.npol, 2, 64) + sizeof(int2) * nb * (nb + 1) / 2;
     }
@@ -1383,6 +1419,8 @@ DeviceView device_view(System &s) {
     v.pa64 = d.pa64;
     v.ps32 = d.ps32;
     v.pa32 = d.pa32;
+    v.rc64 = d.rc64;
+    v.rc32 = d.rc32;
     v.alpha = d.alpha;
     v.pp = d.pp;
     v.e_m2d = d.e_m2d;
@@ -1451,7 +1489,7 @@ void solve_multi(System &s, int nrhs, const double *ext, bool ext_dev, double *i
     long prev = -1;
     const BCol *snap = nullptr;
     for (long t = 0;; t++) {
-        E.tick(refine_eta(), refine_frac());
+        E.tick(refine_eta(), E.m32 == kBatchM32 ? refine_frac_wide() : refine_frac());
         const long seq = E.enqueue_readback();
         if (prev >= 0) {
             snap = E.wait_readback(prev);

@@ -65,6 +65,7 @@ template <typename R> struct FarDev {
     int *leaf_start = nullptr, *order = nullptr, *leaf = nullptr;  // leaf: of every sorted site
     typename std::conditional<sizeof(R) == 8, double4, float4>::type *pos = nullptr;
     R *a = nullptr;
+    const R *rc2 = nullptr;        // damping cutoffs, by polarizable site (row_sweep.h)
     int2 *blocks = nullptr;        // (leaf, first sorted site) of every workgroup of the near field
     R *basis = nullptr;            // [levels - 1][npol][kFarBasis]: B(v / h), degree < p, sorted sites
     R *grad = nullptr;             // [cells][M][3][kFarBasis]: the field's expansion

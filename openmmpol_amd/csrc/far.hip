@@ -27,6 +27,7 @@
 
 #include "far.h"
 #include "pair_math.h"
+#include "row_sweep.h"
 
 namespace ommp {
 
@@ -412,35 +413,13 @@ __global__ __launch_bounds__(kBlock) void k_far_field(FarLevels lv, int p, int n
     }
 }
 
-// v[NT * C] per lane -> lane group k (of 64 / NT lanes) holds the wave's sum of
-// v[k * C .. k * C + C) (as in the per-target matvec).
-template <typename R, int NT, int C> __device__ __forceinline__ void wave_rows(R (&v)[NT * C]) {
-    const int lane = threadIdx.x & 63;
-    int mask = 32;
-#pragma unroll
-    for (int cnt = NT; cnt > 1; cnt >>= 1, mask >>= 1) {
-        const bool hi = lane & mask;
-        const int h = cnt / 2 * C;
-#pragma unroll
-        for (int k = 0; k < NT * C / 2; k++)
-            if (k < h) {
-                const R keep = hi ? v[k + h] : v[k], send = hi ? v[k] : v[k + h];
-                v[k] = keep + __shfl_xor(send, mask, 64);
-            }
-    }
-#pragma unroll
-    for (; mask > 0; mask >>= 1)
-#pragma unroll
-        for (int k = 0; k < C; k++) v[k] += __shfl_xor(v[k], mask, 64);
-}
-
 constexpr int kNearTile = 1024;  // sources listed at once
 
 template <typename R, int M, bool AMOEBA, int T>
 __global__ __launch_bounds__(kBlock) void k_far_near(
     FarLevels lv, int npol, const int2 *__restrict__ blocks, const int *__restrict__ leaf_start,
     const int *__restrict__ order, const typename V4<R>::t *__restrict__ pos, const R *__restrict__ adamp,
-    const R *__restrict__ basis, const R *__restrict__ grad, const double4 *__restrict__ ps,
+    const R *__restrict__ rc2, const R *__restrict__ basis, const R *__restrict__ grad, const double4 *__restrict__ ps,
     const double *__restrict__ pa, const double *__restrict__ alpha, const int *__restrict__ pp_ri,
     const int *__restrict__ pp_ci, const double *__restrict__ pp_f, const double *__restrict__ x, long xstride,
     double *__restrict__ y, long ystride, int dodiag, double *__restrict__ dotpart,
@@ -449,26 +428,18 @@ __global__ __launch_bounds__(kBlock) void k_far_near(
     constexpr int C = 3 * M, W = kBlock / 64;
     if (all_done(skip, M)) return;
     __shared__ int s_src[kNearTile];
-    __shared__ R s_row[W][T][C];
-    __shared__ double s_corr[T][C], s_dot[T][C];
+    __shared__ RowLds<R, M, T> lds;
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int leaf = blocks[blockIdx.x].x, t0 = blocks[blockIdx.x].y;
     const int nl = 1 << lv.levels, lx = leaf & (nl - 1), ly = leaf >> lv.levels & (nl - 1), lz = leaf >> 2 * lv.levels;
     const int nt = min(T, leaf_start[leaf + 1] - t0);
     // targets past the leaf's end repeat the last one; their results are not written
-    R4 pj[T];
-    R aj[T];
+    auto tgt = [&](int t) { return t0 + min(t, nt - 1); };
+    auto id = [&](int i) { return order[i]; };
+    RowAcc<R, M, T> acc;
 #pragma unroll
-    for (int t = 0; t < T; t++) {
-        pj[t] = pos[t0 + min(t, nt - 1)];
-        aj[t] = adamp[t0 + min(t, nt - 1)];
-    }
-    R acc[T][M][3];
-#pragma unroll
-    for (int t = 0; t < T; t++)
-#pragma unroll
-        for (int m = 0; m < M; m++) acc[t][m][0] = acc[t][m][1] = acc[t][m][2] = R(0);
+    for (int t = 0; t < T; t++) row_target(acc, t, pos[tgt(t)], adamp[tgt(t)], rc2[order[tgt(t)]]);
     // far field of level 2 + w (and 6 + w): one basis function per lane
     for (int l = 2 + w; l <= lv.levels; l += W) {
         const int k = lv.levels - l, ns = 1 << l;
@@ -482,7 +453,7 @@ __global__ __launch_bounds__(kBlock) void k_far_near(
         for (int t = 0; t < T; t++) {
             const R bv = b[min(t, nt - 1) * kFarBasis];
 #pragma unroll
-            for (int c = 0; c < C; c++) acc[t][c / 3][c % 3] += bv * gv[c];
+            for (int c = 0; c < C; c++) acc.f[t][c / 3][c % 3] += bv * gv[c];
         }
     }
     // near field: nine runs of sites (three leaves along x each)
@@ -508,12 +479,13 @@ __global__ __launch_bounds__(kBlock) void k_far_near(
         }
         __syncthreads();
         R4 pn, vn[M];
-        R an;
+        R an = R(0);
+        int in = 0;
         auto load = [&](int q) {
-            const int i = s_src[q];
-            pn = pos[i];
-            an = adamp[i];
-            const long j = 3L * order[i];
+            in = s_src[q];
+            pn = pos[in];
+            an = adamp[in];
+            const long j = 3L * order[in];
 #pragma unroll
             for (int m = 0; m < M; m++) {
                 vn[m].x = (R)x[m * xstride + j];
@@ -523,94 +495,19 @@ __global__ __launch_bounds__(kBlock) void k_far_near(
         };
         if (tid < cnt) load(tid);
         for (int q = tid; q < cnt; q += kBlock) {
-            const R4 pi = pn;
-            const R ai = an;
+            const R4 p = pn;
+            const R a = an;
+            const int i = in;
             R4 v[M];
 #pragma unroll
             for (int m = 0; m < M; m++) v[m] = vn[m];
             if (q + kBlock < cnt) load(q + kBlock);  // the next source while this one is used
-#pragma unroll
-            for (int t = 0; t < T; t++) {
-                R dx, dy, dz, k2, k3, arg;
-                bool near;
-                pair_geom<R, AMOEBA>(pj[t], aj[t], pi, ai, dx, dy, dz, k2, k3, arg, near);
-                if (__ballot(near)) pair_damp<R, AMOEBA>(arg, near, k2, k3);
-                pair_accum<R, M>(acc[t], v, dx, dy, dz, k2, k3);
-            }
+            row_source<AMOEBA>(acc, lds, w, i, p, a, v, pos, adamp, tgt);
         }
     }
-    {
-        R flat[T * C];
-#pragma unroll
-        for (int t = 0; t < T; t++)
-#pragma unroll
-            for (int c = 0; c < C; c++) flat[t * C + c] = acc[t][c / 3][c % 3];
-        wave_rows<R, T, C>(flat);
-        constexpr int G = 64 / T;
-        if (lane % G == 0) {
-#pragma unroll
-            for (int c = 0; c < C; c++) s_row[w][lane / G][c] = flat[c];
-        }
-    }
-    // corrections of target t by wave t % W: the listed pairs over its lanes
-    for (int t = w; t < T; t += W) {
-        const int j = order[t0 + min(t, nt - 1)];
-        const int k0 = pp_ri[j], k1 = pp_ri[j + 1];
-        double corr[C];
-#pragma unroll
-        for (int c = 0; c < C; c++) corr[c] = 0.0;
-        if (k0 < k1) {
-            const double4 qj = ps[j];
-            const double bj = pa[j];
-            for (int k = k0 + lane; k < k1; k += 64) {
-                const int i = pp_ci[k];
-                const double f = pp_f[k];
-                const double4 pi = ps[i];
-                const double dx = qj.x - pi.x, dy = qj.y - pi.y, dz = qj.z - pi.z;
-                const double r2 = dx * dx + dy * dy + dz * dz;
-                double k2, k3;
-                dip_kernel<double, AMOEBA>(r2, rsqrt(r2), pi.w, qj.w, pa[i], bj, k2, k3);
-#pragma unroll
-                for (int m = 0; m < M; m++) {
-                    const double *xi = x + m * xstride + 3L * i;
-                    const double c = k3 * (xi[0] * dx + xi[1] * dy + xi[2] * dz);
-                    corr[3 * m + 0] += f * (c * dx - k2 * xi[0]);
-                    corr[3 * m + 1] += f * (c * dy - k2 * xi[1]);
-                    corr[3 * m + 2] += f * (c * dz - k2 * xi[2]);
-                }
-            }
-            wave_rows<double, 1, C>(corr);
-        }
-        if (lane == 0) {
-#pragma unroll
-            for (int c = 0; c < C; c++) s_corr[t][c] = corr[c];
-        }
-    }
-    __syncthreads();
-    if (tid < T * C) {
-        const int t = tid / C, c = tid % C;
-        double out = 0.0;
-        if (t < nt) {
-            const int j = order[t0 + t];
-            R s = s_row[0][t][c];
-#pragma unroll
-            for (int q = 1; q < W; q++) s += s_row[q][t][c];
-            const double xj = x[c / 3 * xstride + 3L * j + c % 3];
-            double v = s_corr[t][c] - (double)s;
-            if (dodiag) v += xj * (1.0 / alpha[j]);
-            y[c / 3 * ystride + 3L * j + c % 3] = v;
-            out = v * xj;
-        }
-        s_dot[t][c] = out;
-    }
-    if (!dotpart) return;
-    __syncthreads();
-    if (tid < M) {
-        double d = 0.0;
-#pragma unroll
-        for (int t = 0; t < T; t++) d += (s_dot[t][3 * tid] + s_dot[t][3 * tid + 1]) + s_dot[t][3 * tid + 2];
-        dotpart[tid * gridDim.x + blockIdx.x] = d;
-    }
+    row_finish<AMOEBA>(acc, lds, w, pos, adamp, x, xstride, ps, pa, pp_ri, pp_ci, pp_f, tgt, id);
+    row_store(lds, nt, alpha, x, xstride, y, ystride, dodiag != 0, dotpart ? dotpart + blockIdx.x : nullptr,
+              (long)gridDim.x, tgt, id);
 }
 
 // The workgroups' y.x partials of column blockIdx.y as kFarDots sums, in a fixed
@@ -663,7 +560,7 @@ void matvec_t(hipStream_t st, const FarDev<R> &f, const int *cnt, const double4 
         HIP_CHECK(hipGetLastError());
     }
     hipLaunchKernelGGL((k_far_near<R, M, AMOEBA, T>), dim3(f.nblocks), dim3(kBlock), 0, st, f.lv, f.npol, f.blocks,
-                       f.leaf_start, f.order, f.pos, f.a, f.basis, f.grad, ps64, pa64, alpha, pp.ri, pp.ci, pp.f, x,
+                       f.leaf_start, f.order, f.pos, f.a, f.rc2, f.basis, f.grad, ps64, pa64, alpha, pp.ri, pp.ci, pp.f, x,
                        xs, y, ys, (int)dodiag, dotpart ? f.dots : nullptr, skip);
     if (dotpart)
         hipLaunchKernelGGL(k_far_dots, dim3(kFarDots, M), dim3(kBlock), 0, st, f.nblocks, f.dots, dotpart, skip, M);

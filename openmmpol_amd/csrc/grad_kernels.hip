@@ -192,6 +192,7 @@ __global__ __launch_bounds__(kSymBlock) void k_gpol_dd_sym(int npol, const int2 
     __shared__ double s_acc[kSymWaves][3][64];
     const int2 pr = pairs[blockIdx.x];
     const int I = pr.x, J = pr.y;
+    const long p = sym_pair_index((npol + kSymBlock - 1) / kSymBlock, I, J);
     const int tid = threadIdx.x, l = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const long n = 3L * npol;
@@ -245,48 +246,48 @@ __global__ __launch_bounds__(kSymBlock) void k_gpol_dd_sym(int npol, const int2 
     };
     double acc[3] = {0.0, 0.0, 0.0};
     __syncthreads();
+    double jown[3] = {0.0, 0.0, 0.0};  // diagonal: the source-side sum of this thread's site
+    const bool diag = I == J;
+    const int phases = diag ? kSymDiagPhases : kSymWaves;
 #pragma unroll 1
-    for (int k = 0; k < kSymWaves; k++) {
-        const bool mirror = I == J && k < w;  // wave-uniform
-        const bool diag = I == J && k == w;
+    for (int ph = 0; ph < phases; ph++) {
+        int k = ph, s0 = 0, ns = 64;
+        if (diag) sym_diag_phase(w, ph, k, s0, ns);
+        const bool half = diag && ph == 0;  // its last step meets every pair twice
         double jacc[3] = {0.0, 0.0, 0.0};
-        if (diag) {
-            // one-sided over the other 63 sites of the sub-tile
-            for (int st = 1; st < 64; st++) {
-                double gx, gy, gz;
-                term(k * 64 + ((l + st) & 63), gx, gy, gz);
-                acc[0] += gx;
-                acc[1] += gy;
-                acc[2] += gz;
-            }
-        } else if (!mirror) {
-            for (int st = 0; st < 64; st++) {
-                double gx, gy, gz;
-                term(k * 64 + ((l + st) & 63), gx, gy, gz);
-                acc[0] += gx;
-                acc[1] += gy;
-                acc[2] += gz;
-                jacc[0] -= gx;
-                jacc[1] -= gy;
-                jacc[2] -= gz;
+        for (int st = s0; st < s0 + ns; st++) {
+            double gx, gy, gz;
+            term(k * 64 + ((l + st) & 63), gx, gy, gz);
+            if (half && st == 32 && l >= 32) gx = gy = gz = 0.0;
+            acc[0] += gx;
+            acc[1] += gy;
+            acc[2] += gz;
+            jacc[0] -= gx;
+            jacc[1] -= gy;
+            jacc[2] -= gz;
 #pragma unroll
-                for (int c = 0; c < 3; c++) jacc[c] = lane_next(jacc[c]);
-            }
+            for (int c = 0; c < 3; c++) jacc[c] = lane_next(jacc[c]);
         }
 #pragma unroll
-        for (int c = 0; c < 3; c++) s_acc[w][c][l] = jacc[c];
+        for (int c = 0; c < 3; c++) s_acc[w][c][(l + s0 + ns) & 63] = jacc[c];
         __syncthreads();
-        if (tid < 3 * 64) {
+        if (diag) {
+#pragma unroll
+            for (int c = 0; c < 3; c++) jown[c] += s_acc[(w - ph) & 3][c][l];
+        } else if (tid < 3 * 64) {
             const int c = tid >> 6, jl = tid & 63;
             double sum = s_acc[0][c][jl];
 #pragma unroll
             for (int q = 1; q < kSymWaves; q++) sum += s_acc[q][c][jl];
-            part_j[((long)blockIdx.x * 3 + c) * kSymBlock + k * 64 + jl] = sum;
+            part_j[(p * 3 + c) * kSymBlock + k * 64 + jl] = sum;
         }
         __syncthreads();
     }
 #pragma unroll
-    for (int c = 0; c < 3; c++) part_i[((long)blockIdx.x * 3 + c) * kSymBlock + tid] = acc[c];
+    for (int c = 0; c < 3; c++) {
+        part_i[(p * 3 + c) * kSymBlock + tid] = acc[c];
+        if (diag) part_j[(p * 3 + c) * kSymBlock + tid] = jown[c];
+    }
 }
 
 // Sum of a site's row (pairs (b, J >= b): target sides) and column (pairs

@@ -131,7 +131,9 @@ int verbosity();
 // engine.cpp
 // Inner-solve target of the mixed refinement: max(eta * outer rms, frac * tol).
 double refine_eta();
+double refine_eta_serving();
 double refine_frac();
+double refine_frac_wide();
 void device_release(System &s);
 void prepare_polelec(System &s);                              // E_M2D on device
 void polarization(System &s, const double *d_field, int solver, int matv, int mask);

@@ -132,6 +132,20 @@ __device__ __forceinline__ void pair_geom(const typename V4<R>::t &pj, R aj, con
     }
 }
 
+// The undamped kernels of one pair; returns r2 (0: the kernels are not finite).
+template <typename R>
+__device__ __forceinline__ R pair_bare(const typename V4<R>::t &pj, const typename V4<R>::t &pi, R &dx, R &dy, R &dz,
+                                       R &k2, R &k3) {
+    dx = pj.x - pi.x;
+    dy = pj.y - pi.y;
+    dz = pj.z - pi.z;
+    const R r2 = fmaa(dz, dz, fmaa(dy, dy, dx * dx));
+    const R ir = fast_rsqrt(r2), ir2 = ir * ir;
+    k2 = ir * ir2;
+    k3 = (R(3) * k2) * ir2;
+    return r2;
+}
+
 template <typename R, bool AMOEBA>
 __device__ __forceinline__ void pair_damp(R arg, bool near, R &k2, R &k3) {
     if (AMOEBA) {

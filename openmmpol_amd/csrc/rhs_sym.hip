@@ -109,6 +109,7 @@ __global__ __launch_bounds__(kSymBlock) void k_rhs_sym(int npol, const int2 *__r
     __shared__ double s_acc[kSymWaves][3][64];
     const int2 pr = pairs[blockIdx.x];
     const int I = pr.x, J = pr.y;
+    const long p = sym_pair_index((npol + kSymBlock - 1) / kSymBlock, I, J);
     const int tid = threadIdx.x, l = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const double far = 1e15, gap = 1e9;
@@ -162,53 +163,51 @@ __global__ __launch_bounds__(kSymBlock) void k_rhs_sym(int npol, const int2 *__r
     };
     double acc[3] = {0.0, 0.0, 0.0};
     __syncthreads();
+    double jown[3] = {0.0, 0.0, 0.0};  // diagonal: the source-side sum of this thread's site
+    const bool diag = I == J;
+    const int phases = diag ? kSymDiagPhases : kSymWaves;
 #pragma unroll 1
-    for (int k = 0; k < kSymWaves; k++) {
-        const bool mirror = I == J && k < w;  // wave-uniform
-        const bool diag = I == J && k == w;
+    for (int ph = 0; ph < phases; ph++) {
+        int k = ph, s0 = 0, n = 64;
+        if (diag) sym_diag_phase(w, ph, k, s0, n);
+        const bool half = diag && ph == 0;  // its last step meets every pair twice
         double jacc[3] = {0.0, 0.0, 0.0};
-        if (diag) {
-            // one-sided over the other 63 sites of the sub-tile
-            for (int s = 1; s < 64; s++) {
-                const int js = k * 64 + ((l + s) & 63);
-                double4 psrc;
-                double q[2 * NQ];
-                load_src(js, psrc, q);
-                double dx, dy, dz, k2, k3, k4;
-                rhs_geom<AMOEBA>(pt, at, psrc, q[KA], dx, dy, dz, k2, k3, k4);
-                rhs_accum<AMOEBA>(q, dx, dy, dz, k2, 3.0 * k3, 6.0 * k3, 15.0 * k4, acc);
-            }
-        } else if (!mirror) {
-            for (int s = 0; s < 64; s++) {
-                const int js = k * 64 + ((l + s) & 63);
-                double4 psrc;
-                double q[2 * NQ];
-                load_src(js, psrc, q);
-                double dx, dy, dz, k2, k3, k4;
-                rhs_geom<AMOEBA>(pt, at, psrc, q[KA], dx, dy, dz, k2, k3, k4);
-                const double k3t = 3.0 * k3, k3s = 6.0 * k3, k4f = 15.0 * k4;
-                rhs_accum<AMOEBA>(q, dx, dy, dz, k2, k3t, k3s, k4f, acc);
-                // the field at the source of this lane's target, d reversed
-                rhs_accum<AMOEBA>(qt, -dx, -dy, -dz, k2, k3t, k3s, k4f, jacc);
+        for (int s = s0; s < s0 + n; s++) {
+            const int js = k * 64 + ((l + s) & 63);
+            double4 psrc;
+            double q[2 * NQ];
+            load_src(js, psrc, q);
+            double dx, dy, dz, k2, k3, k4;
+            rhs_geom<AMOEBA>(pt, at, psrc, q[KA], dx, dy, dz, k2, k3, k4);
+            if (half && s == 32 && l >= 32) k2 = k3 = k4 = 0.0;
+            const double k3t = 3.0 * k3, k3s = 6.0 * k3, k4f = 15.0 * k4;
+            rhs_accum<AMOEBA>(q, dx, dy, dz, k2, k3t, k3s, k4f, acc);
+            // the field at the source of this lane's target, d reversed
+            rhs_accum<AMOEBA>(qt, -dx, -dy, -dz, k2, k3t, k3s, k4f, jacc);
 #pragma unroll
-                for (int c = 0; c < 3; c++) jacc[c] = lane_next(jacc[c]);
-            }
+            for (int c = 0; c < 3; c++) jacc[c] = lane_next(jacc[c]);
         }
 #pragma unroll
-        for (int c = 0; c < 3; c++) s_acc[w][c][l] = jacc[c];
+        for (int c = 0; c < 3; c++) s_acc[w][c][(l + s0 + n) & 63] = jacc[c];
         __syncthreads();
-        // source side of sub-tile k: the waves' rows added in wave order
-        if (tid < 3 * 64) {
+        if (diag) {
+#pragma unroll
+            for (int c = 0; c < 3; c++) jown[c] += s_acc[(w - ph) & 3][c][l];
+        } else if (tid < 3 * 64) {
+            // source side of sub-tile k: the waves' rows added in wave order
             const int c = tid >> 6, jl = tid & 63;
             double sum = s_acc[0][c][jl];
 #pragma unroll
             for (int q = 1; q < kSymWaves; q++) sum += s_acc[q][c][jl];
-            part_j[((long)blockIdx.x * 3 + c) * kSymBlock + k * 64 + jl] = sum;
+            part_j[(p * 3 + c) * kSymBlock + k * 64 + jl] = sum;
         }
         __syncthreads();
     }
 #pragma unroll
-    for (int c = 0; c < 3; c++) part_i[((long)blockIdx.x * 3 + c) * kSymBlock + tid] = acc[c];
+    for (int c = 0; c < 3; c++) {
+        part_i[(p * 3 + c) * kSymBlock + tid] = acc[c];
+        if (diag) part_j[(p * 3 + c) * kSymBlock + tid] = jown[c];
+    }
 }
 
 // E_M2D of 64 sites per workgroup (kRhsSub workgroups per block of kSymBlock):

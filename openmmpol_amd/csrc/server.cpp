@@ -523,7 +523,7 @@ class Server {
                 continue;
             }
             lk.unlock();
-            L.engine->tick(refine_eta(), refine_frac());
+            L.engine->tick(refine_eta_serving(), refine_frac());
             const long seq = L.engine->enqueue_readback();
             int live = 0;
             if (prev >= 0) {

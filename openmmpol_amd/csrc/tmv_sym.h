@@ -12,10 +12,22 @@
 // Every sum has a fixed order (results bitwise reproducible).  Measured
 // alternatives for the source side, both slower: LDS float atomics into a
 // per-wave row (FP32 ones were 14x slower here) and lane shuffles through the
-// LDS crossbar.  In a diagonal block pair (I = J) the sub-tile pairs k < w are
-// the mirror images of pairs handled by wave k and are skipped, and the
-// diagonal sub-tile (k = w) is swept one-sided over s = 1..63.  Scale 1 for every
-// pair (the finalize kernels apply the screening corrections), self excluded.
+// LDS crossbar.  Scale 1 for every pair (the finalize kernels apply the screening
+// corrections), self excluded.
+//
+// A diagonal block pair (I = J) has its ten sub-tile pairs spread evenly: wave w
+// sweeps sub-tile w against itself over s = 1..32 (at s = 32 lanes 0..31 alone),
+// against w + 1 over all 64 steps and against w + 2 over the half that wave w + 2
+// does not (indices mod 4): 128 steps, as many as off the diagonal.  Skipping the
+// mirror images (k < w) instead gave wave 0 255 steps, nearly all of them with
+// damped pairs, one long dependent chain each: at 8,000 sites of a chain in FP64 it
+// took 120 of the sweep's 122 us.
+//
+// Bound by the vector unit's issue (56 instructions per pair, FP64 one column, at
+// 60,000 sites).  us per sweep, before these diagonals and the cutoffs of pair_damp_v
+// and now: FP64 one / two columns at 8,000 sites 123 / 151 and 86 / 113, at 15,000 253 /
+// 310 and 190 / 278, at 60,000 2890 / 4200 and 2590 / 3920; FP32 two columns at 15,000
+// 166 and 152, at 60,000 2190 and 2030.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -26,6 +38,20 @@
 namespace ommp {
 
 constexpr int kSymWaves = kSymBlock / 64;
+
+// Index of block pair (I <= J) of nb blocks in the partial sums (the order in which
+// the pairs are dispatched is another: the diagonal ones first).
+__device__ __forceinline__ long sym_pair_index(int nb, int I, int J) {
+    return (long)I * nb - (long)I * (I - 1) / 2 + J - I;
+}
+
+// Steps [s, s + n) and sub-tile k of wave w in phase ph of a diagonal block pair.
+constexpr int kSymDiagPhases = 3;
+__device__ __forceinline__ void sym_diag_phase(int w, int ph, int &k, int &s, int &n) {
+    k = (w + ph) & 3;
+    s = ph == 0 || (ph == 2 && w >= 2) ? 1 : 0;
+    n = ph == 1 ? 64 : 32;
+}
 
 // Lane l + 1's value at lane l (wave rotate by one lane, DPP).
 __device__ __forceinline__ float lane_next(float v) {
@@ -45,27 +71,24 @@ constexpr int sym_lds_bytes() {
     return (int)(sizeof(typename V4<R>::t) * kSymBlock * (1 + M) + sizeof(R) * kSymWaves * M * 3 * 64);
 }
 
-// Pair geometry with the AMOEBA damping argument from cubed polarizability
-// factors (vi = w_i^3, vj = w_j^3): a u^3 = a r^3 w_i^3 w_j^3 with one multiply
-// fewer than cubing u = r w_i w_j.  Wang (AMBER) damping keeps u itself.
+// Damps the kernels of a pair of distinct sites at distance^2 r2 (pair_bare) where
+// its argument says so.  Beyond the target's cutoff rc2 (row_sweep.h) no pair is
+// damped, so that callers decide by one compare per pair and come here only where a
+// lane of the wave is inside.  AMOEBA: w holds w^3 (vi vj r^3 = u^3).
 template <typename R, bool AMOEBA>
-__device__ __forceinline__ void pair_geom_v(const typename V4<R>::t &pj, R aj, const typename V4<R>::t &pi, R ai,
-                                            R &dx, R &dy, R &dz, R &k2, R &k3, R &arg, bool &near) {
-    if (!AMOEBA) {
-        pair_geom<R, AMOEBA, false>(pj, aj, pi, ai, dx, dy, dz, k2, k3, arg, near);
-        return;
+__device__ __forceinline__ void pair_damp_v(const typename V4<R>::t &pj, R aj, const typename V4<R>::t &pi, R ai,
+                                            R r2, R &k2, R &k3) {
+    const R r = r2 * fast_rsqrt(r2);
+    R arg;
+    bool near;
+    if (AMOEBA) {
+        arg = pos_min(ai, aj) * ((r * r2) * (pi.w * pj.w));
+        near = arg < R(50);
+    } else {
+        arg = r * (pi.w * pj.w);
+        near = arg < R(1);
     }
-    dx = pj.x - pi.x;
-    dy = pj.y - pi.y;
-    dz = pj.z - pi.z;
-    const R r2 = fmaa(dz, dz, fmaa(dy, dy, dx * dx));
-    const R ir = fast_rsqrt(r2);
-    const R ir2 = ir * ir;
-    k2 = ir * ir2;
-    k3 = (R(3) * k2) * ir2;
-    const R r3 = (r2 * ir) * r2;
-    arg = pos_min(ai, aj) * (r3 * (pi.w * pj.w));
-    near = arg < R(50);
+    pair_damp<R, AMOEBA>(arg, near, k2, k3);
 }
 
 // Both directions' accumulation of one pair: E_i += k3 (x_j.d) d - k2 x_j at the
@@ -87,6 +110,102 @@ __device__ __forceinline__ void pair_accum2(R (&acc)[M][3], R *jacc, const typen
     }
 }
 
+// Sources of a block pair: the sites of J to LDS.  Padding sites (past npol, in the
+// last block only) sit far away at distinct points with zero dipoles, so that no pair
+// but the skipped self pair has a zero distance.
+template <typename R, int M, bool AMOEBA>
+__device__ __forceinline__ void sym_sources(int npol, int J, const typename V4<R>::t *__restrict__ site,
+                                            const R *__restrict__ adamp, const double *const (&xcol)[M],
+                                            typename V4<R>::t *s_pos, typename V4<R>::t (*s_x)[kSymBlock]) {
+    const R far = R(1e15), gap = R(1e9);
+    const int tid = threadIdx.x, jj = J * kSymBlock + tid;
+    typename V4<R>::t p, v[M];
+    if (jj < npol) {
+        p = site[jj];
+        if (AMOEBA) p.w = p.w * p.w * p.w;  // w^3 (pair_damp_v)
+#pragma unroll
+        for (int m = 0; m < M; m++) {
+            v[m].x = (R)xcol[m][3L * jj + 0];
+            v[m].y = (R)xcol[m][3L * jj + 1];
+            v[m].z = (R)xcol[m][3L * jj + 2];
+            v[m].w = m == 0 ? adamp[jj] : R(0);
+        }
+    } else {
+        p.x = p.y = p.z = far + gap * (R)tid;
+        p.w = R(1);
+#pragma unroll
+        for (int m = 0; m < M; m++) {
+            v[m].x = v[m].y = v[m].z = R(0);
+            v[m].w = R(0.39);
+        }
+    }
+    s_pos[tid] = p;
+#pragma unroll
+    for (int m = 0; m < M; m++) s_x[m][tid] = v[m];
+}
+
+// Target li of block I: position (w^3 for AMOEBA), damping, cutoff, dipoles.
+template <typename R, int M, bool AMOEBA>
+__device__ __forceinline__ void sym_target(int npol, int I, int li, const typename V4<R>::t *__restrict__ site,
+                                           const R *__restrict__ adamp, const R *__restrict__ rc2,
+                                           const double *const (&xcol)[M], typename V4<R>::t &p, R &a, R &rc,
+                                           R (&x)[M][3]) {
+    const R far = R(1e15), gap = R(1e9);
+    const int i = I * kSymBlock + li;
+    if (i < npol) {
+        p = site[i];
+        if (AMOEBA) p.w = p.w * p.w * p.w;
+        a = adamp[i];
+        rc = rc2[i];
+#pragma unroll
+        for (int m = 0; m < M; m++)
+#pragma unroll
+            for (int c = 0; c < 3; c++) x[m][c] = (R)xcol[m][3L * i + c];
+    } else {
+        p.x = p.y = p.z = far + gap * (R)li;
+        p.w = R(1);
+        a = R(0.39);
+        rc = R(0);
+#pragma unroll
+        for (int m = 0; m < M; m++) x[m][0] = x[m][1] = x[m][2] = R(0);
+    }
+}
+
+// One wave's sweep of sub-tile k (its sources at pos_k, x_k) over steps s .. s + n - 1
+// (n even), two sources at a time: their two dependent chains keep a lone wave busy.
+// jacc ends at the sum of source (l + s + n) & 63.  half: the last step is the one
+// that meets every pair twice; lanes 0..31 keep theirs.
+template <typename R, int M, bool AMOEBA>
+__device__ __forceinline__ void sym_sweep(int s, int n, bool half, const typename V4<R>::t &pj, R aj, R rj,
+                                          const R (&xi)[M][3], const typename V4<R>::t *pos_k,
+                                          const typename V4<R>::t *x_k, R (&acc)[M][3], R (&jacc)[M * 3]) {
+    using R4 = typename V4<R>::t;
+    const int l = threadIdx.x & 63, end = s + n;
+    for (; s < end; s += 2) {
+        R4 xv[2][M], ps[2];
+        R dx[2], dy[2], dz[2], k2[2], k3[2], r2[2];
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const int js = (l + s + u) & 63;
+#pragma unroll
+            for (int m = 0; m < M; m++) xv[u][m] = x_k[m * kSymBlock + js];
+            ps[u] = pos_k[js];
+            r2[u] = pair_bare<R>(pj, ps[u], dx[u], dy[u], dz[u], k2[u], k3[u]);
+        }
+        if (__ballot(r2[0] < rj || r2[1] < rj)) {
+#pragma unroll
+            for (int u = 0; u < 2; u++) pair_damp_v<R, AMOEBA>(pj, aj, ps[u], xv[u][0].w, r2[u], k2[u], k3[u]);
+        }
+        if (half && s + 2 == end && l >= 32) k2[1] = k3[1] = R(0);
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            pair_accum2<R, M>(acc, jacc, xv[u], xi, dx[u], dy[u], dz[u], k2[u], k3[u]);
+#pragma unroll
+            for (int c = 0; c < M * 3; c++) jacc[c] = lane_next(jacc[c]);
+        }
+    }
+}
+
 // Pair (I, J) of blocks with a kSymBlock-thread workgroup: xcol[m] = column m's
 // dipoles [npol][3] (FP64); the target-side sums of component c of column m go
 // to out_i[m][c * kSymBlock + t] (t = the site's index in I), the source-side
@@ -95,128 +214,59 @@ __device__ __forceinline__ void pair_accum2(R (&acc)[M][3], R *jacc, const typen
 // one kernel share it); the body ends with a workgroup barrier.
 template <typename R, int M, bool AMOEBA>
 __device__ __forceinline__ void sym_block_pair(int npol, int I, int J, const typename V4<R>::t *__restrict__ site,
-                                               const R *__restrict__ adamp, const double *const (&xcol)[M],
-                                               R *const (&out_i)[M], R *const (&out_j)[M], char *lds) {
+                                               const R *__restrict__ adamp, const R *__restrict__ rc2,
+                                               const double *const (&xcol)[M], R *const (&out_i)[M],
+                                               R *const (&out_j)[M], char *lds) {
     using R4 = typename V4<R>::t;
     R4 *s_pos = reinterpret_cast<R4 *>(lds);
     R4(*s_x)[kSymBlock] = reinterpret_cast<R4(*)[kSymBlock]>(s_pos + kSymBlock);  // x, y, z; w of column 0: a
     R(*s_acc)[M * 3][64] = reinterpret_cast<R(*)[M * 3][64]>(s_x + M);
     const int tid = threadIdx.x, l = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave index, uniform
-    // Padding sites (past npol, in the last block only) sit far away at distinct
-    // points with zero dipoles, so that no pair but the skipped self pair has a
-    // zero distance.
-    const R far = R(1e15), gap = R(1e9);
-    // sources: the sites of J
-    {
-        const int jj = J * kSymBlock + tid;
-        R4 p, v[M];
-        if (jj < npol) {
-            p = site[jj];
-            if (AMOEBA) p.w = p.w * p.w * p.w;  // w^3 (pair_geom_v)
-#pragma unroll
-            for (int m = 0; m < M; m++) {
-                v[m].x = (R)xcol[m][3L * jj + 0];
-                v[m].y = (R)xcol[m][3L * jj + 1];
-                v[m].z = (R)xcol[m][3L * jj + 2];
-                v[m].w = m == 0 ? adamp[jj] : R(0);
-            }
-        } else {
-            p.x = p.y = p.z = far + gap * (R)tid;
-            p.w = R(1);
-#pragma unroll
-            for (int m = 0; m < M; m++) {
-                v[m].x = v[m].y = v[m].z = R(0);
-                v[m].w = R(0.39);
-            }
-        }
-        s_pos[tid] = p;
-#pragma unroll
-        for (int m = 0; m < M; m++) s_x[m][tid] = v[m];
-    }
-    // targets: this thread's site of I
-    const int i = I * kSymBlock + tid;
+    sym_sources<R, M, AMOEBA>(npol, J, site, adamp, xcol, s_pos, s_x);
     R4 pj;
-    R aj, xi[M][3];
-    if (i < npol) {
-        pj = site[i];
-        if (AMOEBA) pj.w = pj.w * pj.w * pj.w;
-        aj = adamp[i];
-#pragma unroll
-        for (int m = 0; m < M; m++)
-#pragma unroll
-            for (int c = 0; c < 3; c++) xi[m][c] = (R)xcol[m][3L * i + c];
-    } else {
-        pj.x = pj.y = pj.z = far + gap * (R)tid;
-        pj.w = R(1);
-        aj = R(0.39);
-#pragma unroll
-        for (int m = 0; m < M; m++) xi[m][0] = xi[m][1] = xi[m][2] = R(0);
-    }
-    R acc[M][3];
+    R aj, rj, xi[M][3], acc[M][3];
+    sym_target<R, M, AMOEBA>(npol, I, tid, site, adamp, rc2, xcol, pj, aj, rj, xi);
 #pragma unroll
     for (int m = 0; m < M; m++) acc[m][0] = acc[m][1] = acc[m][2] = R(0);
     __syncthreads();
+    const bool diag = I == J;
+    R jown[M * 3];  // diagonal: the source-side sum of this thread's site
 #pragma unroll
-    for (int k = 0; k < kSymWaves; k++) {
-        const bool mirror = I == J && k < w;  // wave-uniform
-        const bool diag = I == J && k == w;
+    for (int c = 0; c < M * 3; c++) jown[c] = R(0);
+    const int phases = diag ? kSymDiagPhases : kSymWaves;
+    for (int ph = 0; ph < phases; ph++) {
+        int k = ph, s = 0, n = 64;
+        if (diag) sym_diag_phase(w, ph, k, s, n);
         R jacc[M * 3];
 #pragma unroll
         for (int c = 0; c < M * 3; c++) jacc[c] = R(0);
-        if (diag) {
-            // one-sided over the other 63 sites of the sub-tile
-            for (int s = 1; s < 64; s++) {
-                const int js = k * 64 + ((l + s) & 63);
-                R4 xv[M];
+        sym_sweep<R, M, AMOEBA>(s, n, diag && ph == 0, pj, aj, rj, xi, s_pos + k * 64, &s_x[0][k * 64], acc, jacc);
 #pragma unroll
-                for (int m = 0; m < M; m++) xv[m] = s_x[m][js];
-                R dx, dy, dz, k2, k3, arg;
-                bool near;
-                pair_geom_v<R, AMOEBA>(pj, aj, s_pos[js], xv[0].w, dx, dy, dz, k2, k3, arg, near);
-                if (__ballot(near)) pair_damp<R, AMOEBA>(arg, near, k2, k3);
-                pair_accum<R, M>(acc, xv, dx, dy, dz, k2, k3);
-            }
-        } else if (!mirror) {
-            // byte offset of the current source within the sub-tile (one add
-            // and one mask per step)
-            constexpr int kRow = 64 * (int)sizeof(R4);
-            const char *pos_k = reinterpret_cast<const char *>(s_pos + k * 64);
-            const char *x_k = reinterpret_cast<const char *>(&s_x[0][k * 64]);
-            int jo = l * (int)sizeof(R4);
-            for (int s = 0; s < 64; s++) {
-                R4 xv[M];
-#pragma unroll
-                for (int m = 0; m < M; m++)
-                    xv[m] = *reinterpret_cast<const R4 *>(x_k + m * kSymBlock * (int)sizeof(R4) + jo);
-                const R4 ps = *reinterpret_cast<const R4 *>(pos_k + jo);
-                R dx, dy, dz, k2, k3, arg;
-                bool near;
-                pair_geom_v<R, AMOEBA>(pj, aj, ps, xv[0].w, dx, dy, dz, k2, k3, arg, near);
-                if (__ballot(near)) pair_damp<R, AMOEBA>(arg, near, k2, k3);
-                pair_accum2<R, M>(acc, jacc, xv, xi, dx, dy, dz, k2, k3);
-#pragma unroll
-                for (int c = 0; c < M * 3; c++) jacc[c] = lane_next(jacc[c]);
-                jo = (jo + (int)sizeof(R4)) & (kRow - 1);
-            }
-        }
-#pragma unroll
-        for (int c = 0; c < M * 3; c++) s_acc[w][c][l] = jacc[c];
+        for (int c = 0; c < M * 3; c++) s_acc[w][c][(l + s + n) & 63] = jacc[c];
         __syncthreads();
-        // source side of sub-tile k: the waves' rows added in wave order
-        for (int e = tid; e < M * 3 * 64; e += kSymBlock) {
-            const int c = e >> 6, jl = e & 63;
-            R sum = s_acc[0][c][jl];
+        if (diag) {
 #pragma unroll
-            for (int q = 1; q < kSymWaves; q++) sum += s_acc[q][c][jl];
-            out_j[c / 3][(c % 3) * kSymBlock + k * 64 + jl] = sum;
+            for (int c = 0; c < M * 3; c++) jown[c] += s_acc[(w - ph) & 3][c][l];
+        } else {
+            // source side of sub-tile k: the waves' rows added in wave order
+            for (int e = tid; e < M * 3 * 64; e += kSymBlock) {
+                const int c = e >> 6, jl = e & 63;
+                R sum = s_acc[0][c][jl];
+#pragma unroll
+                for (int q = 1; q < kSymWaves; q++) sum += s_acc[q][c][jl];
+                out_j[c / 3][(c % 3) * kSymBlock + k * 64 + jl] = sum;
+            }
         }
         __syncthreads();
     }
 #pragma unroll
     for (int m = 0; m < M; m++)
 #pragma unroll
-        for (int c = 0; c < 3; c++) out_i[m][c * kSymBlock + tid] = acc[m][c];
+        for (int c = 0; c < 3; c++) {
+            out_i[m][c * kSymBlock + tid] = acc[m][c];
+            if (diag) out_j[m][c * kSymBlock + tid] = jown[3 * m + c];
+        }
 }
 
 // Off-diagonal block pair (I < J) with two targets per lane: wave w holds the
@@ -228,7 +278,8 @@ __device__ __forceinline__ void sym_block_pair(int npol, int I, int J, const typ
 // LDS and outputs as sym_block_pair.
 template <typename R, int M, bool AMOEBA>
 __device__ __forceinline__ void sym_block_pair2(int npol, int I, int J, const typename V4<R>::t *__restrict__ site,
-                                                const R *__restrict__ adamp, const double *const (&xcol)[M],
+                                                const R *__restrict__ adamp, const R *__restrict__ rc2,
+                                               const double *const (&xcol)[M],
                                                 R *const (&out_i)[M], R *const (&out_j)[M], char *lds) {
     using R4 = typename V4<R>::t;
     static_assert(kSymWaves == 4, "two target and two source halves");
@@ -239,55 +290,13 @@ __device__ __forceinline__ void sym_block_pair2(int npol, int I, int J, const ty
     const int tid = threadIdx.x, l = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int th = w & 1, sh = w >> 1;
-    const R far = R(1e15), gap = R(1e9);
-    {
-        const int jj = J * kSymBlock + tid;
-        R4 p, v[M];
-        if (jj < npol) {
-            p = site[jj];
-            if (AMOEBA) p.w = p.w * p.w * p.w;  // w^3 (pair_geom_v)
-#pragma unroll
-            for (int m = 0; m < M; m++) {
-                v[m].x = (R)xcol[m][3L * jj + 0];
-                v[m].y = (R)xcol[m][3L * jj + 1];
-                v[m].z = (R)xcol[m][3L * jj + 2];
-                v[m].w = m == 0 ? adamp[jj] : R(0);
-            }
-        } else {
-            p.x = p.y = p.z = far + gap * (R)tid;
-            p.w = R(1);
-#pragma unroll
-            for (int m = 0; m < M; m++) {
-                v[m].x = v[m].y = v[m].z = R(0);
-                v[m].w = R(0.39);
-            }
-        }
-        s_pos[tid] = p;
-#pragma unroll
-        for (int m = 0; m < M; m++) s_x[m][tid] = v[m];
-    }
+    sym_sources<R, M, AMOEBA>(npol, J, site, adamp, xcol, s_pos, s_x);
     // targets: sites 128 th + l and 128 th + 64 + l of I
     R4 pt[2];
-    R at[2], xt[2][M][3];
+    R at[2], rt[2], xt[2][M][3];
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
-        const int li = 128 * th + 64 * h + l, i = I * kSymBlock + li;
-        if (i < npol) {
-            pt[h] = site[i];
-            if (AMOEBA) pt[h].w = pt[h].w * pt[h].w * pt[h].w;
-            at[h] = adamp[i];
-#pragma unroll
-            for (int m = 0; m < M; m++)
-#pragma unroll
-                for (int c = 0; c < 3; c++) xt[h][m][c] = (R)xcol[m][3L * i + c];
-        } else {
-            pt[h].x = pt[h].y = pt[h].z = far + gap * (R)li;
-            pt[h].w = R(1);
-            at[h] = R(0.39);
-#pragma unroll
-            for (int m = 0; m < M; m++) xt[h][m][0] = xt[h][m][1] = xt[h][m][2] = R(0);
-        }
-    }
+    for (int h = 0; h < 2; h++)
+        sym_target<R, M, AMOEBA>(npol, I, 128 * th + 64 * h + l, site, adamp, rc2, xcol, pt[h], at[h], rt[h], xt[h]);
     R acc[2][M][3];
 #pragma unroll
     for (int h = 0; h < 2; h++)
@@ -310,14 +319,17 @@ __device__ __forceinline__ void sym_block_pair2(int npol, int I, int J, const ty
             for (int m = 0; m < M; m++)
                 xv[m] = *reinterpret_cast<const R4 *>(x_k + m * kSymBlock * (int)sizeof(R4) + jo);
             const R4 ps = *reinterpret_cast<const R4 *>(pos_k + jo);
+            // both targets' kernels before the branch: two chains for the few waves
+            R dx[2], dy[2], dz[2], k2[2], k3[2], r2[2];
 #pragma unroll
-            for (int h = 0; h < 2; h++) {
-                R dx, dy, dz, k2, k3, arg;
-                bool near;
-                pair_geom_v<R, AMOEBA>(pt[h], at[h], ps, xv[0].w, dx, dy, dz, k2, k3, arg, near);
-                if (__ballot(near)) pair_damp<R, AMOEBA>(arg, near, k2, k3);
-                pair_accum2<R, M>(acc[h], jacc, xv, xt[h], dx, dy, dz, k2, k3);
-            }
+            for (int h = 0; h < 2; h++) r2[h] = pair_bare<R>(pt[h], ps, dx[h], dy[h], dz[h], k2[h], k3[h]);
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+                if (__ballot(r2[h] < rt[h]))
+                    pair_damp_v<R, AMOEBA>(pt[h], at[h], ps, xv[0].w, r2[h], k2[h], k3[h]);
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+                pair_accum2<R, M>(acc[h], jacc, xv, xt[h], dx[h], dy[h], dz[h], k2[h], k3[h]);
 #pragma unroll
             for (int c = 0; c < M * 3; c++) jacc[c] = lane_next(jacc[c]);
             jo = (jo + (int)sizeof(R4)) & (kRow - 1);
@@ -363,15 +375,16 @@ constexpr bool kSymTwoTargets = sizeof(R) == 4 || M <= 2;
 // the width allows it, one otherwise.
 template <typename R, int M, bool AMOEBA>
 __device__ __forceinline__ void sym_block_pair_any(int npol, int I, int J, const typename V4<R>::t *__restrict__ site,
-                                                   const R *__restrict__ adamp, const double *const (&xcol)[M],
+                                                   const R *__restrict__ adamp, const R *__restrict__ rc2,
+                                               const double *const (&xcol)[M],
                                                    R *const (&out_i)[M], R *const (&out_j)[M], char *lds) {
     if constexpr (kSymTwoTargets<R, M>) {
         if (I != J) {
-            sym_block_pair2<R, M, AMOEBA>(npol, I, J, site, adamp, xcol, out_i, out_j, lds);
+            sym_block_pair2<R, M, AMOEBA>(npol, I, J, site, adamp, rc2, xcol, out_i, out_j, lds);
             return;
         }
     }
-    sym_block_pair<R, M, AMOEBA>(npol, I, J, site, adamp, xcol, out_i, out_j, lds);
+    sym_block_pair<R, M, AMOEBA>(npol, I, J, site, adamp, rc2, xcol, out_i, out_j, lds);
 }
 
 }  // namespace ommp

@@ -1,10 +1,10 @@
 // T matvec on the fly with each unordered pair evaluated once (T_ij = T_ji):
 // the geometry and damping of a pair (half of the per-pair work) are shared by
 // its two directions.  One workgroup per pair of 256-site blocks (I <= J),
-// row-major over the upper triangle (pairs[] lists them); the body is
-// sym_block_pair (tmv_sym.h).
+// listed in pairs[] by distance from the diagonal (the diagonal ones, with the most
+// damped pairs, take longest and start first); the body is sym_block_pair (tmv_sym.h).
 //
-// Outputs, per block pair p: target side part_i[p][M * 3][256] (sites of I) and
+// Outputs, per block pair p (row-major over the upper triangle): target side part_i[p][M * 3][256] (sites of I) and
 // source side part_j[p][M * 3][256] (sites of J); k_tmv_sym_finalize adds, for
 // every site, the nb + 1 partials of its row and column in a fixed order.
 #include <hip/hip_runtime.h>
@@ -24,7 +24,8 @@ static_assert(kSymBlock == kBlock, "pair-once blocks are the blocks of the per-s
 template <typename R, int M, bool AMOEBA>
 __global__ __launch_bounds__(kSymBlock) void k_tmv_sym(int npol, const int2 *__restrict__ pairs,
                                                        const typename V4<R>::t *__restrict__ site,
-                                                       const R *__restrict__ adamp, const double *__restrict__ x,
+                                                       const R *__restrict__ adamp, const R *__restrict__ rc2,
+                                                       const double *__restrict__ x,
                                                        long xstride, R *__restrict__ part_i, R *__restrict__ part_j,
                                                        const CgState *__restrict__ skip, int skipM) {
     if (skip) {
@@ -34,15 +35,16 @@ __global__ __launch_bounds__(kSymBlock) void k_tmv_sym(int npol, const int2 *__r
     }
     __shared__ __align__(16) char lds[sym_lds_bytes<R, M>()];
     const int2 pr = pairs[blockIdx.x];
+    const long p = sym_pair_index((npol + kSymBlock - 1) / kSymBlock, pr.x, pr.y);
     const double *xcol[M];
     R *oi[M], *oj[M];
 #pragma unroll
     for (int m = 0; m < M; m++) {
         xcol[m] = x + m * xstride;
-        oi[m] = part_i + ((long)blockIdx.x * M * 3 + 3 * m) * kSymBlock;
-        oj[m] = part_j + ((long)blockIdx.x * M * 3 + 3 * m) * kSymBlock;
+        oi[m] = part_i + (p * M * 3 + 3 * m) * kSymBlock;
+        oj[m] = part_j + (p * M * 3 + 3 * m) * kSymBlock;
     }
-    sym_block_pair_any<R, M, AMOEBA>(npol, pr.x, pr.y, site, adamp, xcol, oi, oj, lds);
+    sym_block_pair_any<R, M, AMOEBA>(npol, pr.x, pr.y, site, adamp, rc2, xcol, oi, oj, lds);
 }
 
 // y = -(row and column block-pair partials) + list_P_P corrections (+ x / alpha),
@@ -186,13 +188,13 @@ int tmv_sym_dot_parts(int npol) { return tmv_sym_blocks(npol) * kSymSub; }
 // The pair-once sweep evaluates half the pairs, at the price of a workgroup per
 // block pair and of its block-pair partial sums; below several thousand sites it
 // has too few workgroups to fill the chip.  Against the per-target sweep
-// (tmv_rows.hip; us per matvec, pair-once / per target): FP64 one column 124 / 131
-// at 8,000 sites and 72 / 59 at 5,003, two columns 153 / 139 and 198 / 251 at 11,000;
-// FP32 one column 62 / 58 and 79 / 101, two columns 86 / 70 and 111 / 129.
-// Used from those sizes while its partial sums for max(ncols, 2) columns stay
-// under 2 GiB (up to ~100,000 sites).
-bool tmv_pair_once(int npol, int prec, int ncols) {
-    const int from = prec == 32 ? (ncols >= 2 ? 9500 : 8500) : (ncols >= 2 ? 9000 : 7500);
+// (tmv_rows.hip; us per matvec, pair-once / per target): FP64 one column 76 / 69
+// at 6,500 sites and 77 / 90 at 7,501, two columns 99 / 94 and 100 / 120; FP32 one
+// column 42 / 39 and 43 / 49, two columns 57 / 55 and 58 / 63.
+// Used from there while its partial sums for max(ncols, 2) columns stay under 2 GiB
+// (up to ~100,000 sites).
+bool tmv_pair_once(int npol, int ncols) {
+    constexpr int from = 6800;
     if (npol < from) return false;
     return tmv_sym_part_bytes(npol, ncols > 2 ? ncols : 2, 64) <= size_t(2) << 30;
 }
@@ -205,7 +207,7 @@ size_t tmv_sym_part_bytes(int npol, int M, int prec) {
 // evb / eve bracket the pair kernel only.
 template <typename R, int M>
 static void sym_launch_t(hipStream_t st, bool amoeba, int npol, const int2 *pairs, const typename V4<R>::t *site,
-                         const R *ad, const double *x, long xs, R *part, const CgState *skip, int skipM,
+                         const R *ad, const R *rc2, const double *x, long xs, R *part, const CgState *skip, int skipM,
                          hipEvent_t evb, hipEvent_t eve) {
     const int nb = tmv_sym_blocks(npol);
     const long np = (long)nb * (nb + 1) / 2;
@@ -213,39 +215,39 @@ static void sym_launch_t(hipStream_t st, bool amoeba, int npol, const int2 *pair
     if (evb) HIP_CHECK(hipEventRecord(evb, st));
     if (amoeba)
         hipLaunchKernelGGL((k_tmv_sym<R, M, true>), dim3((unsigned)np), dim3(kSymBlock), 0, st, npol, pairs, site,
-                           ad, x, xs, part_i, part_j, skip, skipM);
+                           ad, rc2, x, xs, part_i, part_j, skip, skipM);
     else
         hipLaunchKernelGGL((k_tmv_sym<R, M, false>), dim3((unsigned)np), dim3(kSymBlock), 0, st, npol, pairs, site,
-                           ad, x, xs, part_i, part_j, skip, skipM);
+                           ad, rc2, x, xs, part_i, part_j, skip, skipM);
     HIP_CHECK(hipGetLastError());
     if (eve) HIP_CHECK(hipEventRecord(eve, st));
 }
 
 void launch_tmv_sym(hipStream_t st, int prec, bool amoeba, int npol, int M, const int2 *pairs, const double4 *ps64,
-                    const double *pa64, const float4 *ps32, const float *pa32, const double *alpha,
-                    const CsrDev &pp, const double *x, long xstride, double *y, long ystride, bool dodiag,
+                    const double *pa64, const float4 *ps32, const float *pa32, const double *rc64,
+                    const float *rc32, const double *alpha, const CsrDev &pp, const double *x, long xstride, double *y, long ystride, bool dodiag,
                     double *dotpart, void *part, const int *skip_flag, hipEvent_t evb, hipEvent_t eve) {
     if (npol == 0) return;
     const CgState *skip = reinterpret_cast<const CgState *>(skip_flag);
     if (prec == 32) {
         float *pf = (float *)part;
         if (M == 1) {
-            sym_launch_t<float, 1>(st, amoeba, npol, pairs, ps32, pa32, x, xstride, pf, skip, M, evb, eve);
+            sym_launch_t<float, 1>(st, amoeba, npol, pairs, ps32, pa32, rc32, x, xstride, pf, skip, M, evb, eve);
             sym_finalize_t<float, 1>(st, amoeba, npol, pf, ps64, pa64, alpha, pp, x, xstride, y, ystride, dodiag,
                                      dotpart, skip, M);
         } else {
-            sym_launch_t<float, 2>(st, amoeba, npol, pairs, ps32, pa32, x, xstride, pf, skip, M, evb, eve);
+            sym_launch_t<float, 2>(st, amoeba, npol, pairs, ps32, pa32, rc32, x, xstride, pf, skip, M, evb, eve);
             sym_finalize_t<float, 2>(st, amoeba, npol, pf, ps64, pa64, alpha, pp, x, xstride, y, ystride, dodiag,
                                      dotpart, skip, M);
         }
     } else {
         double *pd = (double *)part;
         if (M == 1) {
-            sym_launch_t<double, 1>(st, amoeba, npol, pairs, ps64, pa64, x, xstride, pd, skip, M, evb, eve);
+            sym_launch_t<double, 1>(st, amoeba, npol, pairs, ps64, pa64, rc64, x, xstride, pd, skip, M, evb, eve);
             sym_finalize_t<double, 1>(st, amoeba, npol, pd, ps64, pa64, alpha, pp, x, xstride, y, ystride, dodiag,
                                       dotpart, skip, M);
         } else {
-            sym_launch_t<double, 2>(st, amoeba, npol, pairs, ps64, pa64, x, xstride, pd, skip, M, evb, eve);
+            sym_launch_t<double, 2>(st, amoeba, npol, pairs, ps64, pa64, rc64, x, xstride, pd, skip, M, evb, eve);
             sym_finalize_t<double, 2>(st, amoeba, npol, pd, ps64, pa64, alpha, pp, x, xstride, y, ystride, dodiag,
                                       dotpart, skip, M);
         }

@@ -65,6 +65,32 @@ def test_per_target_matvec(n, amoeba):
 
 
 @pytest.mark.parametrize("amoeba", [True, False])
+@pytest.mark.parametrize("n,kinds", [(n, ("sym64", "sym32")) for n in (1, 33, 64, 65, 129, 255, 257, 449, 513, 769)]
+                         + [(3001, ("plain64", "plain32", "sym64", "sym32"))])
+@pytest.mark.parametrize("scale", [1.0, 0.35])
+def test_damping_cutoff(n, kinds, scale, amoeba):
+    """The pair-once sweep (diagonal and other block pairs, partly filled sub-tiles)
+    and the per-target one with its lists of damped pairs, at 4 bohr and at 1.4 bohr
+    spacing (hundreds of damped pairs a site: the lists overflow), with one outlying
+    polarizability, against the oracle.  FP64: 3,001 terms of rounding 1.1e-16 on
+    sums that cancel to a few of them: 1e-12 of the largest component; FP32 by its
+    rounding of 6e-8: 3e-4."""
+    spec = chain(n, amoeba)
+    spec["cmm"] = spec["cmm"] * scale
+    spec["pol"][n // 2] = 300.0
+    s, o = pair(spec)
+    x = np.random.default_rng(n).normal(0.0, 0.05, size=(2, n, 3))
+    want = np.stack([o.tmatvec(x[0]), o.tmatvec(x[1])])
+    for kind in kinds:
+        for ncols in (1, 2):
+            y, _ = s.tmatvec(x[:ncols], kind=kind)
+            bar = 1e-12 if kind.endswith("64") else 3e-4
+            assert np.abs(y - want[:ncols]).max() <= bar * np.abs(want).max(), (kind, ncols)
+        assert np.array_equal(s.tmatvec(x, kind=kind)[0], y)
+    s.terminate()
+
+
+@pytest.mark.parametrize("amoeba", [True, False])
 @pytest.mark.parametrize("n", [1, 15, 17, 260, 1030])
 def test_thin_source_splits(n, amoeba):
     """The static field and the gradient with sources split down to 16 per
