@@ -33,7 +33,22 @@ void hip_fatal(hipError_t e, const char *what, const char *file, int line) {
 // kOtf64 / kOtf32 pick the pair-once sweep (kSym*) or the per-target one
 // (kPlain*) by size (tmv_pair_once); the explicit kinds force one of them.
 enum MvKind { kOtf64 = 0, kOtf32 = 1, kPack32 = 2, kPack64 = 3, kFmm = 4, kSym64 = 5, kSym32 = 6, kPlain64 = 7,
-              kPlain32 = 8 };
+              kPlain32 = 8, kFar32 = 9 };  // kFar32: of the mixed solver's inner solves
+
+// Tree and buffers of the inner solves' far-field matvec (far.h), kept between
+// geometries and grown on demand.
+struct FarInner {
+    bool valid = false;  // built for the current geometry
+    bool use = false;    // cheaper than the direct sweep on this geometry
+    bool bad = false;    // an inner solve with it did not reduce the residual
+    int M = 0;
+    FarDev<float> far;
+    int *cnt = nullptr;
+    struct Buf {
+        void *p = nullptr;
+        size_t cap = 0;
+    } buf[16];
+};
 
 struct DeviceState {
     int device = 0;
@@ -132,6 +147,7 @@ struct DeviceState {
     std::vector<void *> fmm_ptrs;
     double *fmm_part = nullptr, *fmm_rhs_part = nullptr;
     double *fmm_gpart_pol = nullptr, *fmm_gpart_mm = nullptr;  // gradient partials, on first use
+    FarInner inner;
 };
 
 namespace {
@@ -382,6 +398,7 @@ void upload_geometry(System &s, DeviceState &d) {
     d.grid.valid = false;
     d.nb.list_valid = false;
     d.nb.valid = false;
+    d.inner.valid = d.inner.bad = false;
     // once per geometry, not per solve
     if (s.npol > 0 && s.nmm > kHostCheckAtoms) ensure_grid(s, d);
     else if (coincident_sites(s)) fatal(kCoincident);
@@ -674,6 +691,159 @@ void ensure_fmm(System &s, DeviceState &d) {
     d.fmm_valid = true;
 }
 
+// The inner solves of the mixed solver take the far-field matvec in FP32 (order 8:
+// relative error 2e-5 .. 1e-4) from this many sites where it leaves at most an eighth
+// of the pairs to the near field.  It is an approximate operator of an inner solve,
+// like its preconditioner: the FP64 residuals are of the direct sum, convergence is
+// decided by them, and a geometry where an inner solve does not cut them by 10 goes
+// back to the direct sweep.  us per matvec of two columns, far field / pair-once:
+// 126 / 160 at 15,000 sites, 148 / 260 at 20,001, 285 / 930 at 40,000, 480 / 2040 at
+// 60,000; the tree costs 1.0 to 1.6 ms per geometry and the solve one FP64 residual
+// more.  Whole solves: 15,000 sites 4.4 / 4.4 ms, 24,000 (AMBER) 3.6 / 4.3, 40,000
+// 10.2 / 19.3, 60,000 30.3 / 54.8; a gradient step at 20,001, with its tree, 8.0 / 9.1.
+// Leaves of 24 sites and more in the mean: at 60,000 sites 7.5 and 117 a leaf take
+// 486 and 495 us, the larger ones with an error of 2.6e-5 instead of 1.4e-4.
+constexpr int kFarInnerFrom = 18000, kFarInnerOrder = 8, kFarInnerOccupancy = 24;
+
+// Octree over the polarizable sites for M columns: leaves of at least
+// kFarInnerOccupancy sites in the mean of the occupied ones.
+void ensure_far_inner(System &s, DeviceState &d, int M) {
+    FarInner &in = d.inner;
+    if (in.valid && in.M == M) return;
+    in.valid = true;
+    in.M = M;
+    in.use = false;
+    const int npol = s.npol;
+    double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
+    for (int p = 0; p < npol; p++)
+        for (int c = 0; c < 3; c++) {
+            const double v = s.cmm[3 * s.polar_mm[p] + c];
+            lo[c] = std::min(lo[c], v);
+            hi[c] = std::max(hi[c], v);
+        }
+    FarDev<float> &f = in.far;
+    FarLevels &lv = f.lv;
+    lv.side = 0.0;
+    for (int c = 0; c < 3; c++) lv.side = std::max(lv.side, hi[c] - lo[c]);
+    lv.side = lv.side * (1.0 + 1e-9) + 1e-6;
+    for (int c = 0; c < 3; c++) lv.origin[c] = lo[c] - 0.5 * (lv.side - (hi[c] - lo[c]));
+    std::vector<int> leaf(npol), start, cnt;
+    for (int L = 5;; L--) {  // the cell arrays stay under 100 MB
+        if (L < 2) return;  // every site is near every other
+        const int ns = 1 << L;
+        const double ih = ns / lv.side;
+        start.assign(((size_t)1 << 3 * L) + 1, 0);
+        int occupied = 0;
+        for (int p = 0; p < npol; p++) {
+            const double *r = &s.cmm[3 * s.polar_mm[p]];
+            int k[3];
+            for (int c = 0; c < 3; c++) k[c] = std::min(std::max((int)((r[c] - lv.origin[c]) * ih), 0), ns - 1);
+            leaf[p] = (k[2] * ns + k[1]) * ns + k[0];
+            occupied += start[leaf[p] + 1]++ == 0;
+        }
+        if ((long)occupied * kFarInnerOccupancy > npol) continue;
+        lv.levels = L;
+        break;
+    }
+    const int L = lv.levels, ns = 1 << L;
+    for (int l = 0; l <= L + 1; l++) lv.off[l] = l == 0 ? 0 : lv.off[l - 1] + (1L << 3 * (l - 1));
+    cnt.assign(lv.off[L + 1], 0);
+    double near = 0.0;
+    for (int z = 0; z < ns; z++)
+        for (int y = 0; y < ns; y++)
+            for (int x = 0; x < ns; x++) {
+                const int k = (z * ns + y) * ns + x, c = start[k + 1];
+                if (c == 0) continue;
+                for (int l = 2; l <= L; l++) {
+                    const int u = L - l;
+                    cnt[lv.off[l] + ((((long)(z >> u) << l) + (y >> u)) << l) + (x >> u)] += c;
+                }
+                long all = 0;
+                for (int zz = std::max(z - 1, 0); zz <= std::min(z + 1, ns - 1); zz++)
+                    for (int yy = std::max(y - 1, 0); yy <= std::min(y + 1, ns - 1); yy++)
+                        for (int xx = std::max(x - 1, 0); xx <= std::min(x + 1, ns - 1); xx++)
+                            all += start[(zz * ns + yy) * ns + xx + 1];
+                near += (double)c * all;
+            }
+    if (near > 0.125 * npol * npol) return;
+    in.use = true;
+    std::vector<int2> blocks;
+    const int nleaf = ns * ns * ns;
+    for (int k = 0; k < nleaf; k++) {
+        start[k + 1] += start[k];
+        for (int t = start[k]; t < start[k + 1]; t += kFarNearTargets) blocks.push_back(make_int2(k, t));
+    }
+    std::vector<int> order(npol), sorted(npol), next(start.begin(), start.end() - 1);
+    std::vector<float4> pos(npol);
+    std::vector<float> a(npol);
+    for (int p = 0; p < npol; p++) {
+        const int t = next[leaf[p]]++, i = s.polar_mm[p];
+        const double th = s.thole[i];
+        order[t] = p;
+        sorted[t] = leaf[p];
+        pos[t] = make_float4((float)s.cmm[3 * i], (float)s.cmm[3 * i + 1], (float)s.cmm[3 * i + 2],
+                             th > kEpsRp ? (float)(1.0 / th) : std::numeric_limits<float>::infinity());
+        a[t] = (float)s.thole_damping_mm[i];
+    }
+    f.npol = npol;
+    f.cells = lv.off[L + 1] - lv.off[2];
+    f.groups.width = M == 1 ? 32 : 16;
+    std::vector<int> gcell, glevel;
+    far_group_cells(lv, cnt, f.groups.width, gcell, glevel);
+    f.groups.n = (int)glevel.size();
+    f.nsplit = far_splits(f.groups.n);
+    f.nblocks = (int)blocks.size();
+    int slot = 0;
+    auto room = [&](auto *&p, size_t count) {
+        using T = std::remove_reference_t<decltype(*p)>;
+        FarInner::Buf &b = in.buf[slot++];
+        const size_t bytes = sizeof(T) * std::max<size_t>(count, 1);
+        if (b.cap < bytes) {
+            if (b.p) dfree(d, b.p);
+            b.p = dmalloc(d, bytes);
+            b.cap = bytes;
+        }
+        p = static_cast<T *>(b.p);
+    };
+    auto up = [&](const auto &v, auto *&p) {
+        room(p, v.size());
+        upload(v.data(), p, sizeof(v[0]) * v.size());
+    };
+    up(start, f.leaf_start);
+    up(order, f.order);
+    up(sorted, f.leaf);
+    up(pos, f.pos);
+    up(a, f.a);
+    up(blocks, f.blocks);
+    up(gcell, f.groups.cell);
+    up(glevel, f.groups.level);
+    up(cnt, in.cnt);
+    f.rc2 = d.rc32;
+    if (!f.K) {  // the tables depend on the order alone
+        f.p = kFarInnerOrder;
+        f.nc = far_coefs(f.p);
+        const FarTables<float> &t = far_tables<float>(f.p);
+        f.K = dalloc<float>(d, t.K.size());
+        upload(t.K.data(), f.K, sizeof(float) * t.K.size());
+        f.zero = dalloc<float>(d, f.nc);
+        const std::vector<float> zero(f.nc, 0.f);
+        upload(zero.data(), f.zero, sizeof(float) * f.nc);
+    }
+    room(f.mom, (size_t)f.cells * M * f.nc);
+    room(f.part, (size_t)f.nsplit * f.groups.n * 32 * f.nc);
+    room(f.grad, (size_t)f.cells * M * 3 * kFarBasis);
+    room(f.basis, (size_t)(L - 1) * npol * kFarBasis);
+    room(f.dots, (size_t)M * f.nblocks);
+    far_launch_basis(d.stream, f, d.ps64);
+}
+
+// Whether the mixed solver's inner solves of M columns use it.
+bool far_inner(System &s, DeviceState &d, int M) {
+    if (s.npol < kFarInnerFrom || M != s.n_ipd || d.inner.bad) return false;
+    ensure_far_inner(s, d, M);
+    return d.inner.use;
+}
+
 // Block pairs and block-pair partials of the pair-once sweeps (T matvec and
 // static field), on first use.
 void ensure_sym(const System &s, DeviceState &d) {
@@ -694,6 +864,7 @@ static int matvec_dot_parts(System &s, DeviceState &d, int kind, int M) {
         ensure_fmm(s, d);
         if (fmm_far_matvec(d)) return kFarDots;
     }
+    if (kind == kFar32) return kFarDots;
     const int prec = kind == kOtf32 ? 32 : 64;
     if (kind == kOtf64 || kind == kOtf32)
         return tmv_pair_once(s.npol, M) ? tmv_sym_dot_parts(s.npol) : tmv_rows_dot_parts(s.npol, prec, M);
@@ -715,6 +886,13 @@ void matvec(System &s, DeviceState &d, int kind, int M, const double *x, double 
         fmm_launch_matvec_fields(d.stream, d.fmm, s.amoeba, M, x, n, d.fmm_part);
         launch_tmv_finalize64(d.stream, s.amoeba, s.npol, M, d.fmm_part, kFmmNearSplits + 1, d.ps64, d.pa64, d.alpha,
                               d.pp, x, n, y, n, dodiag, dotpart, reinterpret_cast<const int *>(skip));
+        return;
+    }
+    if (kind == kFar32) {
+        const int pi = prof_begin(d, kOtf32);
+        far_launch_matvec(d.stream, d.inner.far, s.amoeba, M, d.inner.cnt, d.ps64, d.pa64, d.alpha, d.pp, x, n, y, n,
+                          dodiag, dotpart, skip);
+        if (pi >= 0) HCHECK(hipEventRecord(d.prof_pool[2 * pi + 1], d.stream));
         return;
     }
     if (kind == kOtf64 || kind == kOtf32) {
@@ -1008,7 +1186,7 @@ struct MixedResult {
 constexpr int kSpecMaxOuter = 6;
 
 int mixed_solve_ahead(System &s, DeviceState &d, int M, const double *b, double *x, bool zero_guess, double tol,
-                      int kind32, bool nb, MixedResult &res) {
+                      int kind32, double eta, bool nb, MixedResult &res) {
     const int K = s.pred_outer;
     if (K < 2 || K > kSpecMaxOuter) return -1;
     for (int o = 0; o < K - 1; o++)
@@ -1030,7 +1208,7 @@ int mixed_solve_ahead(System &s, DeviceState &d, int M, const double *b, double 
             matvec(s, d, kOtf64, M, x, d.vh, true, nullptr, o == 0 ? nullptr : out);
         }
         launch_residual_rms(d.stream, n, M, b, d.vh, d.vr2, d.alpha, d.red_a, d.scal);
-        launch_refine_decide(d.stream, M, d.scal, out, tol, refine_eta(), refine_frac(), d.tol_dev, o);
+        launch_refine_decide(d.stream, M, d.scal, out, tol, eta, refine_frac(), d.tol_dev, o);
         if (o == K - 1) break;
         CgState *cs = d.cs_spec + 2 * (o + 1);
         double *rb[2] = {d.vr, nb ? d.vr3 : d.vr};
@@ -1083,14 +1261,17 @@ MixedResult mixed_solve(System &s, DeviceState &d, int M, const double *b, doubl
     const long n = d.n;
     MixedResult res;
     const int max_outer = 30;
-    // Inner target per refinement step: max(refine_eta() * rms, refine_frac() * tol).
-    const double eta_min = refine_eta(), frac = refine_frac();
+    // Inner target per refinement step: max(eta * rms, refine_frac() * tol).
+    const double frac = refine_frac();
     const int K = s.pred_outer;
+    bool far = kind32 == kOtf32 && far_inner(s, d, M);
+    double before[2] = {HUGE_VAL, HUGE_VAL};
     // near-field preconditioner for the inner solves (any SPD one will do: the
     // FP64 residual decides convergence)
     const bool nb = s.inner_precond == 1 && s.npol > 0;
     if (nb) ensure_nb(s, d);
-    const int ahead = mixed_solve_ahead(s, d, M, b, x, zero_guess, tol, kind32, nb, res);
+    const int ahead = mixed_solve_ahead(s, d, M, b, x, zero_guess, tol, far ? kFar32 : kind32,
+                                        far ? refine_eta_far() : refine_eta(), nb, res);
     if (ahead > 0) {
         s.pred_outer = res.outer;
         return res;
@@ -1115,15 +1296,28 @@ MixedResult mixed_solve(System &s, DeviceState &d, int M, const double *b, doubl
         for (int m = 0; m < M; m++) {
             const double rms = d.scal_host[m];
             conv = conv && rms < tol;
-            tin[m] = rms < tol ? 1e300 : std::max(eta_min * rms, frac * tol);
+            // the far field's inner solves cut the residual by 1e3 each; where one does
+            // not by 10, its expansions do not fit this geometry
+            if (far && rms >= tol && !(rms < 0.1 * before[m])) d.inner.bad = true;
+            before[m] = rms;
         }
+        if (far && d.inner.bad) {
+            far = false;
+            if (!std::isfinite(before[0]) || (M > 1 && !std::isfinite(before[1]))) {
+                HCHECK(hipMemsetAsync(x, 0, sizeof(double) * M * n, d.stream));
+                xzero = true;
+                continue;
+            }
+        }
+        for (int m = 0; m < M; m++)
+            tin[m] = before[m] < tol ? 1e300 : std::max((far ? refine_eta_far() : refine_eta()) * before[m], frac * tol);
         if (conv) {
             res.ok = true;
             s.pred_outer = res.outer;
             return res;
         }
         // inner FP32 PCG on T delta = r from delta = 0
-        CgResult cr = cg_solve(s, d, kind32, M, d.vr2, d.vd, tin, maxit, true, 0.0, 2 + std::min(outer, 13), nb);
+        CgResult cr = cg_solve(s, d, far ? kFar32 : kind32, M, d.vr2, d.vd, tin, maxit, true, 0.0, 2 + std::min(outer, 13), nb);
         res.inner += std::max(cr.iters[0], M > 1 ? cr.iters[1] : 0);
         launch_axpy(d.stream, n, M, 1.0, d.vd, x);
         xzero = false;
@@ -1138,6 +1332,9 @@ MixedResult mixed_solve(System &s, DeviceState &d, int M, const double *b, doubl
 // the true one; asking for that much (instead of stopping at the tolerance)
 // makes one refinement step enough for most warm-started solves.
 double refine_eta() { return 1e-6; }
+// The far-field matvec of the inner solves is accurate to ~1e-4 (1e-3, 3e-4, 1e-4: one
+// refinement step more or less, the solves within 3% of each other).
+double refine_eta_far() { return 2e-4; }
 // In the serving loop a solve starts from its predecessor, about 1e6 tolerances away,
 // so that 1e-6 of it ends on either side of the tolerance by the sums' rounding (errors
 // of 2e-9 or 1e-8 in the dipoles); a quarter of it, still above FP32's reach, ends below
@@ -1402,6 +1599,8 @@ size_t device_footprint_estimate(const System &s) {
         b += tmv_sym_part_bytes(s.npol, 2, 64) + sizeof(int2) * nb * (nb + 1) / 2;
     }
     b += (size_t)(s.list_S_P_P.nnz() + s.list_S_P_D.nnz() + 2 * s.list_P_P.nnz() + s.list_P_P_dense.nnz()) * 24;
+    if (s.npol >= kFarInnerFrom)  // tree of the far-field inner solves: basis functions, cells, tables
+        b += np * (5 * kFarBasis * sizeof(float) + 64) + (size_t(128) << 20);
     return b + (1 << 20);
 }
 

@@ -67,3 +67,43 @@ def test_static_field_and_gradient_orders(p):
             err.append(np.abs(s.polelec_geomgrad() - gd).max() / np.abs(gd).max())
         assert err[1] <= err[0] / 4.0 and err[2] <= 1.5 * err[1]
     s.terminate()
+
+
+@pytest.mark.parametrize("amoeba", [True, False])
+@pytest.mark.parametrize("shape", ["cube", "plate", "clump"])
+def test_inner_solves(shape, amoeba):
+    """Mixed solves large enough for the far-field inner matvec, from nothing and from
+    the previous dipoles, before and after a change of coordinates, against the FP64
+    solver: a cube, a plate of one layer (most cells empty) and a cube with a few sites
+    so far away that it falls into a few leaves (the direct sweep stays).  Both solvers
+    stop at an rms of 3e-10 of the preconditioned residual; its inverse operator is
+    below 10 here, so that the dipoles agree to an rms of 6e-9."""
+    from openmmpol_amd import OMMPSystem
+    n = 18001
+    spec = chain(n, amoeba, seed=7)
+    rng = np.random.default_rng(8)
+    if shape == "plate":
+        g = np.arange(135)
+        p = np.stack(np.meshgrid(g, g, indexing="ij"), axis=-1).reshape(-1, 2)[:n] * 4.0
+        spec["cmm"] = np.concatenate([p, np.zeros((n, 1))], axis=1) + rng.uniform(-0.8, 0.8, size=(n, 3))
+    elif shape == "clump":
+        spec["cmm"][-8:] += 5000.0 * rng.normal(size=(8, 3))
+    both = []
+    for precision in ("fp64", "mixed"):
+        s = OMMPSystem.from_arrays(amoeba, spec["cmm"], spec["q"], spec["pol"], spec["bonds_ri"], spec["bonds_ci"],
+                                   pgroup=spec["pgroup"] if amoeba else None)
+        s.set_precision(precision)
+        s.set_solver_tolerance(3e-10, 500)
+        field = np.random.default_rng(9).normal(0.0, 1e-2, size=(2, n, 3))
+        got = []
+        for scale in (1.0, 1.02):
+            if scale != 1.0:
+                s.update_coordinates(spec["cmm"] * scale)
+            for f in field:
+                s.set_external_field(f)
+                s.get_polelec_energy()
+                got.append(s.ipd.copy())
+        both.append(np.array(got))
+        s.terminate()
+    d = both[0] - both[1]
+    assert np.sqrt((d * d).mean(axis=(1, 2, 3))).max() <= 6e-9
