@@ -700,7 +700,7 @@ void ensure_fmm(System &s, DeviceState &d) {
 // 126 / 160 at 15,000 sites, 148 / 260 at 20,001, 285 / 930 at 40,000, 480 / 2040 at
 // 60,000; the tree costs 1.0 to 1.6 ms per geometry and the solve one FP64 residual
 // more.  Whole solves: 15,000 sites 4.4 / 4.4 ms, 24,000 (AMBER) 3.6 / 4.3, 40,000
-// 10.2 / 19.3, 60,000 30.3 / 54.8; a gradient step at 20,001, with its tree, 8.0 / 9.1.
+// 10.3 / 19.3, 60,000 31.1 / 54.8; a gradient step at 20,001, with its tree, 8.25 / 9.1.
 // Leaves of 24 sites and more in the mean: at 60,000 sites 7.5 and 117 a leaf take
 // 486 and 495 us, the larger ones with an error of 2.6e-5 instead of 1.4e-4.
 constexpr int kFarInnerFrom = 18000, kFarInnerOrder = 8, kFarInnerOccupancy = 24;
@@ -1168,6 +1168,18 @@ int diis_solve(System &s, DeviceState &d, int kind, const double *rhs, double *x
     return max_norm > tol ? 1 : 0;
 }
 
+// An inner solve aims at max(eta * rms, frac * tol); the FP64 residual after it is
+// accepted below accept * tol (the guess's own below tol).
+struct RefineAim {
+    double eta, frac, accept;
+};
+// The far-field matvec of the inner solves is accurate to ~1e-4 (eta of 1e-3, 3e-4,
+// 1e-4: one refinement step more or less, the solves within 3% of each other).  Two such
+// inner solves may end anywhere around the tolerance; asked for half of it, the result is
+// as close as that of the direct inner solves, which end below their aim of 0.25 (with
+// 1.0 the dipoles of a 20,001-site system were 2e-8 off instead of 5e-9).
+constexpr RefineAim kAimFar = {2e-4, 0.25, 0.5};
+
 // FP32 matvec inside FP64 iterative refinement, columns solved together.
 struct MixedResult {
     int outer = 0, inner = 0;
@@ -1186,7 +1198,7 @@ struct MixedResult {
 constexpr int kSpecMaxOuter = 6;
 
 int mixed_solve_ahead(System &s, DeviceState &d, int M, const double *b, double *x, bool zero_guess, double tol,
-                      int kind32, double eta, bool nb, MixedResult &res) {
+                      int kind32, const RefineAim &aim, bool nb, MixedResult &res) {
     const int K = s.pred_outer;
     if (K < 2 || K > kSpecMaxOuter) return -1;
     for (int o = 0; o < K - 1; o++)
@@ -1208,7 +1220,8 @@ int mixed_solve_ahead(System &s, DeviceState &d, int M, const double *b, double 
             matvec(s, d, kOtf64, M, x, d.vh, true, nullptr, o == 0 ? nullptr : out);
         }
         launch_residual_rms(d.stream, n, M, b, d.vh, d.vr2, d.alpha, d.red_a, d.scal);
-        launch_refine_decide(d.stream, M, d.scal, out, tol, eta, refine_frac(), d.tol_dev, o);
+        launch_refine_decide(d.stream, M, d.scal, out, o == 0 ? tol : aim.accept * tol, aim.eta,
+                             o == 0 ? aim.frac : aim.frac / aim.accept, d.tol_dev, o);
         if (o == K - 1) break;
         CgState *cs = d.cs_spec + 2 * (o + 1);
         double *rb[2] = {d.vr, nb ? d.vr3 : d.vr};
@@ -1261,8 +1274,7 @@ MixedResult mixed_solve(System &s, DeviceState &d, int M, const double *b, doubl
     const long n = d.n;
     MixedResult res;
     const int max_outer = 30;
-    // Inner target per refinement step: max(eta * rms, refine_frac() * tol).
-    const double frac = refine_frac();
+    const RefineAim direct = {refine_eta(), refine_frac(), 1.0};
     const int K = s.pred_outer;
     bool far = kind32 == kOtf32 && far_inner(s, d, M);
     double before[2] = {HUGE_VAL, HUGE_VAL};
@@ -1271,7 +1283,7 @@ MixedResult mixed_solve(System &s, DeviceState &d, int M, const double *b, doubl
     const bool nb = s.inner_precond == 1 && s.npol > 0;
     if (nb) ensure_nb(s, d);
     const int ahead = mixed_solve_ahead(s, d, M, b, x, zero_guess, tol, far ? kFar32 : kind32,
-                                        far ? refine_eta_far() : refine_eta(), nb, res);
+                                        far ? kAimFar : direct, nb, res);
     if (ahead > 0) {
         s.pred_outer = res.outer;
         return res;
@@ -1293,12 +1305,19 @@ MixedResult mixed_solve(System &s, DeviceState &d, int M, const double *b, doubl
         res.outer = outer + 1;
         bool conv = true;
         double tin[2];
+        // (steps enqueued ahead before this one had inner solves too)
+        double accept[2] = {tol, tol};
         for (int m = 0; m < M; m++) {
             const double rms = d.scal_host[m];
-            conv = conv && rms < tol;
-            // the far field's inner solves cut the residual by 1e3 each; where one does
-            // not by 10, its expansions do not fit this geometry
-            if (far && rms >= tol && !(rms < 0.1 * before[m])) d.inner.bad = true;
+            if (far && outer > 0) {
+                // the far field's inner solves cut the residual by 1e3 each; where one does
+                // not by 10, the residual is at its rounding or the expansions do not fit
+                // this geometry
+                const bool stalled = !(rms < 0.1 * before[m]);
+                if (!stalled) accept[m] = kAimFar.accept * tol;
+                else if (!(rms < tol)) d.inner.bad = true;
+            }
+            conv = conv && rms < accept[m];
             before[m] = rms;
         }
         if (far && d.inner.bad) {
@@ -1309,8 +1328,9 @@ MixedResult mixed_solve(System &s, DeviceState &d, int M, const double *b, doubl
                 continue;
             }
         }
+        const RefineAim &aim = far ? kAimFar : direct;
         for (int m = 0; m < M; m++)
-            tin[m] = before[m] < tol ? 1e300 : std::max((far ? refine_eta_far() : refine_eta()) * before[m], frac * tol);
+            tin[m] = before[m] < accept[m] ? 1e300 : std::max(aim.eta * before[m], aim.frac * tol);
         if (conv) {
             res.ok = true;
             s.pred_outer = res.outer;
@@ -1332,9 +1352,6 @@ MixedResult mixed_solve(System &s, DeviceState &d, int M, const double *b, doubl
 // the true one; asking for that much (instead of stopping at the tolerance)
 // makes one refinement step enough for most warm-started solves.
 double refine_eta() { return 1e-6; }
-// The far-field matvec of the inner solves is accurate to ~1e-4 (1e-3, 3e-4, 1e-4: one
-// refinement step more or less, the solves within 3% of each other).
-double refine_eta_far() { return 2e-4; }
 // In the serving loop a solve starts from its predecessor, about 1e6 tolerances away,
 // so that 1e-6 of it ends on either side of the tolerance by the sums' rounding (errors
 // of 2e-9 or 1e-8 in the dipoles); a quarter of it, still above FP32's reach, ends below

@@ -132,7 +132,6 @@ int verbosity();
 // Inner-solve target of the mixed refinement: max(eta * outer rms, frac * tol).
 double refine_eta();
 double refine_eta_serving();
-double refine_eta_far();
 double refine_frac();
 double refine_frac_wide();
 void device_release(System &s);
