@@ -255,7 +255,7 @@ void launch_cg_direction_nb(hipStream_t st, int npol, int M, int it, const doubl
 
 // Mixed-precision refinement step decided on the device (k_refine_decide).
 void launch_refine_decide(hipStream_t st, int M, const double *rms, CgState *out, double tol, double eta,
-                          double frac, double *inner_tol, int outer);
+                          double frac, double *inner_tol, int outer, bool check);
 void launch_cg_update(hipStream_t st, long n, int M, int it, const double *h, double *x, double *r,
                       double *z, const double *p, const double *alpha, const double *red_hp,
                       int nred_hp, double *red_rz, CgState *cs);

@@ -649,6 +649,7 @@ void ensure_fmm(System &s, DeviceState &d) {
         r.pos = f.pol_pos;
         r.a = f.pol_a;
         r.rc2 = d.rc64;
+        r.xs = fmm_alloc<double4>(d, npol);
         auto up = [&](const auto &v) {
             using T = std::decay_t<decltype(v[0])>;
             T *p = fmm_alloc<T>(d, std::max<size_t>(v.size(), 1));
@@ -676,12 +677,7 @@ void ensure_fmm(System &s, DeviceState &d) {
         r.part = fmm_alloc<double>(d, (size_t)r.nsplit * most * 32 * r.nc);
         r.grad = fmm_alloc<double>(d, (size_t)r.cells * 3 * kFarBasis);
         r.basis = fmm_alloc<double>(d, (size_t)std::max(h.levels - 1, 0) * npol * kFarBasis);
-        std::vector<int2> blocks;
-        const int T = kFarNearTargets;
-        for (int k = 0; k + 1 < (int)h.pol_leaf_start.size(); k++)
-            for (int t0 = h.pol_leaf_start[k]; t0 < h.pol_leaf_start[k + 1]; t0 += T) blocks.push_back(make_int2(k, t0));
-        r.nblocks = (int)blocks.size();
-        r.blocks = up(blocks);
+        r.blocks = up(far_blocks(r, h.pol_leaf_start));
         r.dots = fmm_alloc<double>(d, r.nblocks);
         far_launch_basis(d.stream, r, d.ps64);
     }
@@ -697,13 +693,19 @@ void ensure_fmm(System &s, DeviceState &d) {
 // like its preconditioner: the FP64 residuals are of the direct sum, convergence is
 // decided by them, and a geometry where an inner solve does not cut them by 10 goes
 // back to the direct sweep.  us per matvec of two columns, far field / pair-once:
-// 126 / 160 at 15,000 sites, 148 / 260 at 20,001, 285 / 930 at 40,000, 480 / 2040 at
-// 60,000; the tree costs 1.0 to 1.6 ms per geometry and the solve one FP64 residual
-// more.  Whole solves: 15,000 sites 4.4 / 4.4 ms, 24,000 (AMBER) 3.6 / 4.3, 40,000
-// 10.3 / 19.3, 60,000 31.1 / 54.8; a gradient step at 20,001, with its tree, 8.25 / 9.1.
-// Leaves of 24 sites and more in the mean: at 60,000 sites 7.5 and 117 a leaf take
-// 486 and 495 us, the larger ones with an error of 2.6e-5 instead of 1.4e-4.
-constexpr int kFarInnerFrom = 18000, kFarInnerOrder = 8, kFarInnerOccupancy = 24;
+// 110 / 160 at 15,000 sites, 125 / 260 at 20,001, 232 / 930 at 40,000, 387 / 2040 at
+// 60,000, of one column 91 / 107 at 15,000, 100 / 195 at 20,001; the tree costs 1.0 to
+// 1.6 ms per geometry and a solve one or two FP32 residuals of the direct sweep.  Whole
+// solves with two columns: 14,000 sites (water) 2.66 / 3.06, 15,000 3.70 / 4.43, 60,000
+// 24.6 / 54.8; with one column 24,000 3.2 / 4.3; gradient steps with their trees: 20,001
+// 7.5 / 9.1.  With one FP64 residual more instead of the FP32 ones 12,000 sites took
+// 3.25 / 3.29, 10,000 3.0 / 2.8, one column at 15,000 2.04 / 1.94: used from 13,000 and
+// 18,000.
+// Leaves of 24 sites and more in the mean: at 60,000 sites 29 and 171 an occupied leaf
+// take 363 and 387 us, the larger ones with an error of 2.6e-5 instead of 1.4e-4, which
+// saves iterations (solve 33.1 and 28.0 ms).
+constexpr int kFarInnerOrder = 8, kFarInnerOccupancy = 24;
+int far_inner_from(int M) { return M == 2 ? 13000 : 18000; }
 
 // Octree over the polarizable sites for M columns: leaves of at least
 // kFarInnerOccupancy sites in the mean of the occupied ones.
@@ -767,12 +769,7 @@ void ensure_far_inner(System &s, DeviceState &d, int M) {
             }
     if (near > 0.125 * npol * npol) return;
     in.use = true;
-    std::vector<int2> blocks;
-    const int nleaf = ns * ns * ns;
-    for (int k = 0; k < nleaf; k++) {
-        start[k + 1] += start[k];
-        for (int t = start[k]; t < start[k + 1]; t += kFarNearTargets) blocks.push_back(make_int2(k, t));
-    }
+    for (int k = 0; k < ns * ns * ns; k++) start[k + 1] += start[k];
     std::vector<int> order(npol), sorted(npol), next(start.begin(), start.end() - 1);
     std::vector<float4> pos(npol);
     std::vector<float> a(npol);
@@ -792,7 +789,6 @@ void ensure_far_inner(System &s, DeviceState &d, int M) {
     far_group_cells(lv, cnt, f.groups.width, gcell, glevel);
     f.groups.n = (int)glevel.size();
     f.nsplit = far_splits(f.groups.n);
-    f.nblocks = (int)blocks.size();
     int slot = 0;
     auto room = [&](auto *&p, size_t count) {
         using T = std::remove_reference_t<decltype(*p)>;
@@ -814,7 +810,7 @@ void ensure_far_inner(System &s, DeviceState &d, int M) {
     up(sorted, f.leaf);
     up(pos, f.pos);
     up(a, f.a);
-    up(blocks, f.blocks);
+    up(far_blocks(f, start), f.blocks);
     up(gcell, f.groups.cell);
     up(glevel, f.groups.level);
     up(cnt, in.cnt);
@@ -834,12 +830,13 @@ void ensure_far_inner(System &s, DeviceState &d, int M) {
     room(f.grad, (size_t)f.cells * M * 3 * kFarBasis);
     room(f.basis, (size_t)(L - 1) * npol * kFarBasis);
     room(f.dots, (size_t)M * f.nblocks);
+    room(f.xs, (size_t)M * npol);
     far_launch_basis(d.stream, f, d.ps64);
 }
 
 // Whether the mixed solver's inner solves of M columns use it.
 bool far_inner(System &s, DeviceState &d, int M) {
-    if (s.npol < kFarInnerFrom || M != s.n_ipd || d.inner.bad) return false;
+    if (s.npol < far_inner_from(M) || M != s.n_ipd || d.inner.bad) return false;
     ensure_far_inner(s, d, M);
     return d.inner.use;
 }
@@ -1168,17 +1165,11 @@ int diis_solve(System &s, DeviceState &d, int kind, const double *rhs, double *x
     return max_norm > tol ? 1 : 0;
 }
 
-// An inner solve aims at max(eta * rms, frac * tol); the FP64 residual after it is
-// accepted below accept * tol (the guess's own below tol).
-struct RefineAim {
-    double eta, frac, accept;
-};
-// The far-field matvec of the inner solves is accurate to ~1e-4 (eta of 1e-3, 3e-4,
-// 1e-4: one refinement step more or less, the solves within 3% of each other).  Two such
-// inner solves may end anywhere around the tolerance; asked for half of it, the result is
-// as close as that of the direct inner solves, which end below their aim of 0.25 (with
-// 1.0 the dipoles of a 20,001-site system were 2e-8 off instead of 5e-9).
-constexpr RefineAim kAimFar = {2e-4, 0.25, 0.5};
+// With the far-field matvec (relative error 2e-5 to 1e-4) an inner solve is two: each
+// reduces its residual by this much, the FP32 residual of the direct sweep between
+// them, so that both together reach refine_eta() like a direct inner solve.  The second
+// is left out where the first reaches the tolerance.
+constexpr double kEtaFar = 1e-3;
 
 // FP32 matvec inside FP64 iterative refinement, columns solved together.
 struct MixedResult {
@@ -1195,14 +1186,15 @@ struct MixedResult {
 // next step.  Returns -1 when there is no prediction (nothing enqueued), 0 when
 // some column has not converged within the K steps (res.inner counts the inner
 // iterations run; the caller goes on from x), K when every column converged.
-constexpr int kSpecMaxOuter = 6;
+constexpr int kSpecMaxOuter = 8;
 
 int mixed_solve_ahead(System &s, DeviceState &d, int M, const double *b, double *x, bool zero_guess, double tol,
-                      int kind32, const RefineAim &aim, bool nb, MixedResult &res) {
+                      int kind32, bool nb, MixedResult &res) {
     const int K = s.pred_outer;
-    if (K < 2 || K > kSpecMaxOuter) return -1;
+    const bool far = kind32 == kFar32;  // steps 1, 3, ..: FP32 residuals, -1: left out
+    if (K < 2 || K > kSpecMaxOuter || (far && K % 2 == 0)) return -1;
     for (int o = 0; o < K - 1; o++)
-        if (s.pred_iters[2 + o] <= 0) return -1;
+        if (s.pred_iters[2 + o] <= 0 && !(far && o % 2 && s.pred_iters[2 + o] == -1)) return -1;
     const long n = d.n;
     const int W = 2 * (kSpecMaxOuter + 1);
     if (!d.cs_spec) {
@@ -1213,15 +1205,19 @@ int mixed_solve_ahead(System &s, DeviceState &d, int M, const double *b, double 
     const int nred_hp = matvec_dot_parts(s, d, kind32, M);
     bool xzero = zero_guess;
     for (int o = 0; o < K; o++) {
-        if (xzero) {
+        const bool r32 = far && o % 2;
+        if (r32 && s.pred_iters[2 + o] == -1) continue;
+        if (r32) {
+            matvec(s, d, kOtf32, M, d.vd, d.vh, true, nullptr, out);
+        } else if (xzero) {
             HCHECK(hipMemsetAsync(d.vh, 0, sizeof(double) * M * n, d.stream));
         } else {
             // out still holds the previous solve's state until step 0 is decided
             matvec(s, d, kOtf64, M, x, d.vh, true, nullptr, o == 0 ? nullptr : out);
         }
-        launch_residual_rms(d.stream, n, M, b, d.vh, d.vr2, d.alpha, d.red_a, d.scal);
-        launch_refine_decide(d.stream, M, d.scal, out, o == 0 ? tol : aim.accept * tol, aim.eta,
-                             o == 0 ? aim.frac : aim.frac / aim.accept, d.tol_dev, o);
+        launch_residual_rms(d.stream, n, M, r32 ? d.vr2 : b, d.vh, d.vr2, d.alpha, d.red_a, d.scal);
+        launch_refine_decide(d.stream, M, d.scal, out, tol, far ? kEtaFar : refine_eta(), refine_frac(), d.tol_dev, o,
+                             !r32);
         if (o == K - 1) break;
         CgState *cs = d.cs_spec + 2 * (o + 1);
         double *rb[2] = {d.vr, nb ? d.vr3 : d.vr};
@@ -1252,6 +1248,7 @@ int mixed_solve_ahead(System &s, DeviceState &d, int M, const double *b, double 
     // next predictions: an inner solve that ran out of launches gets two more
     for (int o = 0; o < K - 1; o++) {
         const int ran = s.pred_iters[2 + o];
+        if (ran < 0) continue;
         int most = 0;
         for (int m = 0; m < M; m++)
             most = std::max(most, h[2 * (o + 1) + m].done ? h[2 * (o + 1) + m].iters : ran + 2);
@@ -1274,73 +1271,82 @@ MixedResult mixed_solve(System &s, DeviceState &d, int M, const double *b, doubl
     const long n = d.n;
     MixedResult res;
     const int max_outer = 30;
-    const RefineAim direct = {refine_eta(), refine_frac(), 1.0};
+    // Inner target per refinement step: max(eta * rms, refine_frac() * tol).
+    const double frac = refine_frac();
     const int K = s.pred_outer;
     bool far = kind32 == kOtf32 && far_inner(s, d, M);
+    const bool far_ahead = far;
     double before[2] = {HUGE_VAL, HUGE_VAL};
     // near-field preconditioner for the inner solves (any SPD one will do: the
     // FP64 residual decides convergence)
     const bool nb = s.inner_precond == 1 && s.npol > 0;
     if (nb) ensure_nb(s, d);
-    const int ahead = mixed_solve_ahead(s, d, M, b, x, zero_guess, tol, far ? kFar32 : kind32,
-                                        far ? kAimFar : direct, nb, res);
+    const int ahead = mixed_solve_ahead(s, d, M, b, x, zero_guess, tol, far ? kFar32 : kind32, nb, res);
     if (ahead > 0) {
         s.pred_outer = res.outer;
+        if (far) res.outer = (res.outer + 1) / 2;
         return res;
     }
     // one refinement step per host round trip, from x (after the steps enqueued
     // ahead, if any: the last of them is redone with its inner solve)
-    bool xzero = zero_guess && ahead < 0;
-    for (int outer = ahead < 0 ? 0 : K - 1; outer < max_outer; outer++) {
-        // FP64 residual r = b - T x and its preconditioned rms per column
-        if (xzero) {
-            HCHECK(hipMemsetAsync(d.vh, 0, sizeof(double) * M * n, d.stream));
-            launch_residual_rms(d.stream, n, M, b, d.vh, d.vr2, d.alpha, d.red_a, d.scal);
-        } else {
-            matvec(s, d, kOtf64, M, x, d.vh, true, nullptr, nullptr);
-            launch_residual_rms(d.stream, n, M, b, d.vh, d.vr2, d.alpha, d.red_a, d.scal);
-        }
+    bool xzero = zero_guess && ahead < 0, done[2] = {false, false};
+    int step = ahead < 0 ? 0 : K - 1;
+    for (res.outer = far_ahead ? step / 2 : step; res.outer < max_outer; step++) {
+        // FP64 residual r = b - T x and its preconditioned rms per column; in odd steps
+        // of the far field the FP32 one after an inner solve's correction, r -= T d
+        const bool r32 = far && step % 2;
+        if (r32) matvec(s, d, kOtf32, M, d.vd, d.vh, true, nullptr, nullptr);
+        else if (xzero) HCHECK(hipMemsetAsync(d.vh, 0, sizeof(double) * M * n, d.stream));
+        else matvec(s, d, kOtf64, M, x, d.vh, true, nullptr, nullptr);
+        launch_residual_rms(d.stream, n, M, r32 ? d.vr2 : b, d.vh, d.vr2, d.alpha, d.red_a, d.scal);
         HCHECK(hipMemcpyAsync(d.scal_host, d.scal, sizeof(double) * M, hipMemcpyDeviceToHost, d.stream));
         HCHECK(hipStreamSynchronize(d.stream));
-        res.outer = outer + 1;
-        bool conv = true;
-        double tin[2];
-        // (steps enqueued ahead before this one had inner solves too)
-        double accept[2] = {tol, tol};
+        if (!r32) res.outer++;
+        bool conv = true, finite = true;
         for (int m = 0; m < M; m++) {
             const double rms = d.scal_host[m];
-            if (far && outer > 0) {
-                // the far field's inner solves cut the residual by 1e3 each; where one does
-                // not by 10, the residual is at its rounding or the expansions do not fit
-                // this geometry
-                const bool stalled = !(rms < 0.1 * before[m]);
-                if (!stalled) accept[m] = kAimFar.accept * tol;
-                else if (!(rms < tol)) d.inner.bad = true;
-            }
-            conv = conv && rms < accept[m];
+            finite = finite && std::isfinite(rms);
+            if (!r32) done[m] = rms < tol;
+            conv = conv && done[m];
+            // the far field's inner solves cut the residual by 1e3 each; where one does
+            // not by 10, its expansions do not fit this geometry
+            if (far && !(rms < tol) && !(rms < 0.1 * before[m])) d.inner.bad = true;
             before[m] = rms;
         }
-        if (far && d.inner.bad) {
-            far = false;
-            if (!std::isfinite(before[0]) || (M > 1 && !std::isfinite(before[1]))) {
-                HCHECK(hipMemsetAsync(x, 0, sizeof(double) * M * n, d.stream));
-                xzero = true;
-                continue;
-            }
-        }
-        const RefineAim &aim = far ? kAimFar : direct;
-        for (int m = 0; m < M; m++)
-            tin[m] = before[m] < accept[m] ? 1e300 : std::max(aim.eta * before[m], aim.frac * tol);
-        if (conv) {
+        if (!r32 && conv) {
             res.ok = true;
-            s.pred_outer = res.outer;
+            s.pred_outer = step + 1;
             return res;
         }
+        if (far && d.inner.bad) {
+            // the direct inner solves take over, from x or, where it is lost, from nothing
+            far = false;
+            if (!finite) HCHECK(hipMemsetAsync(x, 0, sizeof(double) * M * n, d.stream));
+            xzero = !finite;
+            if (r32 || !finite) continue;
+        }
+        double tin[2];
+        bool reached = true, last = true;  // the target already; with this inner solve
+        for (int m = 0; m < M; m++) {
+            const double eta = far ? kEtaFar : refine_eta();
+            tin[m] = done[m] ? 1e300 : std::max(eta * before[m], frac * tol);
+            reached = reached && before[m] <= tin[m];
+            last = last && (done[m] || tin[m] <= frac * tol);
+        }
+        const int slot = 2 + std::min(step, 13);
+        if (r32 && reached) {
+            s.pred_iters[slot] = -1;
+            continue;
+        }
         // inner FP32 PCG on T delta = r from delta = 0
-        CgResult cr = cg_solve(s, d, far ? kFar32 : kind32, M, d.vr2, d.vd, tin, maxit, true, 0.0, 2 + std::min(outer, 13), nb);
+        CgResult cr = cg_solve(s, d, far ? kFar32 : kind32, M, d.vr2, d.vd, tin, maxit, true, 0.0, slot, nb);
         res.inner += std::max(cr.iters[0], M > 1 ? cr.iters[1] : 0);
         launch_axpy(d.stream, n, M, 1.0, d.vd, x);
         xzero = false;
+        if (far && !r32 && last) {
+            step++;
+            s.pred_iters[2 + std::min(step, 13)] = -1;
+        }
     }
     return res;
 }
@@ -1616,7 +1622,7 @@ size_t device_footprint_estimate(const System &s) {
         b += tmv_sym_part_bytes(s.npol, 2, 64) + sizeof(int2) * nb * (nb + 1) / 2;
     }
     b += (size_t)(s.list_S_P_P.nnz() + s.list_S_P_D.nnz() + 2 * s.list_P_P.nnz() + s.list_P_P_dense.nnz()) * 24;
-    if (s.npol >= kFarInnerFrom)  // tree of the far-field inner solves: basis functions, cells, tables
+    if (s.npol >= far_inner_from(s.n_ipd))  // tree of the far-field inner solves: basis functions, cells, tables
         b += np * (5 * kFarBasis * sizeof(float) + 64) + (size_t(128) << 20);
     return b + (1 << 20);
 }

@@ -29,7 +29,6 @@ constexpr int kFarMaxLevels = 7;
 constexpr int kFarOffsets = 343;  // (dz + 3) 49 + (dy + 3) 7 + dx + 3
 constexpr int kFarMaxTiles = 5;   // tiles of 16 coefficients: orders up to 8
 constexpr int kFarBasis = 64;     // basis functions of degree < p, p <= 8
-constexpr int kFarNearTargets = 8;  // sites per workgroup of the near field
 constexpr int kFarDots = 64;      // y.x partials per column of the matvec
 
 inline int far_coefs(int p) { return ((p + 1) * (p + 1) - 1 + 15) / 16 * 16; }
@@ -61,10 +60,11 @@ template <typename R> struct FarDev {
     R *zero = nullptr;             // [nc] zeros
     R *part = nullptr;             // [nsplit][groups][32][nc]
     // T matvec: sites by leaf
-    int npol = 0, nblocks = 0;
+    int npol = 0, nblocks = 0, near = 16;  // near: sites per workgroup of the near field, 16 or 32
     int *leaf_start = nullptr, *order = nullptr, *leaf = nullptr;  // leaf: of every sorted site
     typename std::conditional<sizeof(R) == 8, double4, float4>::type *pos = nullptr;
     R *a = nullptr;
+    typename std::conditional<sizeof(R) == 8, double4, float4>::type *xs = nullptr;  // [M][npol] the dipoles sorted; w of column 0: a
     const R *rc2 = nullptr;        // damping cutoffs, by polarizable site (row_sweep.h)
     int2 *blocks = nullptr;        // (leaf, first sorted site) of every workgroup of the near field
     R *basis = nullptr;            // [levels - 1][npol][kFarBasis]: B(v / h), degree < p, sorted sites
@@ -80,6 +80,8 @@ template <typename R> struct FarTables {
 };
 template <typename R> const FarTables<R> &far_tables(int p);
 int far_splits(int ngroups);
+// Workgroups of the near field: f.near and (leaf, first sorted site) of each.
+template <typename R> std::vector<int2> far_blocks(FarDev<R> &f, const std::vector<int> &leaf_start);
 
 // Groups of the cells with cnt != 0 of the levels 2 .. levels (host tree).
 void far_group_cells(const FarLevels &lv, const std::vector<int> &cnt, int width, std::vector<int> &cell,

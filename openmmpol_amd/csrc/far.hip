@@ -1,4 +1,5 @@
-// Far field on the matrix cores (far.h).  A T matvec is four launches:
+// Far field on the matrix cores (far.h).  A T matvec is five launches:
+//   k_far_sort    the dipoles in the order of the sorted sites;
 //   k_far_p2m     moments of every occupied cell of every level straight from its
 //                 sites (no translation upwards: a level is one more pass over the
 //                 stored basis functions, 16 KB per 64 sites);
@@ -10,16 +11,15 @@
 //   k_far_field   the sums of the splits, as the expansion of the field (its
 //                 gradient form) of every cell;
 //   k_far_near    per T sites of a leaf: the 27 leaves around it pair by pair, the
-//                 field expansions of all levels (added before the sum over the
-//                 lanes, one basis function per lane), the screened-pair
-//                 corrections, the diagonal and the y.x partial.
+//                 field expansions of all levels, the screened-pair corrections, the
+//                 diagonal and the y.x partial.
 // Every sum has a fixed order.
 //
 // The FP64 form replaces, for orders up to 8, a chain of complex kernels (one
 // thread per coefficient, both factors of every product from LDS, a launch per
-// level up and down, the near field as 27 partial fields): 3.1 -> 0.85 ms per
-// matvec of one dipole set at 120,000 sites, order 8 (near field 0.50, transfer
-// 0.20, moments 0.09).
+// level up and down, the near field as 27 partial fields): 3.1 -> 0.56 ms per
+// matvec of one dipole set at 120,000 sites, order 8 (near field 0.27, transfer
+// 0.20, moments 0.06).
 // What bounds it: the near field's vector ALUs and the transfer's matrix rate.
 #include <hip/hip_runtime.h>
 
@@ -27,7 +27,6 @@
 
 #include "far.h"
 #include "pair_math.h"
-#include "row_sweep.h"
 
 namespace ommp {
 
@@ -287,6 +286,27 @@ __global__ __launch_bounds__(kBlock) void k_far_basis(FarLevels lv, int p, int n
         for (int i = p * p; i < kFarBasis; i++) out[i] = R(0);
 }
 
+// The dipoles in the order of the sorted sites (order given) or already in it: both
+// the moments and the near field then read neighbours as neighbours (gathered there, 64
+// lanes of 24 bytes each, they made the moments of 60,000 sites, two columns in FP32, 74
+// instead of 32 us and the near field 397 instead of 353; this pass takes 5).
+template <typename R>
+__global__ __launch_bounds__(kBlock) void k_far_sort(int npol, const int *__restrict__ order,
+                                                     const R *__restrict__ adamp, const double *__restrict__ x,
+                                                     long xstride, typename V4<R>::t *__restrict__ xs,
+                                                     const CgState *__restrict__ skip, int M) {
+    if (all_done(skip, M)) return;
+    const int t = blockIdx.x * kBlock + threadIdx.x;
+    if (t >= npol) return;
+    const double *v = x + blockIdx.y * xstride + 3L * (order ? order[t] : t);
+    typename V4<R>::t o;
+    o.x = (R)v[0];
+    o.y = (R)v[1];
+    o.z = (R)v[2];
+    o.w = adamp[t];
+    xs[(long)blockIdx.y * npol + t] = o;
+}
+
 // Moments of one cell (blockIdx.x: a place in the groups), added to init where
 // given: sums A_c,i = sum mu_c B_i
 // over its sites, one basis function per lane, then
@@ -298,9 +318,10 @@ constexpr int kP2mThreads = 512, kP2mWaves = kP2mThreads / 64;
 template <typename R, int M>
 __global__ __launch_bounds__(kP2mThreads) void k_far_p2m(FarLevels lv, int p, int nc, int npol, int width,
                                                     const int *__restrict__ gcell, const int *__restrict__ glevel,
-                                                    const int *__restrict__ leaf_start, const int *__restrict__ order,
-                                                    const R *__restrict__ basis, const double *__restrict__ x,
-                                                    long xstride, const R *__restrict__ init,
+                                                    const int *__restrict__ leaf_start,
+                                                    const R *__restrict__ basis,
+                                                    const typename V4<R>::t *__restrict__ xs,
+                                                    const R *__restrict__ init,
                                                     R *__restrict__ mom,
                                                     const CgState *__restrict__ skip) {
     if (all_done(skip, M)) return;
@@ -321,11 +342,13 @@ __global__ __launch_bounds__(kP2mThreads) void k_far_p2m(FarLevels lv, int p, in
 #pragma unroll 8
         for (int t = leaf_start[row] + w; t < t1; t += kP2mWaves) {
             const R b = bas[(long)t * kFarBasis];
-            const long j = 3L * (order ? order[t] : t);
 #pragma unroll
-            for (int m = 0; m < M; m++)
-#pragma unroll
-                for (int c = 0; c < 3; c++) a[m][c] += (R)x[m * xstride + j + c] * b;
+            for (int m = 0; m < M; m++) {
+                const typename V4<R>::t v = xs[(long)m * npol + t];
+                a[m][0] += v.x * b;
+                a[m][1] += v.y * b;
+                a[m][2] += v.z * b;
+            }
         }
     }
 #pragma unroll
@@ -413,47 +436,60 @@ __global__ __launch_bounds__(kBlock) void k_far_field(FarLevels lv, int p, int n
     }
 }
 
-constexpr int kNearTile = 1024;  // sources listed at once
+// T targets of a leaf and its 27 leaves: thread (t, s) meets every (256 / T)-th source
+// from the s-th for target t.  Sources pass through LDS, read there by T lanes at once.
+// Damped pairs (a few per thread, in half of a wave's steps) are left out of the sweep:
+// each thread lists its own within a tile and does them at the tile's end, where the
+// exact argument decides (cutoffs as in row_sweep.h); a full list damps in place.
+//
+// Bound by the vector unit.  One target per thread keeps its data in registers and
+// leaves three sums per thread and column to add up.  With the sources over the threads
+// instead (as the per-target matvec, which sweeps thousands of them) each of 8 targets'
+// sums went over 256 threads: half of the instructions at the 500 sources of a leaf of
+// 29 sites.  120,000 sites FP64, one column: 497 -> 267 us (187 of them vector issue);
+// FP32, two columns: 20,001 sites 72 -> 53, 60,000 sites in leaves of 171: 353 -> 336
+// (292 issue, 37 instructions per pair).
+constexpr int kNearCap = 12;  // listed pairs per thread and tile
+template <typename R> constexpr int kNearTile = sizeof(R) == 8 ? 256 : 512;  // sources in LDS
 
 template <typename R, int M, bool AMOEBA, int T>
 __global__ __launch_bounds__(kBlock) void k_far_near(
     FarLevels lv, int npol, const int2 *__restrict__ blocks, const int *__restrict__ leaf_start,
     const int *__restrict__ order, const typename V4<R>::t *__restrict__ pos, const R *__restrict__ adamp,
-    const R *__restrict__ rc2, const R *__restrict__ basis, const R *__restrict__ grad, const double4 *__restrict__ ps,
-    const double *__restrict__ pa, const double *__restrict__ alpha, const int *__restrict__ pp_ri,
-    const int *__restrict__ pp_ci, const double *__restrict__ pp_f, const double *__restrict__ x, long xstride,
-    double *__restrict__ y, long ystride, int dodiag, double *__restrict__ dotpart,
-    const CgState *__restrict__ skip) {
+    const R *__restrict__ rc2, const typename V4<R>::t *__restrict__ xs, const R *__restrict__ basis,
+    const R *__restrict__ grad, const double4 *__restrict__ ps, const double *__restrict__ pa,
+    const double *__restrict__ alpha, const int *__restrict__ pp_ri, const int *__restrict__ pp_ci,
+    const double *__restrict__ pp_f, const double *__restrict__ x, long xstride, double *__restrict__ y, long ystride,
+    int dodiag, double *__restrict__ dotpart, const CgState *__restrict__ skip) {
     using R4 = typename V4<R>::t;
-    constexpr int C = 3 * M, W = kBlock / 64;
+    constexpr int C = 3 * M, NS = kBlock / T, TILE = kNearTile<R>, NB = kFarBasis / NS;
+    static_assert(T <= 32 && NB >= 1, "whole slices per wave");
     if (all_done(skip, M)) return;
-    __shared__ int s_src[kNearTile];
-    __shared__ RowLds<R, M, T> lds;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    __shared__ R4 s_pos[TILE], s_x[M][TILE];
+    __shared__ unsigned short s_list[kNearCap][kBlock];
+    __shared__ double s_sum[kBlock / 64][T][C], s_dot[T][C];
+    const int tid = threadIdx.x, tt = tid % T, sl = tid / T;
     const int leaf = blocks[blockIdx.x].x, t0 = blocks[blockIdx.x].y;
     const int nl = 1 << lv.levels, lx = leaf & (nl - 1), ly = leaf >> lv.levels & (nl - 1), lz = leaf >> 2 * lv.levels;
     const int nt = min(T, leaf_start[leaf + 1] - t0);
     // targets past the leaf's end repeat the last one; their results are not written
-    auto tgt = [&](int t) { return t0 + min(t, nt - 1); };
-    auto id = [&](int i) { return order[i]; };
-    RowAcc<R, M, T> acc;
+    const int ti = t0 + min(tt, nt - 1), site = order[ti];
+    const R4 pt = pos[ti];
+    const R at = adamp[ti], rc = rc2[site];
+    R f[M][3];
 #pragma unroll
-    for (int t = 0; t < T; t++) row_target(acc, t, pos[tgt(t)], adamp[tgt(t)], rc2[order[tgt(t)]]);
-    // far field of level 2 + w (and 6 + w): one basis function per lane
-    for (int l = 2 + w; l <= lv.levels; l += W) {
+    for (int m = 0; m < M; m++) f[m][0] = f[m][1] = f[m][2] = R(0);
+    // far field of every level: NB basis functions per thread
+    for (int l = 2; l <= lv.levels; l++) {
         const int k = lv.levels - l, ns = 1 << l;
         const long cell = lv.off[l] - lv.off[2] + ((long)(lz >> k) * ns + (ly >> k)) * ns + (lx >> k);
-        const R *g = grad + cell * C * kFarBasis + lane;
-        const R *b = basis + ((long)(l - 2) * npol + t0) * kFarBasis + lane;
-        R gv[C];
+        const R *g = grad + cell * C * kFarBasis + sl * NB;
+        const R *bas = basis + ((long)(l - 2) * npol + ti) * kFarBasis + sl * NB;
 #pragma unroll
-        for (int c = 0; c < C; c++) gv[c] = g[c * kFarBasis];
+        for (int i = 0; i < NB; i++) {
+            const R bv = bas[i];
 #pragma unroll
-        for (int t = 0; t < T; t++) {
-            const R bv = b[min(t, nt - 1) * kFarBasis];
-#pragma unroll
-            for (int c = 0; c < C; c++) acc.f[t][c / 3][c % 3] += bv * gv[c];
+            for (int c = 0; c < C; c++) f[c / 3][c % 3] += bv * g[c * kFarBasis + i];
         }
     }
     // near field: nine runs of sites (three leaves along x each)
@@ -469,45 +505,124 @@ __global__ __launch_bounds__(kBlock) void k_far_near(
         before[r + 1] = before[r] + (in ? leaf_start[row + x1 + 1] - start[r] : 0);
     }
     const int total = before[9];
-    for (int tile = 0; tile < total; tile += kNearTile) {
-        const int cnt = min(kNearTile, total - tile);
+    for (int tile = 0; tile < total; tile += TILE) {
+        const int cnt = min(TILE, total - tile), cntp = (cnt + NS - 1) / NS * NS;
         __syncthreads();
+        for (int q = tid; q < cntp; q += kBlock) {
+            R4 p, v[M];
+            if (q < cnt) {
+                int i = start[0] + tile + q;
 #pragma unroll
-        for (int r = 0; r < 9; r++) {
-            const int lo = max(before[r], tile), hi = min(before[r + 1], tile + cnt);
-            for (int q = lo + tid; q < hi; q += kBlock) s_src[q - tile] = start[r] + q - before[r];
+                for (int r = 1; r < 9; r++)
+                    if (tile + q >= before[r]) i = start[r] + tile + q - before[r];
+                p = pos[i];
+#pragma unroll
+                for (int m = 0; m < M; m++) v[m] = xs[(long)m * npol + i];
+            } else {
+                p.x = p.y = p.z = R(1e15);
+                p.w = R(1);
+#pragma unroll
+                for (int m = 0; m < M; m++) {
+                    v[m].x = v[m].y = v[m].z = R(0);
+                    v[m].w = R(0.39);
+                }
+            }
+            s_pos[q] = p;
+#pragma unroll
+            for (int m = 0; m < M; m++) s_x[m][q] = v[m];
         }
         __syncthreads();
-        R4 pn, vn[M];
-        R an = R(0);
-        int in = 0;
-        auto load = [&](int q) {
-            in = s_src[q];
-            pn = pos[in];
-            an = adamp[in];
-            const long j = 3L * order[in];
-#pragma unroll
-            for (int m = 0; m < M; m++) {
-                vn[m].x = (R)x[m * xstride + j];
-                vn[m].y = (R)x[m * xstride + j + 1];
-                vn[m].z = (R)x[m * xstride + j + 2];
-            }
-        };
-        if (tid < cnt) load(tid);
-        for (int q = tid; q < cnt; q += kBlock) {
-            const R4 p = pn;
-            const R a = an;
-            const int i = in;
+        int n = 0;
+#pragma unroll 2
+        for (int q = sl; q < cntp; q += NS) {
+            const R4 p = s_pos[q];
             R4 v[M];
 #pragma unroll
-            for (int m = 0; m < M; m++) v[m] = vn[m];
-            if (q + kBlock < cnt) load(q + kBlock);  // the next source while this one is used
-            row_source<AMOEBA>(acc, lds, w, i, p, a, v, pos, adamp, tgt);
+            for (int m = 0; m < M; m++) v[m] = s_x[m][q];
+            R dx, dy, dz, k2, k3;
+            const bool in = pair_bare<R>(pt, p, dx, dy, dz, k2, k3) < rc;  // the target itself among them
+            if (__ballot(in)) {
+                if (in) {
+                    if (n < kNearCap) {
+                        s_list[n++][tid] = (unsigned short)q;
+                        k2 = k3 = R(0);
+                    } else {
+                        R arg;
+                        bool near;
+                        pair_geom<R, AMOEBA>(pt, at, p, v[0].w, dx, dy, dz, k2, k3, arg, near);
+                        pair_damp<R, AMOEBA>(arg, near, k2, k3);
+                    }
+                }
+            }
+            pair_accum<R, M>(f, v, dx, dy, dz, k2, k3);
+        }
+        for (int e = 0; __ballot(e < n); e++) {
+            if (e >= n) continue;
+            const int q = s_list[e][tid];
+            const R4 p = s_pos[q];
+            R4 v[M];
+#pragma unroll
+            for (int m = 0; m < M; m++) v[m] = s_x[m][q];
+            R dx, dy, dz, k2, k3, arg;
+            bool near;
+            pair_geom<R, AMOEBA>(pt, at, p, v[0].w, dx, dy, dz, k2, k3, arg, near);  // 0 for itself
+            pair_damp<R, AMOEBA>(arg, near, k2, k3);
+            pair_accum<R, M>(f, v, dx, dy, dz, k2, k3);
         }
     }
-    row_finish<AMOEBA>(acc, lds, w, pos, adamp, x, xstride, ps, pa, pp_ri, pp_ci, pp_f, tgt, id);
-    row_store(lds, nt, alpha, x, xstride, y, ystride, dodiag != 0, dotpart ? dotpart + blockIdx.x : nullptr,
-              (long)gridDim.x, tgt, id);
+    // screened pairs (FP64), then the sum over the slices
+    double sum[C];
+#pragma unroll
+    for (int c = 0; c < C; c++) sum[c] = -(double)f[c / 3][c % 3];
+    const int k1 = pp_ri[site + 1];
+    for (int k = pp_ri[site] + sl; k < k1; k += NS) {
+        const int i = pp_ci[k];
+        const double fk = pp_f[k];
+        const double4 qj = ps[site], pi = ps[i];
+        const double dx = qj.x - pi.x, dy = qj.y - pi.y, dz = qj.z - pi.z;
+        const double r2 = dx * dx + dy * dy + dz * dz;
+        double k2, k3;
+        dip_kernel<double, AMOEBA>(r2, rsqrt(r2), pi.w, qj.w, pa[i], pa[site], k2, k3);
+#pragma unroll
+        for (int m = 0; m < M; m++) {
+            const double *xi = x + m * xstride + 3L * i;
+            const double c = k3 * (xi[0] * dx + xi[1] * dy + xi[2] * dz);
+            sum[3 * m + 0] += fk * (c * dx - k2 * xi[0]);
+            sum[3 * m + 1] += fk * (c * dy - k2 * xi[1]);
+            sum[3 * m + 2] += fk * (c * dz - k2 * xi[2]);
+        }
+    }
+#pragma unroll
+    for (int mask = T; mask < 64; mask <<= 1)
+#pragma unroll
+        for (int c = 0; c < C; c++) sum[c] += __shfl_xor(sum[c], mask, 64);
+    if ((tid & 63) < T) {
+#pragma unroll
+        for (int c = 0; c < C; c++) s_sum[tid >> 6][tt][c] = sum[c];
+    }
+    __syncthreads();
+    if (tid < T * C) {
+        const int t = tid / C, c = tid % C;
+        double out = 0.0;
+        if (t < nt) {
+            const int j = order[t0 + t];
+            const double xj = x[c / 3 * xstride + 3L * j + c % 3];
+            double v = s_sum[0][t][c];
+#pragma unroll
+            for (int q = 1; q < kBlock / 64; q++) v += s_sum[q][t][c];
+            if (dodiag) v += xj * (1.0 / alpha[j]);
+            y[c / 3 * ystride + 3L * j + c % 3] = v;
+            out = v * xj;
+        }
+        s_dot[t][c] = out;
+    }
+    if (!dotpart) return;
+    __syncthreads();
+    if (tid < M) {
+        double d = 0.0;
+        for (int t = 0; t < T; t++) d += (s_dot[t][3 * tid] + s_dot[t][3 * tid + 1]) + s_dot[t][3 * tid + 2];
+        dotpart[tid * (long)gridDim.x + blockIdx.x] = d;
+    }
 }
 
 // The workgroups' y.x partials of column blockIdx.y as kFarDots sums, in a fixed
@@ -522,6 +637,13 @@ __global__ __launch_bounds__(kBlock) void k_far_dots(int n, const double *__rest
     for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += kFarDots * kBlock) v += dots[(long)blockIdx.y * n + i];
     v = block_sum_all(v, sh);
     if (threadIdx.x == 0) out[blockIdx.y * kFarDots + blockIdx.x] = v;
+}
+
+template <typename R>
+void sort(hipStream_t st, const FarDev<R> &f, const int *order, int M, const double *x, long xs, const CgState *skip) {
+    hipLaunchKernelGGL(k_far_sort<R>, dim3((unsigned)((f.npol + kBlock - 1) / kBlock), M), dim3(kBlock), 0, st, f.npol,
+                       order, f.a, x, xs, f.xs, skip, M);
+    HIP_CHECK(hipGetLastError());
 }
 
 template <typename R, int M, bool MONO>
@@ -547,11 +669,11 @@ template <typename R, int M, bool AMOEBA>
 void matvec_t(hipStream_t st, const FarDev<R> &f, const int *cnt, const double4 *ps64, const double *pa64,
               const double *alpha, const CsrDev &pp, const double *x, long xs, double *y, long ys, bool dodiag,
               double *dotpart, const CgState *skip) {
-    constexpr int T = kFarNearTargets;
     const int places = f.groups.n * f.groups.width;
+    sort<R>(st, f, f.order, M, x, xs, skip);
     if (f.groups.n > 0) {
         hipLaunchKernelGGL((k_far_p2m<R, M>), dim3(places), dim3(kP2mThreads), 0, st, f.lv, f.p, f.nc, f.npol,
-                           f.groups.width, f.groups.cell, f.groups.level, f.leaf_start, f.order, f.basis, x, xs,
+                           f.groups.width, f.groups.cell, f.groups.level, f.leaf_start, f.basis, f.xs,
                            (const R *)nullptr, f.mom, skip);
         HIP_CHECK(hipGetLastError());
         m2l<R, M, false>(st, f, f.groups, cnt, f.mom, skip);
@@ -559,9 +681,13 @@ void matvec_t(hipStream_t st, const FarDev<R> &f, const int *cnt, const double4 
                            f.groups.n, f.groups.width, f.groups.cell, f.groups.level, f.part, f.grad, skip);
         HIP_CHECK(hipGetLastError());
     }
-    hipLaunchKernelGGL((k_far_near<R, M, AMOEBA, T>), dim3(f.nblocks), dim3(kBlock), 0, st, f.lv, f.npol, f.blocks,
-                       f.leaf_start, f.order, f.pos, f.a, f.rc2, f.basis, f.grad, ps64, pa64, alpha, pp.ri, pp.ci, pp.f, x,
-                       xs, y, ys, (int)dodiag, dotpart ? f.dots : nullptr, skip);
+    auto near = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(f.nblocks), dim3(kBlock), 0, st, f.lv, f.npol, f.blocks, f.leaf_start, f.order,
+                           f.pos, f.a, f.rc2, f.xs, f.basis, f.grad, ps64, pa64, alpha, pp.ri, pp.ci, pp.f, x, xs, y,
+                           ys, (int)dodiag, dotpart ? f.dots : nullptr, skip);
+    };
+    if (f.near == 16) near(k_far_near<R, M, AMOEBA, 16>);
+    else near(k_far_near<R, M, AMOEBA, 32>);
     if (dotpart)
         hipLaunchKernelGGL(k_far_dots, dim3(kFarDots, M), dim3(kBlock), 0, st, f.nblocks, f.dots, dotpart, skip, M);
     HIP_CHECK(hipGetLastError());
@@ -582,10 +708,12 @@ void far_launch_locals(hipStream_t st, const FarDev<double> &f, const FarGroups 
     const double *mom = with_static && !dip ? f.mom_static : f.mom;
     hipLaunchKernelGGL(k_far_zero, dim3((unsigned)((nl + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, nl,
                        loc + f.lv.off[2] * (f.p + 1) * (f.p + 1));
-    if (dip && src.n > 0)
+    if (dip && src.n > 0) {
+        sort<double>(st, f, nullptr, 1, dip, 0L, nullptr);
         hipLaunchKernelGGL((k_far_p2m<double, 1>), dim3(src.n * src.width), dim3(kP2mThreads), 0, st, f.lv, f.p, f.nc,
-                           f.npol, src.width, src.cell, src.level, f.leaf_start, (const int *)nullptr, f.basis, dip,
-                           0L, with_static ? f.mom_static : nullptr, f.mom, (const CgState *)nullptr);
+                           f.npol, src.width, src.cell, src.level, f.leaf_start, f.basis, f.xs,
+                           with_static ? f.mom_static : nullptr, f.mom, (const CgState *)nullptr);
+    }
     HIP_CHECK(hipGetLastError());
     if (tgt.n == 0) return;
     if (with_static) m2l<double, 1, true>(st, f, tgt, cnt_src, mom, nullptr);

@@ -112,6 +112,20 @@ template <typename R> const FarTables<R> &far_tables(int p) {
 template const FarTables<double> &far_tables<double>(int p);
 template const FarTables<float> &far_tables<float>(int p);
 
+template <typename R> std::vector<int2> far_blocks(FarDev<R> &f, const std::vector<int> &leaf_start) {
+    int occupied = 0;
+    for (size_t k = 0; k + 1 < leaf_start.size(); k++) occupied += leaf_start[k + 1] > leaf_start[k];
+    // 32 sites share a workgroup's sources where most leaves have several such groups
+    f.near = f.npol > 96L * occupied ? 32 : 16;
+    std::vector<int2> blocks;
+    for (int k = 0; k + 1 < (int)leaf_start.size(); k++)
+        for (int t = leaf_start[k]; t < leaf_start[k + 1]; t += f.near) blocks.push_back(make_int2(k, t));
+    f.nblocks = (int)blocks.size();
+    return blocks;
+}
+template std::vector<int2> far_blocks<double>(FarDev<double> &, const std::vector<int> &);
+template std::vector<int2> far_blocks<float>(FarDev<float> &, const std::vector<int> &);
+
 // Enough workgroups to fill the chip when a tree has few groups of cells.
 int far_splits(int ngroups) {
     const int s = (1024 + ngroups - 1) / std::max(ngroups, 1);

@@ -839,19 +839,19 @@ void launch_cg_init2(hipStream_t st, int M, const double *red, int nred, CgState
 }
 
 // One refinement step's decision on the device: the FP64 residual rms of each
-// column (rms[m]) marks the column converged (out[m].done) when below tol; a
-// converged column stays converged (later residuals of it are not computed).
+// column (rms[m]) marks the column converged (out[m].done) when below tol (check: not
+// the FP32 residual between two far-field inner solves); a converged column stays converged (later residuals of it are not computed).
 // The inner solve's tolerances go to inner_tol[0..1] (max(eta rms, frac tol)),
 // its small-step thresholds inner_tol[2..3] = 0.
 __global__ void k_refine_decide(int M, const double *__restrict__ rms, CgState *__restrict__ out, double tol,
-                                double eta, double frac, double *__restrict__ inner_tol, int outer) {
+                                double eta, double frac, double *__restrict__ inner_tol, int outer, int check) {
     if (threadIdx.x != 0) return;
     for (int m = 0; m < M; m++) {
         if (outer == 0) {
             out[m].done = 0;
             out[m].status = 2;
         }
-        if (!out[m].done) {
+        if (!out[m].done && check) {
             out[m].rms = rms[m];
             out[m].iters = outer + 1;
             if (rms[m] < tol) {
@@ -859,7 +859,7 @@ __global__ void k_refine_decide(int M, const double *__restrict__ rms, CgState *
                 out[m].status = 0;
             }
         }
-        inner_tol[m] = out[m].done ? 0.0 : fmax(eta * out[m].rms, frac * tol);
+        inner_tol[m] = out[m].done ? 0.0 : fmax(eta * rms[m], frac * tol);
         inner_tol[2 + m] = 0.0;
     }
     if (M == 1) {
@@ -869,8 +869,8 @@ __global__ void k_refine_decide(int M, const double *__restrict__ rms, CgState *
 }
 
 void launch_refine_decide(hipStream_t st, int M, const double *rms, CgState *out, double tol, double eta,
-                          double frac, double *inner_tol, int outer) {
-    hipLaunchKernelGGL(k_refine_decide, dim3(1), dim3(64), 0, st, M, rms, out, tol, eta, frac, inner_tol, outer);
+                          double frac, double *inner_tol, int outer, bool check) {
+    hipLaunchKernelGGL(k_refine_decide, dim3(1), dim3(64), 0, st, M, rms, out, tol, eta, frac, inner_tol, outer, (int)check);
     HIP_CHECK(hipGetLastError());
 }
 
@@ -1159,8 +1159,9 @@ void launch_axpy(hipStream_t st, long n, int M, double a, const double *x, doubl
 }
 
 // r = b - tx; partial sums of alpha r^2 (the CG convergence norm)
-__global__ __launch_bounds__(kBlock) void k_resid(long n, const double *__restrict__ b, const double *__restrict__ tx,
-                                                  double *__restrict__ r, const double *__restrict__ alpha,
+// (b may be r)
+__global__ __launch_bounds__(kBlock) void k_resid(long n, const double *b, const double *__restrict__ tx, double *r,
+                                                  const double *__restrict__ alpha,
                                                   double *__restrict__ red) {
     __shared__ double sh[4];
     const int m = blockIdx.y;

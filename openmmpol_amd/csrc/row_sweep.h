@@ -1,6 +1,5 @@
 // Sweep of T targets over sources that are spread over the 256 threads of a
-// workgroup: the inner part of the per-target T matvec (tmv_rows.hip) and of the
-// near field of the far-field matvec (far.hip).
+// workgroup: the inner part of the per-target T matvec (tmv_rows.hip).
 //
 // A pair is compared with the target's cutoff rc2 (beyond it no pair of the target is
 // damped, whatever the source), one compare per pair; damping acts within a few
