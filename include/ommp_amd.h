@@ -18,8 +18,9 @@ extern "C" {
 
 /* Precision of the T matvec inside the solvers.
    FP64  : every step in FP64, reference algorithm and iterate sequence.
-   MIXED : FP32 T matvec (pair arithmetic) inside an FP64 iterative-refinement
-           loop; the residual r = E - T mu, CG dot products and step lengths,
+   MIXED : FP32 T matvec (pair arithmetic; for large systems with the far field
+           by multipole expansions) inside an FP64 iterative-refinement loop; the
+           residual r = E - T mu (direct sum), CG dot products and step lengths,
            the dipole accumulation and the energy sum are FP64.  D and P sets
            are solved together (two right-hand sides per matvec). */
 #define OMMP_AMD_PREC_FP64 0
