@@ -699,13 +699,13 @@ void ensure_fmm(System &s, DeviceState &d) {
 // solves with two columns: 14,000 sites (water) 2.66 / 3.06, 15,000 3.70 / 4.43, 60,000
 // 24.6 / 54.8; with one column 24,000 3.2 / 4.3; gradient steps with their trees: 20,001
 // 7.5 / 9.1.  With one FP64 residual more instead of the FP32 ones 12,000 sites took
-// 3.25 / 3.29, 10,000 3.0 / 2.8, one column at 15,000 2.04 / 1.94: used from 13,000 and
-// 18,000.
+// 3.25 / 3.29, 10,000 3.0 / 2.8; with them 11,000 2.95 / 2.88, one column at 15,000 1.98
+// / 2.0 and at 17,000 2.2 / 2.4: used from 13,000 and 16,000.
 // Leaves of 24 sites and more in the mean: at 60,000 sites 29 and 171 an occupied leaf
 // take 363 and 387 us, the larger ones with an error of 2.6e-5 instead of 1.4e-4, which
 // saves iterations (solve 33.1 and 28.0 ms).
 constexpr int kFarInnerOrder = 8, kFarInnerOccupancy = 24;
-int far_inner_from(int M) { return M == 2 ? 13000 : 18000; }
+int far_inner_from(int M) { return M == 2 ? 13000 : 16000; }
 
 // Octree over the polarizable sites for M columns: leaves of at least
 // kFarInnerOccupancy sites in the mean of the occupied ones.
