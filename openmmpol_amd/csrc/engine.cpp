@@ -434,7 +434,8 @@ void upload_sites(System &s, DeviceState &d) {
     for (int p = 0; p < s.npol; p++) {
         const double ww = w[s.polar_mm[p]] * wmin;
         auto cut = [&](double x) {
-            const double r = s.amoeba ? std::cbrt(x / (amin * ww * ww * ww)) : 1.0 / ww;
+            const double aw3 = amin * ww * ww * ww;  // not positive (or 0 inf): no bound on the distance
+            const double r = !s.amoeba ? 1.0 / ww : (aw3 > 0.0 ? std::cbrt(x / aw3) : inf);
             return std::max(r * r * (1.0 + 1e-4), 1e-3);
         };
         rc[p] = cut(42.0);

@@ -34,8 +34,10 @@ def chain(n, amoeba, seed=5):
 
 def pair(spec):
     from openmmpol_amd import OMMPSystem
+    td = spec.get("td", np.full(len(spec["pol"]), 0.39))
     s = OMMPSystem.from_arrays(spec["amoeba"], spec["cmm"], spec["q"], spec["pol"], spec["bonds_ri"],
-                               spec["bonds_ci"], pgroup=spec["pgroup"] if spec["amoeba"] else None)
+                               spec["bonds_ci"], pgroup=spec["pgroup"] if spec["amoeba"] else None,
+                               thole_a=spec.get("td"))
     q = spec["q"].copy()
     if spec["amoeba"]:
         q[:, 4:10] /= 3.0
@@ -45,7 +47,7 @@ def pair(spec):
     n = len(spec["pol"])
     o = oa.OracleSystem(dict(nmm=n, amoeba=spec["amoeba"], cmm=spec["cmm"], q=q, pol=spec["pol"],
                              adj_ri=spec["bonds_ri"], adj_ci=spec["bonds_ci"], grp=spec["pgroup"],
-                             td=np.full(n, 0.39), scales=np.array(scales, dtype=float),
+                             td=td, scales=np.array(scales, dtype=float),
                              thole_scale=0.0 if spec["amoeba"] else 2.5874))
     return s, o
 
@@ -87,6 +89,28 @@ def test_damping_cutoff(n, kinds, scale, amoeba):
             bar = 1e-12 if kind.endswith("64") else 3e-4
             assert np.abs(y - want[:ncols]).max() <= bar * np.abs(want).max(), (kind, ncols)
         assert np.array_equal(s.tmatvec(x, kind=kind)[0], y)
+    s.terminate()
+
+
+@pytest.mark.parametrize("a", [0.0, -0.4])
+@pytest.mark.parametrize("n", [300, 3001])
+def test_damping_factor_not_positive(n, a):
+    """AMOEBA damping factors that bound no distance: 0 damps every pair of its site
+    to nothing, a negative one lets its pairs grow with the distance (per-target sweep
+    alone: they overflow beyond some 20 bohr).  FP64 against the oracle, 1e-12 of the largest component (3,001 terms of rounding 1.1e-16,
+    and of an exponential's argument of up to ~280: 280 eps = 6e-14)."""
+    spec = chain(n, True)
+    spec["td"] = np.full(n, 0.39)
+    spec["td"][n // 2] = a
+    if a < 0.0:
+        spec["cmm"] = spec["cmm"] * (0.35 if n == 300 else 0.2)
+    s, o = pair(spec)
+    x = np.random.default_rng(n).normal(0.0, 0.05, size=(2, n, 3))
+    want = np.stack([o.tmatvec(x[0]), o.tmatvec(x[1])])
+    assert np.isfinite(want).all()
+    for kind in ("plain64", "sym64")[:1 if a < 0.0 else 2]:
+        y, _ = s.tmatvec(x, kind=kind)
+        assert np.abs(y - want).max() <= 1e-12 * np.abs(want).max(), kind
     s.terminate()
 
 
