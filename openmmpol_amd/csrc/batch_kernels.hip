@@ -35,6 +35,11 @@ __device__ __forceinline__ bool mv_active(const BCol &c, int use_p) {
 
 // Grouped on-the-fly pair kernel body: one target per thread, sources of one
 // split staged through LDS, MM columns cidx[] (per-pair arithmetic of pair_math.h).
+// The damping argument of every pair is formed with its geometry: at these sizes most
+// pairs of sources have a damped pair in some lane of the wave, and deciding by the
+// sites' cutoffs first, as the pair-once sweep does, formed their geometry twice (SCF
+// sequences of two systems of 500 and 700 sites 6.3 -> 6.7 ms, of four of 1,000 to
+// 4,000 10.1 -> 10.5; one field of 5,004 sites 2.04 -> 2.17).
 template <typename R, int MM, bool AMOEBA>
 __device__ __forceinline__ void bpairs_body(const BSeg &S, const int4 w, const double *__restrict__ xin,
                                             const int (&cidx)[MM]) {
@@ -49,11 +54,10 @@ __device__ __forceinline__ void bpairs_body(const BSeg &S, const int4 w, const d
     const int j = w.y * kBlock + tid;
     const bool valid = j < npol;
     R4 pj;
-    R aj, rj = R(0);
+    R aj;
     if (valid) {
         pj = site[j];
         aj = adamp[j];
-        rj = SegSites<R>::cut(S)[j];
     } else {
         pj.x = pj.y = pj.z = R(0);
         pj.w = R(1);
@@ -106,18 +110,13 @@ __device__ __forceinline__ void bpairs_body(const BSeg &S, const int4 w, const d
                 xa[m] = s_x[m][k];
                 xb[m] = s_x[m][k + 1];
             }
-            // the self pair is inside its site's cutoff: guarded in the branch
-            const R4 pa = s_pos[k], pb = s_pos[k + 1];
-            R dxa, dya, dza, k2a, k3a, dxb, dyb, dzb, k2b, k3b;
-            const R r2a = pair_bare<R>(pj, pa, dxa, dya, dza, k2a, k3a);
-            const R r2b = pair_bare<R>(pj, pb, dxb, dyb, dzb, k2b, k3b);
-            if (__ballot(r2a < rj || r2b < rj)) {
-                R arg;
-                bool near;
-                pair_geom<R, AMOEBA>(pj, aj, pa, xa[0].w, dxa, dya, dza, k2a, k3a, arg, near);
-                pair_damp<R, AMOEBA>(arg, near, k2a, k3a);
-                pair_geom<R, AMOEBA>(pj, aj, pb, xb[0].w, dxb, dyb, dzb, k2b, k3b, arg, near);
-                pair_damp<R, AMOEBA>(arg, near, k2b, k3b);
+            R dxa, dya, dza, k2a, k3a, arga, dxb, dyb, dzb, k2b, k3b, argb;
+            bool neara, nearb;
+            pair_geom<R, AMOEBA>(pj, aj, s_pos[k], xa[0].w, dxa, dya, dza, k2a, k3a, arga, neara);
+            pair_geom<R, AMOEBA>(pj, aj, s_pos[k + 1], xb[0].w, dxb, dyb, dzb, k2b, k3b, argb, nearb);
+            if (__ballot(neara || nearb)) {
+                pair_damp<R, AMOEBA>(arga, neara, k2a, k3a);
+                pair_damp<R, AMOEBA>(argb, nearb, k2b, k3b);
             }
             pair_accum<R, MM>(acc, xa, dxa, dya, dza, k2a, k3a);
             pair_accum<R, MM>(acc, xb, dxb, dyb, dzb, k2b, k3b);
