@@ -97,7 +97,7 @@ __device__ __forceinline__ void row_source(RowAcc<R, M, T> &a, RowLds<R, M, T> &
         if (T < kRowListT) {
             if (mask) {
                 pair_geom<R, AMOEBA>(pt, a.a[t], p, pa, dx, dy, dz, k2, k3, arg, near);
-                pair_damp<R, AMOEBA>(arg, near, k2, k3);
+                if (__ballot(near)) pair_damp<R, AMOEBA>(arg, near, k2, k3);
             }
         } else if (mask) {
             const int c = __popcll(mask);
@@ -110,7 +110,7 @@ __device__ __forceinline__ void row_source(RowAcc<R, M, T> &a, RowLds<R, M, T> &
                 k3 = in ? R(0) : k3;
             } else {
                 pair_geom<R, AMOEBA>(site[tgt(t)], adamp[tgt(t)], site[i], adamp[i], dx, dy, dz, k2, k3, arg, near);
-                pair_damp<R, AMOEBA>(arg, near, k2, k3);
+                if (__ballot(near)) pair_damp<R, AMOEBA>(arg, near, k2, k3);
             }
         }
         pair_accum<R, M>(a.f[t], v, dx, dy, dz, k2, k3);
