@@ -247,18 +247,18 @@ __global__ __launch_bounds__(kSymBlock) void k_gpol_dd_sym(int npol, const int2 
     double acc[3] = {0.0, 0.0, 0.0};
     __syncthreads();
     double jown[3] = {0.0, 0.0, 0.0};  // diagonal: the source-side sum of this thread's site
-    const bool diag = I == J;
-    const int phases = diag ? kSymDiagPhases : kSymWaves;
-#pragma unroll 1
-    for (int ph = 0; ph < phases; ph++) {
+    // one phase: a diagonal block pair's, or sub-tile ph of J off the diagonal, whose 64
+    // steps then have fixed bounds and no test (as in k_rhs_sym)
+    auto phase = [&](int ph, auto on_diag) {
+        constexpr bool D = decltype(on_diag)::value;
         int k = ph, s0 = 0, ns = 64;
-        if (diag) sym_diag_phase(w, ph, k, s0, ns);
-        const bool half = diag && ph == 0;  // its last step meets every pair twice
+        if (D) sym_diag_phase(w, ph, k, s0, ns);
+        const bool half = D && ph == 0;  // its last step meets every pair twice
         double jacc[3] = {0.0, 0.0, 0.0};
-        for (int st = s0; st < s0 + ns; st++) {
+        for (int st = D ? s0 : 0; st < (D ? s0 + ns : 64); st++) {
             double gx, gy, gz;
             term(k * 64 + ((l + st) & 63), gx, gy, gz);
-            if (half && st == 32 && l >= 32) gx = gy = gz = 0.0;
+            if (D && half && st == 32 && l >= 32) gx = gy = gz = 0.0;
             acc[0] += gx;
             acc[1] += gy;
             acc[2] += gz;
@@ -269,9 +269,9 @@ __global__ __launch_bounds__(kSymBlock) void k_gpol_dd_sym(int npol, const int2 
             for (int c = 0; c < 3; c++) jacc[c] = lane_next(jacc[c]);
         }
 #pragma unroll
-        for (int c = 0; c < 3; c++) s_acc[w][c][(l + s0 + ns) & 63] = jacc[c];
+        for (int c = 0; c < 3; c++) s_acc[w][c][D ? (l + s0 + ns) & 63 : l] = jacc[c];
         __syncthreads();
-        if (diag) {
+        if (D) {
 #pragma unroll
             for (int c = 0; c < 3; c++) jown[c] += s_acc[(w - ph) & 3][c][l];
         } else if (tid < 3 * 64) {
@@ -282,11 +282,18 @@ __global__ __launch_bounds__(kSymBlock) void k_gpol_dd_sym(int npol, const int2 
             part_j[(p * 3 + c) * kSymBlock + k * 64 + jl] = sum;
         }
         __syncthreads();
+    };
+    if (I == J) {
+#pragma unroll 1
+        for (int ph = 0; ph < kSymDiagPhases; ph++) phase(ph, std::true_type{});
+    } else {
+#pragma unroll 1
+        for (int ph = 0; ph < kSymWaves; ph++) phase(ph, std::false_type{});
     }
 #pragma unroll
     for (int c = 0; c < 3; c++) {
         part_i[(p * 3 + c) * kSymBlock + tid] = acc[c];
-        if (diag) part_j[(p * 3 + c) * kSymBlock + tid] = jown[c];
+        if (I == J) part_j[(p * 3 + c) * kSymBlock + tid] = jown[c];
     }
 }
 

@@ -25,6 +25,8 @@
 // direction.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "device.h"
 #include "pair_math.h"
 #include "tmv_sym.h"
@@ -164,22 +166,23 @@ __global__ __launch_bounds__(kSymBlock) void k_rhs_sym(int npol, const int2 *__r
     double acc[3] = {0.0, 0.0, 0.0};
     __syncthreads();
     double jown[3] = {0.0, 0.0, 0.0};  // diagonal: the source-side sum of this thread's site
-    const bool diag = I == J;
-    const int phases = diag ? kSymDiagPhases : kSymWaves;
-#pragma unroll 1
-    for (int ph = 0; ph < phases; ph++) {
+    // one phase: a diagonal block pair's, or sub-tile ph of J off the diagonal, whose 64
+    // steps then have fixed bounds and no test (one loop for both: 15,000 sites 393
+    // instead of 378 us per sweep, 60,000 5,750 instead of 5,370)
+    auto phase = [&](int ph, auto on_diag) {
+        constexpr bool D = decltype(on_diag)::value;
         int k = ph, s0 = 0, n = 64;
-        if (diag) sym_diag_phase(w, ph, k, s0, n);
-        const bool half = diag && ph == 0;  // its last step meets every pair twice
+        if (D) sym_diag_phase(w, ph, k, s0, n);
+        const bool half = D && ph == 0;  // its last step meets every pair twice
         double jacc[3] = {0.0, 0.0, 0.0};
-        for (int s = s0; s < s0 + n; s++) {
+        for (int s = D ? s0 : 0; s < (D ? s0 + n : 64); s++) {
             const int js = k * 64 + ((l + s) & 63);
             double4 psrc;
             double q[2 * NQ];
             load_src(js, psrc, q);
             double dx, dy, dz, k2, k3, k4;
             rhs_geom<AMOEBA>(pt, at, psrc, q[KA], dx, dy, dz, k2, k3, k4);
-            if (half && s == 32 && l >= 32) k2 = k3 = k4 = 0.0;
+            if (D && half && s == 32 && l >= 32) k2 = k3 = k4 = 0.0;
             const double k3t = 3.0 * k3, k3s = 6.0 * k3, k4f = 15.0 * k4;
             rhs_accum<AMOEBA>(q, dx, dy, dz, k2, k3t, k3s, k4f, acc);
             // the field at the source of this lane's target, d reversed
@@ -188,9 +191,9 @@ __global__ __launch_bounds__(kSymBlock) void k_rhs_sym(int npol, const int2 *__r
             for (int c = 0; c < 3; c++) jacc[c] = lane_next(jacc[c]);
         }
 #pragma unroll
-        for (int c = 0; c < 3; c++) s_acc[w][c][(l + s0 + n) & 63] = jacc[c];
+        for (int c = 0; c < 3; c++) s_acc[w][c][D ? (l + s0 + n) & 63 : l] = jacc[c];
         __syncthreads();
-        if (diag) {
+        if (D) {
 #pragma unroll
             for (int c = 0; c < 3; c++) jown[c] += s_acc[(w - ph) & 3][c][l];
         } else if (tid < 3 * 64) {
@@ -202,11 +205,18 @@ __global__ __launch_bounds__(kSymBlock) void k_rhs_sym(int npol, const int2 *__r
             part_j[(p * 3 + c) * kSymBlock + k * 64 + jl] = sum;
         }
         __syncthreads();
+    };
+    if (I == J) {
+#pragma unroll 1
+        for (int ph = 0; ph < kSymDiagPhases; ph++) phase(ph, std::true_type{});
+    } else {
+#pragma unroll 1
+        for (int ph = 0; ph < kSymWaves; ph++) phase(ph, std::false_type{});
     }
 #pragma unroll
     for (int c = 0; c < 3; c++) {
         part_i[(p * 3 + c) * kSymBlock + tid] = acc[c];
-        if (diag) part_j[(p * 3 + c) * kSymBlock + tid] = jown[c];
+        if (I == J) part_j[(p * 3 + c) * kSymBlock + tid] = jown[c];
     }
 }
 
