@@ -701,7 +701,8 @@ def main():
     value = args.steps / mixed["elapsed"]
     calls, ms = mixed["stats"]["otf32"]
     avg_ms = ms / max(calls, 1)
-    # at 15,000 sites both pair kernels are the pair-once sweep k_tmv_sym
+    # at 15,000 sites the direct FP32 sweep (the residuals between two far-field inner
+    # solves) is the pair-once sweep k_tmv_sym
     flops = sym_pair_flops(n, 2)
     achieved = flops / (avg_ms * 1e-3) / 1e12 if calls else None
     # the rate non-packed vector FMAs reach on this device (the build emits no
@@ -745,7 +746,8 @@ def main():
                                 "pair-once count (each unordered pair once, m = 2 columns)",
                      "flop_formula": "N(N-1)/2*(29+36m)",
                      "kernel": "k_tmv_sym<float,2,AMOEBA> (on-the-fly FP32 pair kernel, each unordered pair "
-                               "evaluated once)",
+                               "evaluated once; in the step it forms the FP32 residuals between the far-field "
+                               "inner solves)",
                      "achieved": achieved, "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / PEAK_FP32_TFLOPS if achieved else None,
                      "traffic": profile_traffic("k_tmv_sym<float,2,AMOEBA>"),

@@ -133,8 +133,10 @@ double ommp_amd_block_tmatvec(OMMP_SYSTEM_PRT s, int32_t ncols, const double *x,
    stream launch is bracketed by HIP events.  stats receives, per class
    k = 0 on-the-fly FP64, 1 on-the-fly FP32, 2 packed FP32, 3 packed FP64,
    4 static field, 5 geometric-gradient pair sweeps: stats[2k] = launches,
-   stats[2k+1] = total milliseconds.  stats must hold 12 entries; reset clears
-   the counters. */
+   stats[2k+1] = total milliseconds.  The far-field product of large mixed solves
+   is in none of them: class 1 is the direct FP32 sweep alone, there the residuals
+   between two inner solves.  stats must hold 12 entries; reset clears the
+   counters. */
 void ommp_amd_profile_kernels(OMMP_SYSTEM_PRT s, bool enable);
 /* Same, bracketing only every `every`-th launch of each class (each bracketed
    launch costs a few microseconds of idle GPU for the two event records);

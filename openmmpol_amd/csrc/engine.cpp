@@ -886,11 +886,9 @@ void matvec(System &s, DeviceState &d, int kind, int M, const double *x, double 
                               d.pp, x, n, y, n, dodiag, dotpart, reinterpret_cast<const int *>(skip));
         return;
     }
-    if (kind == kFar32) {
-        const int pi = prof_begin(d, kOtf32);
+    if (kind == kFar32) {  // a chain of kernels over fewer pairs: in no class of the statistics
         far_launch_matvec(d.stream, d.inner.far, s.amoeba, M, d.inner.cnt, d.ps64, d.pa64, d.alpha, d.pp, x, n, y, n,
                           dodiag, dotpart, skip);
-        if (pi >= 0) HCHECK(hipEventRecord(d.prof_pool[2 * pi + 1], d.stream));
         return;
     }
     if (kind == kOtf64 || kind == kOtf32) {

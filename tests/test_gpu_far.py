@@ -107,3 +107,23 @@ def test_inner_solves(shape, amoeba):
         s.terminate()
     d = both[0] - both[1]
     assert np.sqrt((d * d).mean(axis=(1, 2, 3))).max() <= 6e-9
+
+
+def test_kernel_statistics():
+    """Mixed solves with far-field inner solves: the class of the direct FP32 sweep
+    counts the FP32 residuals (at most one per FP64 step), not the inner products,
+    in the first solve and in one enqueued ahead from its iteration counts."""
+    n = 13500
+    s = _system(n, True)
+    s.set_precision("mixed")
+    s.set_solver_tolerance(3e-10, 500)
+    s.profile_kernels(True)
+    field = np.random.default_rng(2).normal(0.0, 1e-2, size=(n, 3))
+    for _ in range(2):
+        s.kernel_stats(reset=True)
+        s.reset_guess()
+        s.set_external_field(field)
+        outer, inner = s.last_iterations[2:4]
+        launches = s.kernel_stats(reset=True)["otf32"][0]
+        assert inner >= 2 * outer and 1 <= launches < outer, (launches, outer, inner)
+    s.terminate()
