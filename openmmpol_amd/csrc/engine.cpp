@@ -1606,8 +1606,9 @@ void refresh_host_ipd(System &s) {
     s.host_ipd_stale = false;
 }
 
-// Device bytes ensure_device() allocates for a system (packed T, dense T and
-// the batched multi-RHS state come on top, on demand).
+// Device bytes ensure_device() allocates for a system (packed T, dense T, the tree
+// of the far-field inner solves and the batched multi-RHS state come on top, on
+// demand; the serving loop's batches build none of the first three).
 size_t device_footprint_estimate(const System &s) {
     const size_t np = s.npol, nm = s.nmm, n = 3 * np;
     size_t b = np * (sizeof(double4) + sizeof(float4) + 3 * sizeof(double) + sizeof(float) + sizeof(int));
@@ -1621,8 +1622,6 @@ size_t device_footprint_estimate(const System &s) {
         b += tmv_sym_part_bytes(s.npol, 2, 64) + sizeof(int2) * nb * (nb + 1) / 2;
     }
     b += (size_t)(s.list_S_P_P.nnz() + s.list_S_P_D.nnz() + 2 * s.list_P_P.nnz() + s.list_P_P_dense.nnz()) * 24;
-    if (s.npol >= far_inner_from(s.n_ipd))  // tree of the far-field inner solves: basis functions, cells, tables
-        b += np * (5 * kFarBasis * sizeof(float) + 64) + (size_t(128) << 20);
     return b + (1 << 20);
 }
 

@@ -185,6 +185,26 @@ def test_server_admission_waits_for_memory(requests):
         assert np.array_equal(mix[k][0], tight[k][0]) and np.array_equal(mix[k][1], tight[k][1])
 
 
+def test_server_holds_what_it_uses():
+    """The memory held for a request grows with its sites alone (about with their square
+    from the pair-once sizes on): 13,200 sites, where the single solver's far-field tree
+    begins, take little more than 12,800 ((13,200 / 12,800)^2 = 1.06; the tree, which
+    the serving loop does not build, would double it)."""
+    from openmmpol_amd.serving import Server
+    from test_gpu_rows import chain, pair
+    peak = []
+    for n in (12800, 13200):
+        s, _ = pair(chain(n, True))
+        s.set_precision("mixed")
+        srv = Server(hbm_budget=64e9, max_active=2)
+        srv.submit(s, np.array([[[-20.0, -20.0, -20.0, 0.5], [-22.0, -20.0, -20.0, -0.5]]]))
+        srv.wait()
+        peak.append(srv.stats()["peak_bytes"])
+        srv.close()
+        s.terminate()
+    assert peak[1] <= 1.1 * peak[0], peak
+
+
 # ------------------------------------------------ pair-once sweep in batches
 def test_multi_rhs_pair_once_matches_oracle(tight_oracle):
     """A 7,500-site system (30 blocks of 256, the last one padded): its FP64
