@@ -115,8 +115,11 @@ double *ommp_amd_get_pol(OMMP_SYSTEM_PRT s);
    (each the sweep the solvers use at this size), 2 packed in-core FP32, 3 packed
    in-core FP64, 4 fast multipoles (FP64, with the system's FMM settings),
    5 / 6 on-the-fly FP64 / FP32 evaluating each unordered pair once, 7 / 8
-   on-the-fly FP64 / FP32 per target.  repeat > 1 launches it that
-   many times back to back and returns the mean device time per launch (ms). */
+   on-the-fly FP64 / FP32 per target, 9 the FP32 far-field product of the inner
+   solves of large mixed solves (of order 8: relative error 2e-5 to 1e-4; fatal
+   where it would leave more than an eighth of the pairs to its near field).
+   repeat > 1 launches it that many times back to back and returns the mean device
+   time per launch (ms). */
 double ommp_amd_tmatvec(OMMP_SYSTEM_PRT s, int32_t kind, int32_t ncols, const double *x, double *y,
                         int32_t repeat);
 

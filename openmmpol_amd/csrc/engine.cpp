@@ -1993,10 +1993,14 @@ const double *device_ipd(System &s) {
 
 double tmatvec_host(System &s, int kind, int ncols, const double *x, double *y, int repeat) {
     if (ncols < 1 || ncols > 2) fatal("tmatvec supports 1 or 2 columns");
-    if (kind < 0 || kind > 8) fatal("Unknown matvec kind");
+    if (kind < 0 || kind > kFar32) fatal("Unknown matvec kind");
     if (s.npol == 0) return 0.0;
     DeviceState &d = ensure_device(s);
     const long n = d.n;
+    if (kind == kFar32) {
+        ensure_far_inner(s, d, ncols);
+        if (!d.inner.use) fatal("The far-field matvec leaves more than an eighth of this system's pairs to its near field");
+    }
     HCHECK(hipMemcpyAsync(d.vd, x, sizeof(double) * ncols * n, hipMemcpyHostToDevice, d.stream));
     matvec(s, d, kind, ncols, d.vd, d.vr2, true, nullptr, nullptr);  // builds packed T if needed
     if (repeat < 1) repeat = 1;

@@ -1,6 +1,7 @@
 """The matrix-core transfer and T matvec of the fast multipoles (orders up to 8)
 on small trees: one leaf, two per side (no far field), and far fields of two and
-three levels, odd sizes, orders whose coefficients fill 1 to 5 tiles; AMOEBA and
+three levels, leaves of 6 to 141 sites (from 97 on 32 targets share a
+workgroup), odd sizes, orders whose coefficients fill 1 to 5 tiles; AMOEBA and
 AMBER.  Against the complex kernels, which an order of the static field above 8
 selects and which sum the same truncated expansions in another order: 1e-12 of
 the largest component (FP64 sums of a few thousand terms); and with no far field
@@ -21,7 +22,7 @@ def _system(n, amoeba):
 
 
 @pytest.mark.parametrize("amoeba", [True, False])
-@pytest.mark.parametrize("n,cell", [(7, 40.0), (301, 12.0), (1003, 8.0), (3001, 7.0)])
+@pytest.mark.parametrize("n,cell", [(7, 40.0), (301, 12.0), (1003, 8.0), (3001, 7.0), (9001, 20.0)])
 def test_matvec_small_trees(n, cell, amoeba):
     s = _system(n, amoeba)
     x = np.random.default_rng(3).normal(0.0, 0.05, size=(2, n, 3))
@@ -126,4 +127,44 @@ def test_kernel_statistics():
         outer, inner = s.last_iterations[2:4]
         launches = s.kernel_stats(reset=True)["otf32"][0]
         assert inner >= 2 * outer and 1 <= launches < outer, (launches, outer, inner)
+    s.terminate()
+
+
+@pytest.mark.parametrize("p", [4, 8])
+def test_unequal_orders(p):
+    """Orders 4 and 8 of the two expansions: the transfer serves the one of order 8,
+    the complex kernels and their tables the other; both against trees with an order
+    of 9, where the complex kernels serve both (1e-12 as above)."""
+    n = 1003
+    s = _system(n, True)
+    x = np.random.default_rng(3).normal(0.0, 0.05, size=(2, n, 3))
+    s.enable_fmm(lmax=12 - p, lmax_pol=p, distance=1.0, min_cell_size=8.0)
+    y, e = s.tmatvec(x, kind="fmm")[0], s.e_m2d
+    s.enable_fmm(lmax=9, lmax_pol=p, distance=1.0, min_cell_size=8.0)
+    want = s.tmatvec(x, kind="fmm")[0]
+    assert np.abs(y - want).max() <= 1e-12 * np.abs(want).max()
+    s.enable_fmm(lmax=12 - p, lmax_pol=9, distance=1.0, min_cell_size=8.0)
+    want = s.e_m2d
+    assert np.abs(e - want).max() <= 1e-12 * np.abs(want).max()
+    s.terminate()
+
+
+@pytest.mark.parametrize("amoeba", [True, False])
+@pytest.mark.parametrize("n,ncols", [(13500, 1), (13500, 2), (60000, 1), (60000, 2)])
+def test_inner_product(n, ncols, amoeba):
+    """The FP32 far-field product alone (leaves of 26 and of 117 sites, the latter with
+    32 targets a workgroup) against the direct FP64 one.  An inner solve is to reduce
+    its residual by 1e-3: 5e-4 of the product's norm asked, and no component further
+    off than 20 times the mean error that allows."""
+    s = _system(n, amoeba)
+    x = np.random.default_rng(4).normal(0.0, 0.05, size=(ncols, n, 3))
+    want, _ = s.tmatvec(x, kind="sym64")
+    y, _ = s.tmatvec(x, kind="far32")
+    assert np.array_equal(s.tmatvec(x, kind="far32")[0], y)
+    for m in range(ncols):
+        rms = np.sqrt((want[m] ** 2).mean())
+        err = np.linalg.norm(y[m] - want[m]) / np.linalg.norm(want[m])
+        print(n, ncols, amoeba, f"{err:.1e}")
+        assert err <= 5e-4, m
+        assert np.abs(y[m] - want[m]).max() <= 20 * 5e-4 * rms, m
     s.terminate()
