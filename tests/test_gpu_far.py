@@ -168,3 +168,108 @@ def test_inner_product(n, ncols, amoeba):
         assert err <= 5e-4, m
         assert np.abs(y[m] - want[m]).max() <= 20 * 5e-4 * rms, m
     s.terminate()
+
+
+def _solver(spec, precision, tol, td=None):
+    from openmmpol_amd import OMMPSystem
+    s = OMMPSystem.from_arrays(True, spec["cmm"], spec["q"], spec["pol"], spec["bonds_ri"], spec["bonds_ci"],
+                               pgroup=spec["pgroup"], thole_a=td)
+    s.set_precision(precision)
+    s.set_solver_tolerance(tol, 500)
+    return s
+
+
+def _solve(s, field):
+    """Dipoles, FP64 steps, inner iterations and launches of the direct FP32 sweep."""
+    s.kernel_stats(reset=True)
+    s.set_external_field(field)
+    return (s.ipd.copy(), *s.last_iterations[2:4], s.kernel_stats(reset=True)["otf32"][0])
+
+
+@pytest.mark.parametrize("shape", ["cube", "plate", "clump"])
+def test_inner_path(shape):
+    """Which product the inner solves of test_inner_solves' systems run: the far field
+    for the cube and the plate (direct FP32 sweeps: at most one residual per FP64 step),
+    the direct sweep for the cube that falls into a few leaves.  Iterations: a solve of
+    1e-6 in one piece or in two of 1e-3 each, one more per piece."""
+    n = 18001
+    spec = chain(n, True, seed=7)
+    rng = np.random.default_rng(8)
+    if shape == "plate":
+        g = np.arange(135)
+        p = np.stack(np.meshgrid(g, g, indexing="ij"), axis=-1).reshape(-1, 2)[:n] * 4.0
+        spec["cmm"] = np.concatenate([p, np.zeros((n, 1))], axis=1) + rng.uniform(-0.8, 0.8, size=(n, 3))
+    elif shape == "clump":
+        spec["cmm"][-8:] += 5000.0 * rng.normal(size=(8, 3))
+    s = _solver(spec, "mixed", 3e-10)
+    s.profile_kernels(True)
+    field = rng.normal(0.0, 1e-2, size=(n, 3))
+    for _ in range(3):
+        s.reset_guess()
+        _, outer, inner, launches = _solve(s, field)
+        print(shape, outer, inner, launches)
+        assert outer == 3
+        if shape == "clump":
+            assert inner <= launches <= inner + 2 * outer
+        else:
+            assert 1 <= launches < outer
+        assert inner <= 30
+    s.terminate()
+
+
+def test_inner_fallback():
+    """A geometry that the expansions do not fit: damping factors of 1e-4 damp pairs out
+    to 60 bohr, far beyond the 27 leaves of 13 bohr where the product damps them.  The
+    direct sweep takes over within the first solve, serves the following ones on this
+    geometry, and the far field is tried again on the next (here damped as usual).
+    Dipoles against the FP64 solver: T is close to 1 / alpha here, so that two solves to
+    an rms of 3e-10 of sqrt(alpha) r differ by sqrt(30) 2 3e-10 = 3.3e-9; 1e-8 asked."""
+    n = 18001
+    spec = chain(n, True, seed=7)
+    spec["pol"][:] = 30.0
+    td = np.full(n, 1e-4)
+    field = np.random.default_rng(9).normal(0.0, 1e-2, size=(2, n, 3)) + 1e-2
+    ref = _solver(spec, "fp64", 3e-10, td)
+    s = _solver(spec, "mixed", 3e-10, td)
+    s.profile_kernels(True)
+    for k, f in enumerate((field[0], field[1], field[0])):
+        ref.set_external_field(f)
+        got, outer, inner, launches = _solve(s, f)
+        print(k, outer, inner, launches)
+        assert np.sqrt(((got - ref.ipd) ** 2).mean()) <= 1e-8, k
+        assert launches >= 3, k
+        if k:
+            assert launches >= inner, (k, launches, inner)
+    # stretched so far that no pair is damped beyond the leaves: the far field again
+    spec["cmm"] = spec["cmm"] * 8.0
+    s.update_coordinates(spec["cmm"])
+    ref.update_coordinates(spec["cmm"])
+    ref.set_external_field(field[0])
+    got, outer, inner, launches = _solve(s, field[0])
+    print("stretched", outer, inner, launches)
+    assert np.sqrt(((got - ref.ipd) ** 2).mean()) <= 1e-8
+    assert launches < outer
+    ref.terminate()
+    s.terminate()
+
+
+def test_inner_guess_not_finite():
+    """A guess that is not finite (written over the dipoles in device memory): the steps
+    enqueued ahead come to nothing, the residual after them says so, and the solve starts
+    again from nothing with the direct sweep.  Against the solve before it, both to an
+    rms of 3e-10 (6e-9 as above)."""
+    import ctypes
+    n = 18001
+    s = _solver(chain(n, True, seed=7), "mixed", 3e-10)
+    s.profile_kernels(True)
+    field = np.random.default_rng(9).normal(0.0, 1e-2, size=(n, 3))
+    want = _solve(s, field)[0]
+    bad = np.full((2, n, 3), np.nan)
+    hip = ctypes.CDLL("libamdhip64.so")
+    assert hip.hipMemcpy(ctypes.c_void_p(s.device_ipd_ptr()), bad.ctypes.data_as(ctypes.c_void_p),
+                         ctypes.c_size_t(bad.nbytes), 1) == 0
+    got, outer, inner, launches = _solve(s, field)
+    print(outer, inner, launches)
+    assert np.sqrt(((got - want) ** 2).mean()) <= 6e-9
+    assert launches >= 10  # direct inner iterations
+    s.terminate()

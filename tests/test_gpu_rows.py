@@ -76,7 +76,7 @@ def test_damping_cutoff(n, kinds, scale, amoeba):
     spacing (hundreds of damped pairs a site: the lists overflow), with one outlying
     polarizability, against the oracle.  FP64: 3,001 terms of rounding 1.1e-16 on
     sums that cancel to a few of them: 1e-12 of the largest component; FP32 by its
-    rounding of 6e-8: 3e-4."""
+    rounding of 6e-8: 3e-4 at 1.4 bohr, and 2e-6 at 4 bohr, where they do not cancel."""
     spec = chain(n, amoeba)
     spec["cmm"] = spec["cmm"] * scale
     spec["pol"][n // 2] = 300.0
@@ -86,7 +86,7 @@ def test_damping_cutoff(n, kinds, scale, amoeba):
     for kind in kinds:
         for ncols in (1, 2):
             y, _ = s.tmatvec(x[:ncols], kind=kind)
-            bar = 1e-12 if kind.endswith("64") else 3e-4
+            bar = 1e-12 if kind.endswith("64") else 2e-6 if scale == 1.0 else 3e-4
             assert np.abs(y - want[:ncols]).max() <= bar * np.abs(want).max(), (kind, ncols)
         assert np.array_equal(s.tmatvec(x, kind=kind)[0], y)
     s.terminate()
