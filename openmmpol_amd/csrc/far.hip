@@ -533,7 +533,6 @@ __global__ __launch_bounds__(kBlock) void k_far_near(
         }
         __syncthreads();
         int n = 0;
-#pragma unroll 2
         for (int q = sl; q < cntp; q += NS) {
             const R4 p = s_pos[q];
             R4 v[M];
@@ -574,24 +573,7 @@ __global__ __launch_bounds__(kBlock) void k_far_near(
     double sum[C];
 #pragma unroll
     for (int c = 0; c < C; c++) sum[c] = -(double)f[c / 3][c % 3];
-    const int k1 = pp_ri[site + 1];
-    for (int k = pp_ri[site] + sl; k < k1; k += NS) {
-        const int i = pp_ci[k];
-        const double fk = pp_f[k];
-        const double4 qj = ps[site], pi = ps[i];
-        const double dx = qj.x - pi.x, dy = qj.y - pi.y, dz = qj.z - pi.z;
-        const double r2 = dx * dx + dy * dy + dz * dz;
-        double k2, k3;
-        dip_kernel<double, AMOEBA>(r2, rsqrt(r2), pi.w, qj.w, pa[i], pa[site], k2, k3);
-#pragma unroll
-        for (int m = 0; m < M; m++) {
-            const double *xi = x + m * xstride + 3L * i;
-            const double c = k3 * (xi[0] * dx + xi[1] * dy + xi[2] * dz);
-            sum[3 * m + 0] += fk * (c * dx - k2 * xi[0]);
-            sum[3 * m + 1] += fk * (c * dy - k2 * xi[1]);
-            sum[3 * m + 2] += fk * (c * dz - k2 * xi[2]);
-        }
-    }
+    screened_pairs<AMOEBA, M>(site, sl, NS, ps, pa, pp_ri, pp_ci, pp_f, x, xstride, sum);
 #pragma unroll
     for (int mask = T; mask < 64; mask <<= 1)
 #pragma unroll

@@ -8,39 +8,13 @@
 #include <mutex>
 #include <type_traits>
 
-#include "far.h"
+#include "fmm_host.h"
 
 namespace ommp {
 
 namespace {
 
 using cplx = std::complex<double>;
-
-cplx ipow(int e) {
-    static const cplx v[4] = {{1.0, 0.0}, {0.0, 1.0}, {-1.0, 0.0}, {0.0, -1.0}};
-    return v[e & 3];
-}
-
-// T_n^m(v), all m, index n^2 + n + m.
-std::vector<cplx> transfer(int p, const double v[3]) {
-    const double r2 = v[0] * v[0] + v[1] * v[1] + v[2] * v[2], ir2 = 1.0 / r2;
-    const cplx w(v[0], v[1]);
-    std::vector<cplx> t((p + 1) * (p + 1));
-    cplx pmm = 1.0 / std::sqrt(r2);
-    for (int m = 0; m <= p; m++) {
-        if (m > 0) pmm *= (2.0 * m - 1.0) * w * ir2;
-        cplx before = 0.0, cur = pmm;
-        for (int n = m; n <= p; n++) {
-            const cplx f = ipow(m) * ((n & 1) ? -1.0 : 1.0);
-            t[n * n + n + m] = f * cur;
-            t[n * n + n - m] = f * std::conj(cur);
-            const cplx next = ((2.0 * n + 1.0) * v[2] * cur - (double)(n + m) * (double)(n - m) * before) * ir2;
-            before = cur;
-            cur = next;
-        }
-    }
-    return t;
-}
 
 // Coefficients of Re and Im Phi in the complex functions of +m and -m.
 struct Term {
@@ -49,13 +23,13 @@ struct Term {
 };
 std::vector<Term> source_terms(int m, bool im) {
     // R^m = (-i)^m (c - i s), R^-m = (-i)^m (c + i s)
-    std::vector<Term> out = {{m, ipow(-m) * (im ? cplx(0.0, -1.0) : cplx(1.0))}};
-    if (m > 0) out.push_back({-m, ipow(-m) * (im ? cplx(0.0, 1.0) : cplx(1.0))});
+    std::vector<Term> out = {{m, fmm_ipow(-m) * (im ? cplx(0.0, -1.0) : cplx(1.0))}};
+    if (m > 0) out.push_back({-m, fmm_ipow(-m) * (im ? cplx(0.0, 1.0) : cplx(1.0))});
     return out;
 }
 std::vector<Term> local_terms(int j, int k, bool im) {
     // S^k = i^-k (-1)^j (c + i s), S^-k = i^-k (-1)^j (c - i s)
-    const cplx f = ipow(-k) * ((j & 1) ? -1.0 : 1.0);
+    const cplx f = fmm_ipow(-k) * ((j & 1) ? -1.0 : 1.0);
     std::vector<Term> out = {{k, f * (im ? cplx(0.0, 1.0) : cplx(1.0))}};
     if (k > 0) out.push_back({-k, f * (im ? cplx(0.0, -1.0) : cplx(1.0))});
     return out;
@@ -81,13 +55,15 @@ template <typename R> void make_tables(int p, FarTables<R> &out) {
         const int d[3] = {o % 7 - 3, o / 7 % 7 - 3, o / 49 - 3};
         if (std::abs(d[0]) <= 1 && std::abs(d[1]) <= 1 && std::abs(d[2]) <= 1) continue;
         const double v[3] = {(double)d[0], (double)d[1], (double)d[2]};
-        const std::vector<cplx> t = transfer(2 * p, v);
+        std::vector<double2> tv((2 * p + 1) * (2 * p + 1));
+        fmm_transfer(2 * p, v, tv.data());
+        auto t = [&](int k) { return cplx(tv[k].x, tv[k].y); };
         for (int row = 0; row < ncoef; row++) {
             for (int col = 0; col < ncoef; col++) {
                 const int n = deg[row] + deg[col];
                 cplx s = 0.0;
                 for (const Term &a : loc[row])
-                    for (const Term &b : src[col]) s += a.f * b.f * t[n * n + n + b.m - a.m];
+                    for (const Term &b : src[col]) s += a.f * b.f * t(n * n + n + b.m - a.m);
                 // lane (row % 16, col / per), element col % per in vectors of 16 bytes
                 const int lane = row % 16 + 16 * (col / per), e = col % per;
                 out.K[((((size_t)o * tiles + row / 16) * (per / vec) + e / vec) * 64 + lane) * vec + e % vec] =
@@ -95,7 +71,7 @@ template <typename R> void make_tables(int p, FarTables<R> &out) {
             }
             cplx s = 0.0;
             const int n = deg[row];
-            for (const Term &a : loc[row]) s += a.f * t[n * n + n - a.m];
+            for (const Term &a : loc[row]) s += a.f * t(n * n + n - a.m);
             out.K0[((size_t)o * tiles + row / 16) * 64 + row % 16] = (R)s.real();
         }
     }

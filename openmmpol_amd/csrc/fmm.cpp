@@ -19,15 +19,6 @@ using cplx = std::complex<double>;
 
 inline int hidx(int n, int m) { return n * n + n + m; }
 
-cplx ipow(int e) {
-    switch (e & 3) {
-        case 0: return {1.0, 0.0};
-        case 1: return {0.0, 1.0};
-        case 2: return {-1.0, 0.0};
-        default: return {0.0, -1.0};
-    }
-}
-
 // Phi_n^m(v), m >= 0 (see fmm_kernels.hip), into phi[hidx(n, m)].
 void phi_all(int p, const double v[3], std::vector<cplx> &phi) {
     const double r2 = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
@@ -75,13 +66,13 @@ void psi_all(int p, const double v[3], std::vector<cplx> &psi) {
     }
 }
 
-// R_n^+-m (source moments), S_n^+-m (local evaluation), T_n^+-m (transfer).
+// R_n^+-m (source moments), S_n^+-m (local evaluation); T_n^+-m (transfer) below.
 void r_all(int p, const double v[3], double2 *out) {
     std::vector<cplx> phi;
     phi_all(p, v, phi);
     for (int n = 0; n <= p; n++)
         for (int m = 0; m <= n; m++) {
-            const cplx f = ipow(-m);
+            const cplx f = fmm_ipow(-m);
             const cplx a = f * std::conj(phi[hidx(n, m)]), b = f * phi[hidx(n, m)];
             out[hidx(n, m)] = make_double2(a.real(), a.imag());
             out[hidx(n, -m)] = make_double2(b.real(), b.imag());
@@ -92,25 +83,25 @@ void s_all(int p, const double v[3], double2 *out) {
     phi_all(p, v, phi);
     for (int n = 0; n <= p; n++)
         for (int m = 0; m <= n; m++) {
-            const cplx f = ipow(-m) * ((n & 1) ? -1.0 : 1.0);
+            const cplx f = fmm_ipow(-m) * ((n & 1) ? -1.0 : 1.0);
             const cplx a = f * phi[hidx(n, m)], b = f * std::conj(phi[hidx(n, m)]);
             out[hidx(n, m)] = make_double2(a.real(), a.imag());
             out[hidx(n, -m)] = make_double2(b.real(), b.imag());
         }
 }
-void t_all(int p, const double v[3], double2 *out) {
+}  // namespace
+
+void fmm_transfer(int p, const double v[3], double2 *out) {
     std::vector<cplx> psi;
     psi_all(p, v, psi);
     for (int n = 0; n <= p; n++)
         for (int m = 0; m <= n; m++) {
-            const cplx f = ipow(m) * ((n & 1) ? -1.0 : 1.0);
+            const cplx f = fmm_ipow(m) * ((n & 1) ? -1.0 : 1.0);
             const cplx a = f * psi[hidx(n, m)], b = f * std::conj(psi[hidx(n, m)]);
             out[hidx(n, m)] = make_double2(a.real(), a.imag());
             out[hidx(n, -m)] = make_double2(b.real(), b.imag());
         }
 }
-
-}  // namespace
 
 FmmHost fmm_build(const System &s, int p_pol, int p_static, double min_cell, double distance) {
     FmmHost f;
@@ -221,7 +212,7 @@ FmmHost fmm_build(const System &s, int p_pol, int p_static, double min_cell, dou
                         if (std::abs(dx) <= 1 && std::abs(dy) <= 1 && std::abs(dz) <= 1) continue;
                         const double v[3] = {dx * h, dy * h, dz * h};
                         const int o = (dz + 3) * 49 + (dy + 3) * 7 + (dx + 3);
-                        t_all(2 * pt, v, &f.tab_m2l[((size_t)l * 343 + o) * f.ncoef2_tab]);
+                        fmm_transfer(2 * pt, v, &f.tab_m2l[((size_t)l * 343 + o) * f.ncoef2_tab]);
                     }
     }
     return f;

@@ -174,6 +174,36 @@ __device__ __forceinline__ void pair_accum(R (&acc)[M][3], const typename V4<R>:
     }
 }
 
+// Screened pairs of target j (pp lists, f = 1 - s), entries first, first + step, ...:
+// f times the damped dipole field, scale 1, is taken out again of T x.
+template <bool AMOEBA, int M>
+__device__ __forceinline__ void screened_pairs(int j, int first, int step, const double4 *__restrict__ ps,
+                                               const double *__restrict__ pa, const int *__restrict__ pp_ri,
+                                               const int *__restrict__ pp_ci, const double *__restrict__ pp_f,
+                                               const double *__restrict__ x, long xstride, double (&sum)[3 * M]) {
+    const int k0 = pp_ri[j], k1 = pp_ri[j + 1];
+    if (k0 >= k1) return;
+    const double4 qj = ps[j];
+    const double bj = pa[j];
+    for (int k = k0 + first; k < k1; k += step) {
+        const int i = pp_ci[k];
+        const double f = pp_f[k];
+        const double4 pi = ps[i];
+        const double dx = qj.x - pi.x, dy = qj.y - pi.y, dz = qj.z - pi.z;
+        const double r2 = dx * dx + dy * dy + dz * dz;
+        double k2, k3;
+        dip_kernel<double, AMOEBA>(r2, rsqrt(r2), pi.w, qj.w, pa[i], bj, k2, k3);
+#pragma unroll
+        for (int m = 0; m < M; m++) {
+            const double *xi = x + m * xstride + 3L * i;
+            const double c = k3 * (xi[0] * dx + xi[1] * dy + xi[2] * dz);
+            sum[3 * m + 0] += f * (c * dx - k2 * xi[0]);
+            sum[3 * m + 1] += f * (c * dy - k2 * xi[1]);
+            sum[3 * m + 2] += f * (c * dz - k2 * xi[2]);
+        }
+    }
+}
+
 // ----------------------------------------------------------- static field
 // Field at polarizable target j of MM source i (charge, dipole, quadrupole),
 // damped kernel with maxder 3 (AMOEBA) or 1 (Wang), as damped_coulomb_kernel +

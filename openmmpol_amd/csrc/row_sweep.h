@@ -184,28 +184,7 @@ __device__ __forceinline__ void row_finish(RowAcc<R, M, T> &a, RowLds<R, M, T> &
                 for (int c = 0; c < C; c++) corr[c] -= (double)f[c / 3][c % 3];
             }
         }
-        const int k0 = pp_ri[j], k1 = pp_ri[j + 1];
-        if (k0 < k1) {
-            const double4 qj = ps[j];
-            const double bj = pa[j];
-            for (int k = k0 + lane; k < k1; k += 64) {
-                const int i = pp_ci[k];
-                const double f = pp_f[k];
-                const double4 pi = ps[i];
-                const double dx = qj.x - pi.x, dy = qj.y - pi.y, dz = qj.z - pi.z;
-                const double r2 = dx * dx + dy * dy + dz * dz;
-                double k2, k3;
-                dip_kernel<double, AMOEBA>(r2, rsqrt(r2), pi.w, qj.w, pa[i], bj, k2, k3);
-#pragma unroll
-                for (int m = 0; m < M; m++) {
-                    const double *xi = x + m * xstride + 3L * i;
-                    const double c = k3 * (xi[0] * dx + xi[1] * dy + xi[2] * dz);
-                    corr[3 * m + 0] += f * (c * dx - k2 * xi[0]);
-                    corr[3 * m + 1] += f * (c * dy - k2 * xi[1]);
-                    corr[3 * m + 2] += f * (c * dz - k2 * xi[2]);
-                }
-            }
-        }
+        screened_pairs<AMOEBA, M>(j, lane, 64, ps, pa, pp_ri, pp_ci, pp_f, x, xstride, corr);
         wave_rows<double, 1, C>(corr);
         if (lane == 0) {
 #pragma unroll
