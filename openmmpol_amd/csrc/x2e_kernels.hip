@@ -242,7 +242,9 @@ static int x2e_point_blocks(int n) { return (n + kBlock * x2e_points(n) - 1) / (
 
 int x2e_splits(int n, int nsrc) {
     const int pb = x2e_point_blocks(n), pf = n > kX2eNoAllocMaxPoints ? pb : (n + kBlock - 1) / kBlock;
-    const int thin = std::min((nsrc + 15) / 16, (512 + pb - 1) / pb);  // two workgroups per CU
+    // two workgroups per CU and not a few more: a third on some CUs sets the time (20,000
+    // points, 5,004 charges, field: 520 workgroups 118 us, 500 95)
+    const int thin = std::min((nsrc + 15) / 16, std::max(1, 512 / pb));
     const int full = std::min((nsrc + kBlock - 1) / kBlock, (2048 + pf - 1) / pf);
     return std::max(1, std::max(thin, full));
 }
@@ -303,7 +305,7 @@ void launch_x2e(hipStream_t st, int n, const double *cext, bool mm, bool pol, bo
 // summed result and the coincident-point flag.  Split counts are those of the
 // allocating entry (x2e_splits), so both give the same bits.  For n points
 // each source kind takes at most ceil(2048 / ceil(n / 256)) splits, or
-// ceil(512 / ceil(n / 512)) or ceil(512 / ceil(n / 256)), which is fewer, so the
+// 512 / ceil(n / 512) or 512 / ceil(n / 256), which is fewer, so the
 // partial sums need at most 2 (2048 + ceil(n / 256) - 1) 256 double4.
 // Every call on a GPU uses that GPU's array: calls that overlap on one GPU
 // (other host threads, other streams) race; each call waits for its own work.
