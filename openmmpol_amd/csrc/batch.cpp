@@ -46,10 +46,11 @@ SegLayout seg_layout(int npol, int nrhs, int nsets, int m32, int num_cu, int ext
     L.xs = m32 == kBatchM32 ? align256(sizeof(unsigned short) * kBxParts * ncols * (size_t)bx_ld(npol)) : 0;
     // the pair-once sweep from the sizes where it beats the batched per-target
     // sweep, its partials under 8 GiB (SCF sequences of six systems of 500 to 9,000
-    // sites: from 11,000 / 7,000 sites in FP32 / FP64 20.2 ms, from 6,000 / 5,000
-    // 17.5, from 4,000 17.6, from 2,500 18.1; three systems up to 4,000 sites: 7.3 ms
-    // below the limit, 9.5 above it); wide batches run both matvecs on the matrix
-    // cores with their own tiling (partials per source split)
+    // sites: from 8,000 / 7,000 sites in FP32 / FP64 21.0 ms, from 7,000 / 6,000 21.2,
+    // from 6,000 / 5,000 18.5; of three systems of 6,100 to 6,900 sites 17.2, 16.3 and
+    // 13.7, of 5,100 to 5,900 14.0, 14.1 and 13.8; from 4,000 and 2,500 sites on slower
+    // again, three systems up to 4,000 sites 9.5 instead of 7.3); wide batches run both
+    // matvecs on the matrix cores with their own tiling (partials per source split)
     const bool sym_fits = m32 == 2 && tmv_sym_part_bytes(npol, std::max(ncols, 2), 64) <= size_t(8) << 30;
     L.sym32 = sym_fits && npol >= 6000;
     L.sym64 = sym_fits && npol >= 5000;

@@ -694,17 +694,22 @@ void ensure_fmm(System &s, DeviceState &d) {
 // like its preconditioner: the FP64 residuals are of the direct sum, convergence is
 // decided by them, and a geometry where an inner solve does not cut them by 10 goes
 // back to the direct sweep.  us per matvec of two columns, far field / pair-once:
-// 110 / 160 at 15,000 sites, 125 / 260 at 20,001, 232 / 930 at 40,000, 387 / 2040 at
-// 60,000, of one column 91 / 107 at 15,000, 100 / 195 at 20,001; the tree costs 1.0 to
-// 1.6 ms per geometry and a solve one or two FP32 residuals of the direct sweep.  Whole
-// solves with two columns: 14,000 sites (water) 2.66 / 3.06, 15,000 3.70 / 4.43, 60,000
-// 24.6 / 54.8; with one column 24,000 3.2 / 4.3; gradient steps with their trees: 20,001
-// 7.5 / 9.1.  With one FP64 residual more instead of the FP32 ones 12,000 sites took
-// 3.25 / 3.29, 10,000 3.0 / 2.8; with them 11,000 2.95 / 2.88, one column at 15,000 1.98
-// / 2.0 and at 17,000 2.2 / 2.4: used from 13,000 and 16,000.
-// Leaves of 24 sites and more in the mean: at 60,000 sites 29 and 171 an occupied leaf
-// take 363 and 387 us, the larger ones with an error of 2.6e-5 instead of 1.4e-4, which
-// saves iterations (solve 33.1 and 28.0 ms).
+// 101 / 139 at 13,500 sites, 108 / 157 at 15,000, 125 / 259 at 20,001, 239 / 898 at
+// 40,000, 400 / 1970 at 60,000, 468 / 5530 at 100,000, of one column 91 / 101 at 13,500,
+// 93 / 115 at 15,000, 104 / 183 at 20,001; a solve costs one or two FP32 residuals of
+// the direct sweep, the tree (host, mostly behind the static field's sweep) 0.02 to 0.12
+// ms of a solve on a new geometry up to 20,001 sites.
+// Where the line lies, ms with far-field / direct inner solves.  Two columns, solve on a
+// new geometry (tree and lists with it): 10,002 sites 2.67 / 2.45, 12,000 2.93 / 2.91,
+// 13,500 3.26 / 3.39, 15,000 4.04 / 4.68, 20,001 4.75 / 6.07; solve from the previous
+// dipoles on the same geometry: 12,000 1.68 / 1.61, 13,500 1.84 / 1.87, 15,000 2.54 / 2.86.
+// One column, new geometry: 15,000 2.22 / 2.09, 17,001 2.43 / 2.50, 20,001 2.74 / 3.27;
+// from nothing 17,001 2.17 / 2.36; from the previous dipoles 17,001 1.65 / 1.62, 20,001
+// 1.90 / 2.15.
+// Leaves of 24 sites and more in the mean, solves with the smaller / larger leaves where
+// both are possible: 35,000 sites 12.8 / 10.1 ms, 50,000 19.5 / 17.9, 65,000 28.4 / 28.6,
+// 80,000 38.9 / 41.7, 100,000 55.7 / 61.9; one column 65,001 13.4 / 14.0 (the rule takes
+// the smaller ones from about 62,000 sites of a compact system).
 constexpr int kFarInnerOrder = 8, kFarInnerOccupancy = 24;
 int far_inner_from(int M) { return M == 2 ? 13000 : 16000; }
 
@@ -938,9 +943,9 @@ void matvec(System &s, DeviceState &d, int kind, int M, const double *x, double 
 }
 
 // The preconditioner of the current geometry on the device: lists built once per
-// coordinates (the sites closer than kNbCut, each row in site order), tensors B recomputed before the first mixed solve of a
-// geometry (and after a reset of the static field), which also clears a
-// breakdown switch-off.
+// coordinates (the sites closer than kNbCut, each row in site order), tensors B
+// recomputed before the first mixed solve of a geometry (and after a reset of the
+// static field), which also clears a breakdown switch-off.
 void ensure_nb(System &s, DeviceState &d) {
     NbDev &nb = d.nb;
     if (!nb.list_valid) {
@@ -1358,15 +1363,18 @@ MixedResult mixed_solve(System &s, DeviceState &d, int M, const double *b, doubl
 // makes one refinement step enough for most warm-started solves.
 double refine_eta() { return 1e-6; }
 // In the serving loop a solve starts from its predecessor, about 1e6 tolerances away,
-// so that 1e-6 of it ends on either side of the tolerance by the sums' rounding (errors
-// of 2e-9 or 1e-8 in the dipoles); a quarter of it, still above FP32's reach, ends below
-// in one inner solve (all under 5e-9; six systems of 500 to 9,000 sites 17.5 -> 18.0 ms).
+// so that 1e-6 of it ends on either side of the tolerance by the sums' rounding; a
+// quarter of it, still above FP32's reach, ends below in one inner solve (largest error
+// of the dipoles over four draws of two to six systems 1.2e-8 to 2.3e-8 and 0.5e-8 to
+// 1.1e-8, for 5 to 8% more inner iterations: six systems of 500 to 9,000 sites 12.0 and
+// 12.9 ms).
 double refine_eta_serving() { return 2.5e-7; }
 // The last inner solve aims well below the tolerance: a CG iteration reduces the
 // residual by ~0.35, so an aim of f tol ends anywhere in 0.35 f tol .. f tol, and
 // with f = 0.25 the result's error does not depend on where the sums' rounding
 // makes it end (with 0.8 the gradient's error moved by 1.6 times between two
-// summation orders); about one inner iteration more.
+// summation orders); about one inner iteration more (one field of 648 sites 1.35 and
+// 1.42 ms with errors of 2.9e-9 and 0.9e-9, of 5,004 sites 1.86 and 2.03).
 double refine_frac() { return 0.25; }
 // A wide batch iterates over all its columns until the last one is done, so that one
 // more iteration costs every column (5% at 15,000 sites and 64 right-hand sides): they
@@ -1591,8 +1599,7 @@ double fixedelec_energy(System &s) {
     HCHECK(hipStreamSynchronize(d.stream));
     int bad = 0;
     std::memcpy(&bad, d.scal_host + 1, sizeof(int));
-    if (bad)
-        fatal(kCoincident);
+    if (bad) fatal(kCoincident);
     s.e_mm = d.scal_host[0];
     s.m2m_done = true;
     return s.e_mm;
@@ -1797,8 +1804,7 @@ void x2e_host(System &s, int n, const double *cext, bool mm, bool pol, double *V
     HCHECK(hipMemcpyAsync(out.data(), d.x2e_out, sizeof(double) * 4L * n, hipMemcpyDeviceToHost, d.stream));
     HCHECK(hipMemcpyAsync(&bad, d.x2e_bad, sizeof(int), hipMemcpyDeviceToHost, d.stream));
     HCHECK(hipStreamSynchronize(d.stream));
-    if (bad)
-        fatal(kCoincident);
+    if (bad) fatal(kCoincident);
     for (long j = 0; j < n; j++) {
         if (V) V[j] += out[4 * j];
         if (E)
@@ -1823,8 +1829,7 @@ void x2e_field_noalloc_host(System &s, int n, const double *cext, double *E) {
     DeviceState &d = ensure_device(s);  // exists: at most re-uploads coordinates, no allocation
     const int bad = x2e_field_noalloc(d.stream, d.device, n, cext, true, pol, s.amoeba, s.ld_cart, s.nmm, d.ms64,
                                       d.mq, s.npol, d.ps64, d.ipd, E);
-    if (bad)
-        fatal(kCoincident);
+    if (bad) fatal(kCoincident);
 }
 
 namespace {

@@ -1,4 +1,4 @@
-// Far field on the matrix cores (far.h).  A T matvec is five launches:
+// Far field on the matrix cores (far.h).  A T matvec is six launches:
 //   k_far_sort    the dipoles in the order of the sorted sites;
 //   k_far_p2m     moments of every occupied cell of every level straight from its
 //                 sites (no translation upwards: a level is one more pass over the
@@ -12,7 +12,8 @@
 //                 gradient form) of every cell;
 //   k_far_near    per T sites of a leaf: the 27 leaves around it pair by pair, the
 //                 field expansions of all levels, the screened-pair corrections, the
-//                 diagonal and the y.x partial.
+//                 diagonal and the y.x partial;
+//   k_far_dots    the workgroups' y.x partials as kFarDots sums.
 // Every sum has a fixed order.
 //
 // The FP64 form replaces, for orders up to 8, a chain of complex kernels (one

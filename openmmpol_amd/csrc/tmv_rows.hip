@@ -12,14 +12,17 @@
 // loads a thread makes; above, the vector ALUs.  Measured against the sweep it
 // replaces (one target per thread, the sources split over workgroups, partial
 // sums added by a second kernel; chain systems, us per matvec, FP64 one column /
-// FP32 two columns): 99 sites 21.5 -> 2.9 / 15.7 -> 3.2, 648 43 -> 4.8 / 31 ->
-// 4.7, 2,001 51 -> 12.7 / 37 -> 10.2, 5,003 76 -> 59 / 47 -> 38.
+// FP32 two columns): 99 sites 21.5 -> 3.2 / 15.7 -> 4.1, 648 43 -> 5.1 / 31 ->
+// 5.4, 2,001 51 -> 11.9 / 37 -> 11.3, 5,003 75 -> 42 / 48 -> 38.
 //
-// T (rows_targets), us at T = 1 / 2 / 4 / 8: with few sites one target per
-// workgroup keeps the most workgroups (99 sites, FP64: 2.9 / 3.2 / 4.7 / 5.2); then
-// one source load has to serve several pairs (3,000 sites, FP64: 41 / 24.0 / 25.1 /
-// 27; 5,003: 108 / 60 / 59 / 60); FP32 with two columns does the least per
-// source and wants eight (5,003: 74 / 43.6 / 46.0 / 38.5).
+// T (rows_targets), us at T = 1 / 2 / 4: with few sites one target per workgroup
+// keeps the most workgroups (FP64 one column: 99 sites 3.2 / 3.5 / 5.0, 512 4.3 / 4.2 /
+// 5.9); then one source load has to serve several pairs (1,300 sites 9.1 / 8.1 / 9.4,
+// 2,400 20.5 / 15.5 / 16.1, 2,700 24.6 / 19.2 / 17.6, 4,000 49 / 33 / 29), and from 4
+// targets on damped pairs are listed.  FP32 with two columns does the least per source
+// and wants eight instead of four (1 / 2 / 8: 2,400 sites 21 / 14.4 / 19.3, 3,300 35 /
+// 23.0 / 23.0, 3,600 42 / 26.4 / 24.7, 5,003 71 / 43.5 / 38).  The line at 3,000 lies
+// between those of the two precisions.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
