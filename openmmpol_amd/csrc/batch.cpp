@@ -44,16 +44,15 @@ SegLayout seg_layout(int npol, int nrhs, int nsets, int m32, int num_cu, int ext
     }
     L.vec = align256(sizeof(double) * ncols * n);
     L.xs = m32 == kBatchM32 ? align256(sizeof(unsigned short) * kBxParts * ncols * (size_t)bx_ld(npol)) : 0;
-    // the pair-once sweep from the sizes where it beats the batched per-target
-    // sweep, its partials under 8 GiB (SCF sequences of six systems of 500 to 9,000
-    // sites: from 8,000 / 7,000 sites in FP32 / FP64 21.0 ms, from 7,000 / 6,000 21.2,
-    // from 6,000 / 5,000 18.5; of three systems of 6,100 to 6,900 sites 17.2, 16.3 and
-    // 13.7, of 5,100 to 5,900 14.0, 14.1 and 13.8; from 4,000 and 2,500 sites on slower
-    // again, three systems up to 4,000 sites 9.5 instead of 7.3); wide batches run both
-    // matvecs on the matrix cores with their own tiling (partials per source split)
-    const bool sym_fits = m32 == 2 && tmv_sym_part_bytes(npol, std::max(ncols, 2), 64) <= size_t(8) << 30;
-    L.sym32 = sym_fits && npol >= 6000;
-    L.sym64 = sym_fits && npol >= 5000;
+    // the pair-once sweep from the size where it beats the batched per-target sweep, its
+    // partials under 8 GiB (SCF sequences of three systems, pair-once / per target in
+    // both precisions: 2,510 to 2,900 sites 10.2 / 9.4 ms, 3,510 to 3,900 10.9 / 9.7,
+    // 4,100 to 4,450 10.7 / 10.6, 4,550 to 4,950 11.4 / 12.4, 5,010 to 5,300 11.7 / 13.2
+    // with FP32 per target, 6,100 to 6,900 13.7 / 17.2; six of 500 to 9,000 with the line
+    // at 4,500 18.1, at 7,000 / 6,000 in FP32 / FP64 21.2); wide batches run both matvecs
+    // on the matrix cores with their own tiling (partials per source split)
+    L.sym32 = L.sym64 =
+        m32 == 2 && npol >= 4500 && tmv_sym_part_bytes(npol, std::max(ncols, 2), 64) <= size_t(8) << 30;
     size_t part = sizeof(double) * L.nsplit * ncols * n;
     if (L.sym32 || L.sym64) part = std::max(part, tmv_sym_part_bytes(npol, ncols, 64));
     L.part = align256(part);

@@ -39,7 +39,7 @@ __device__ __forceinline__ bool mv_active(const BCol &c, int use_p) {
 // pairs of sources have a damped pair in some lane of the wave, and deciding by the
 // sites' cutoffs first, as the pair-once sweep does, formed their geometry twice (SCF
 // sequences of two systems of 500 and 700 sites 6.3 -> 6.7 ms, of four of 1,000 to
-// 4,000 10.1 -> 10.5; one field of 5,004 sites 2.04 -> 2.17).
+// 4,000 10.1 -> 10.5; longer chains from one evaluation in the branch 6.9 and 10.3).
 template <typename R, int MM, bool AMOEBA>
 __device__ __forceinline__ void bpairs_body(const BSeg &S, const int4 w, const double *__restrict__ xin,
                                             const int (&cidx)[MM]) {
