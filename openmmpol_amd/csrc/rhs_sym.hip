@@ -61,9 +61,12 @@ __device__ __forceinline__ void rhs_geom(const double4 &pt, double at, const dou
         }
     } else {
         k3 = k4 = 0.0;
-        const double u = (r2 * ir) * (pt.w * ps.w);
+        double u = (r2 * ir) * (pt.w * ps.w);
         const bool near = u < 1.0;
         if (__ballot(near)) {
+            // keeps the damping inside the branch (formed for every pair: 20,001 sites
+            // 317 instead of 258 us)
+            asm volatile("" : "+v"(u));
             const double u3 = u * u * u;
             k2 = near ? k2 * (4.0 * u3 - 3.0 * u3 * u) : k2;
         }
