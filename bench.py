@@ -743,7 +743,9 @@ def main():
                                 "pair; priced against the published FP32 peak, which counts packed FP32 "
                                 "instructions that this build does not emit (vector_fma_measured gives the rate "
                                 "non-packed FMAs reach on this device); FLOP = N(N-1)/2 (29 + 36m), the "
-                                "pair-once count (each unordered pair once, m = 2 columns)",
+                                "pair-once count (each unordered pair once, m = 2 columns), the damping of every "
+                                "pair among it, which the kernel forms for close pairs only (so that this rate can "
+                                "pass that of executed FMAs)",
                      "flop_formula": "N(N-1)/2*(29+36m)",
                      "kernel": "k_tmv_sym<float,2,AMOEBA> (on-the-fly FP32 pair kernel, each unordered pair "
                                "evaluated once; in the step it forms the FP32 residuals between the far-field "
