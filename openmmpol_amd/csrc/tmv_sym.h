@@ -23,11 +23,11 @@
 // damped pairs, one long dependent chain each: at 8,000 sites of a chain in FP64 it
 // took 120 of the sweep's 122 us.
 //
-// Bound by the vector unit's issue (56 instructions per pair, FP64 one column, at
-// 60,000 sites).  us per sweep, before these diagonals and the cutoffs of pair_damp_v
-// and now: FP64 one / two columns at 8,000 sites 123 / 151 and 86 / 113, at 15,000 253 /
-// 310 and 190 / 278, at 60,000 2890 / 4200 and 2590 / 3920; FP32 two columns at 15,000
-// 166 and 152, at 60,000 2190 and 2030.
+// Bound by the vector unit's issue (instructions per pair at 60,000 sites: FP64 one / two
+// columns 45 / 67, FP32 37 / 58).  us per sweep, before these diagonals and the cutoffs of
+// pair_damp_v and now: FP64 one / two columns at 8,000 sites 113 / 144 and 77 / 105, at
+// 15,000 (water) 221 / 309 and 189 / 270, at 60,000 2895 / 4260 and 2565 / 3945; FP32 two
+// columns at 15,000 164 and 147, at 60,000 2190 and 2015.
 #pragma once
 
 #include <hip/hip_runtime.h>
