@@ -230,6 +230,22 @@ def test_multi_rhs_pair_once_matches_oracle(tight_oracle):
     s.terminate()
 
 
+@pytest.mark.parametrize("n", [4499, 4500, 4609])
+def test_one_field_around_pair_once_size(n):
+    """A batch of one field just below the pair-once size, at it and with one site in
+    its last block, against the FP64 solver: both stop at an rms of 1e-10 of the
+    preconditioned residual, the dipoles within 1e-7 as everywhere here."""
+    from test_gpu_rows import chain, pair
+    s, _ = pair(chain(n, True))
+    s.set_solver_tolerance(TOL, 500)
+    ext = np.random.default_rng(n).normal(0.0, 1e-2, size=(1, n, 3))
+    ipd, ep = s.set_external_fields_multi(ext)
+    s.set_external_field(ext[0])
+    assert np.abs(ipd[0] - s.ipd).max() < 1e-7
+    assert abs(ep[0] - s.get_polelec_energy()) <= 1e-8 * abs(ep[0])
+    s.terminate()
+
+
 def test_server_pair_once_sizes_alone_and_in_mix(tight_oracle):
     """Requests of 7,500 sites (FP64 matvec pair-once), 13,000 (both matvecs
     pair-once) and 700 (per-target) together: each request's results alone and
